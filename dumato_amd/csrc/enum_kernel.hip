@@ -23,11 +23,12 @@
 //     passes the canonical rule).  The valid elements E_l are exactly the
 //     reference's extensions after canonicalFilter2; the mask bits are the
 //     reference's induction bits (forward_induce / aggregate_pattern).
-//   * The last level is never materialised: for each child c of level K-3,
-//     one pass over N(c) (an LDS membership bitmap of U_{K-3} first; the
-//     elements it does not rule out are searched in U_{K-3}) gives, per mask
-//     value, how many leaves are adjacent to c, and the class of every leaf
-//     follows from (mask, adjacency to c) through the class table.
+//   * The last two levels are never materialised.  A leaf of a node of level
+//     K-3 is an unordered pair of valid elements of U_{K-3}, or a valid
+//     element and a new neighbour of it; its class follows from the two masks
+//     and the pair's adjacency through the class table.  One pass over the
+//     out-neighbours N+(x) of U_{K-3}'s elements finds the edges inside U_{K-3}
+//     (motif_leaf); everything else is counted in closed form.
 //   * Work: static per-worker queues of (root, lo, hi) jobs, stealing of
 //     other workers' static jobs, and donation of the lowest level's
 //     remaining children to a device queue when workers are idle (the
@@ -37,6 +38,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <type_traits>
 
 #include "internal.h"
 
@@ -57,7 +59,6 @@ constexpr int kThreads = 256;
 template <int W, int MODE>
 constexpr int min_waves() { return W == 64 && MODE == 1 ? 4 : 3; }
 constexpr int kDeepMotifWaves = 6;
-constexpr int kMaxPm = 32;  // 2^(K-2) mask values for K <= 7
 
 // ---------------------------------------------------------------------------
 // virtual-wave primitives
@@ -117,8 +118,38 @@ DEV int uni(int x) {
     else return x;
 }
 
+// The same for 64-bit values and pointers: what a worker's lanes share and
+// read from memory stays in scalar registers for a full wave.
+template <int W, class T>
+DEV T unil(T x) {
+    if constexpr (W == 64) {
+        const uint64_t v = (uint64_t)x;
+        const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
+        const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
+        return (T)(((uint64_t)hi << 32) | lo);
+    } else {
+        return x;
+    }
+}
+
 DEV void wsync() { __threadfence_block(); }
 
+// Orders a wave's LDS accesses (executed in order per wave) for the compiler.
+DEV void lsync() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
+
+// LDS words addressed as such (ds instructions; a generic pointer takes flat ones)
+using lds_u32 = __attribute__((address_space(3))) uint32_t;
+using lds_u64 = __attribute__((address_space(3))) uint64_t;
+// LDS address of a generic pointer into LDS
+DEV uint32_t lds_at(const void *a) { return (uint32_t)(uintptr_t)(lds_u32 *)a; }
+template <class P, class T>
+DEV void ladd(P *a, T v) {
+    (void)__hip_atomic_fetch_add(a, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+}
+template <class P>
+DEV void lor(P *a, uint64_t v) {
+    (void)__hip_atomic_fetch_or(a, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+}
 DEV int lower_bound(const int32_t *a, int n, int32_t x) {
     int lo = 0, hi = n;
     while (lo < hi) {
@@ -151,18 +182,16 @@ struct Lvl {
 
 // Per-worker LDS record, at fixed offsets from one base so that a worker
 // holds a single pointer to it: uint64 st[kStats] (the worker's statistics),
-// int32 jid[kJobIds] (the prefix of the current job), uint32 n_gt[kMaxPm]
-// (motif leaf-phase counters), then Lvl lv[nlv], nlv = max(K-2, 1).
+// int32 jid[kJobIds] (the prefix of the current job), then Lvl lv[nlv], nlv =
+// max(K-2, 1).
 enum { kStBusy, kStJobs, kStFirst, kStStatic, kStLast, kStQCount, kStDonated, kStT0, kStJobMax, kStats };
 constexpr int kJidOff = 80;
-constexpr int kNgtOff = kJidOff + kJobIds * 4;
-constexpr int kLvOff = (kNgtOff + kMaxPm * 4 + 15) & ~15;
+constexpr int kLvOff = (kJidOff + kJobIds * 4 + 15) & ~15;
 static_assert(kStats * 8 <= kJidOff, "worker statistics overlap the job prefix");
 struct WorkerLDS {
     char *b;
     DEV unsigned long long *st() const { return (unsigned long long *)b; }
     DEV int32_t *jid() const { return (int32_t *)(b + kJidOff); }
-    DEV uint32_t *n_gt() const { return (uint32_t *)(b + kNgtOff); }
     DEV Lvl *lv() const { return (Lvl *)(b + kLvOff); }
 };
 DEV int nlevels(int K) { return K - 2 > 1 ? K - 2 : 1; }
@@ -175,6 +204,347 @@ DEV WorkerLDS worker_lds(char *base, int K) {
     WorkerLDS w;
     w.b = base;
     return w;
+}
+
+// ---------------------------------------------------------------------------
+// The motif leaf node: a node of level K-3 with prefix id[0..K-3], U = U_{K-3},
+// npm = 2^(K-2) mask values, E = the valid elements of U.  Each of its
+// K-subgraphs is the prefix plus either two elements of E, or an element of E
+// and one of its neighbours above id[0] outside U; the class depends on the
+// two masks and the adjacency alone, not on which is the child and which the
+// leaf.  So the counts per class need only, per mask i:
+//   n_i   elements of E with mask i,
+//   q_i   sum of |N(x) above id[0]| over them,
+//   e_ij  edges between E-elements of masks i and j (e_i0: to U \ E),
+// as pairs(i, j) = e_ij adjacent, n_i n_j - e_ij (C(n_i, 2) - e_ii) not, and
+// new(i) = q_i - sum_j e_ij - e_ii.
+// Every edge {x, y} inside U, x < y, is found once, from N+(x): the work is
+// sum over U of |N+(x)| membership tests of U, not sum over E of |N(x)|.  A
+// degree-ordered N+ is short where N is long, so beside hubs this is 3-5x
+// fewer (over the leaf nodes of Chung-Lu 18K k = 4: 305 M against 1,116 M;
+// Barabasi-Albert 100K k = 4: 678 M against 3,557 M).  Calls against the
+// leaf that streamed every child's N(c): Chung-Lu 18K k = 4 4.76 -> 2.12 ms,
+// Barabasi-Albert 100K k = 4 16.5 -> 5.9 ms, 12K k = 5 167 -> 43 ms.
+//
+// U is held in a hash table for these tests: buckets of two 32-bit slots, two
+// buckets per element, so a test is two 8-byte LDS reads and no loop.  A slot
+// holds the bits of the element's hash that its bucket does not determine
+// (32 - b), whether it sits in its second bucket, and its 6-bit code ^ 63
+// (code: its mask if valid, 32 if not; 63 marks an empty slot); together they
+// identify any 31-bit id once b >= 7.  The table is in LDS, or in the worker's
+// arena where U is too large for that.
+constexpr uint32_t kEmpty = 63;
+
+struct LeafSum {
+    unsigned long long cnt, bytes;  // this lane's share
+    int big;                        // > 0: needs a table of 2^big slots in memory
+};
+
+// The table's b and hash split; slots are reached through lds (LDS) or glb.
+template <bool LDS>
+struct LeafTab {
+    using P32 = std::conditional_t<LDS, lds_u32 *, uint32_t *>;
+    using P64 = std::conditional_t<LDS, lds_u64 *, uint64_t *>;
+    P32 t;
+    int b, sh;     // 2^b buckets, sh = 32 - b
+    uint32_t mul;  // odd: the hash is a bijection
+    DEV uint32_t other(uint32_t bk, uint32_t r) const { return bk ^ (((r >> (sh - b)) ^ (r >> 1)) & ((1u << b) - 1)); }
+    // code of x (0: not in U)
+    DEV int find(int32_t x) const {
+        const uint32_t h = (uint32_t)x * mul;
+        const uint32_t b1 = h >> sh, r = h & ((1u << sh) - 1), b2 = other(b1, r);
+        const uint32_t k1 = r << 7, k2 = k1 | 64;
+        const uint64_t s1 = ((P64)t)[b1], s2 = ((P64)t)[b2];
+        const uint32_t a0 = (uint32_t)s1 ^ k1, a1 = (uint32_t)(s1 >> 32) ^ k1;
+        const uint32_t a2 = (uint32_t)s2 ^ k2, a3 = (uint32_t)(s2 >> 32) ^ k2;
+        const uint32_t m0 = a0 < a1 ? a0 : a1, m1 = a2 < a3 ? a2 : a3;
+        const uint32_t m = m0 < m1 ? m0 : m1;
+        return m < 63 ? (int)(m ^ 63) : 0;
+    }
+    // adds mask bit `bit` to x if it is in U and valid; false: not in U
+    DEV bool mark(int32_t x, uint32_t bit) const {
+        const uint32_t h = (uint32_t)x * mul;
+        const uint32_t b1 = h >> sh, r = h & ((1u << sh) - 1), b2 = other(b1, r);
+        const uint32_t k1 = r << 7;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            P32 s = t + 2 * (i < 2 ? b1 : b2) + (i & 1);
+            const uint32_t v = *s, a = v ^ (k1 | (i < 2 ? 0 : 64));
+            if (a < 63) {
+                if (a != (32 ^ 63)) *s = v ^ bit;
+                return true;
+            }
+        }
+        return false;
+    }
+    // inserts x (not present); false when no slot was found: a full bucket's
+    // element is moved on to its other bucket, which one by a mixed bit (a
+    // fixed order runs into cycles from half load on)
+    DEV bool insert(int32_t x, int code) const {
+        const uint32_t h = (uint32_t)x * mul;
+        uint32_t bk = h >> sh, v = ((h & ((1u << sh) - 1)) << 7) | (uint32_t)(code ^ 63);
+        for (uint32_t it = 0; it < 256; it++) {
+            P32 s = t + 2 * bk;
+            if (cas(s, v) || cas(s + 1, v)) return true;
+            if (it == 0) {
+                P32 o = t + 2 * other(bk, v >> 7);
+                if (cas(o, v ^ 64) || cas(o + 1, v ^ 64)) return true;
+            }
+            v = __hip_atomic_exchange(s + (((v + it) * 0x85EBCA6Bu) >> 31), v, __ATOMIC_RELAXED, kScope);
+            bk = other(bk, v >> 7);
+            v ^= 64;
+        }
+        return false;
+    }
+    static constexpr int kScope = LDS ? __HIP_MEMORY_SCOPE_WAVEFRONT : __HIP_MEMORY_SCOPE_AGENT;
+    DEV static bool cas(P32 s, uint32_t v) {
+        uint32_t e = kEmpty;
+        return __hip_atomic_compare_exchange_strong(s, &e, v, __ATOMIC_RELAXED, __ATOMIC_RELAXED, kScope);
+    }
+    DEV static void sync() {
+        if constexpr (LDS) lsync();
+        else wsync();
+    }
+    // U of the leaf: the parent's list (masks pm, nullptr: all 1) with the
+    // order rule x > c, then nc[0, q), whose new elements get mask newc
+    template <int W>
+    DEV bool build(const Grp<W> &g, const int32_t *puid, const uint8_t *pupm, int pnu, int32_t c, const int32_t *nc,
+                   int q, int newc) const {
+        for (int j = g.gl; j < (1 << b); j += W) ((P64)t)[j] = ((uint64_t)kEmpty << 32) | kEmpty;
+        sync();
+        bool ok = true;
+        for (int j = g.gl; j < pnu; j += W) {
+            const int32_t x = puid[j];
+            const int pm = pupm ? pupm[j] : 0x81;
+            ok &= insert(x, (pm & 0x80) && x > c ? pm & 0x7f : 32);
+        }
+        sync();
+        for (int j0 = 0; j0 < q; j0 += W) {
+            const int j = j0 + g.gl;
+            bool add = false;
+            int32_t x = 0;
+            if (j < q) {
+                x = nc[j];
+                add = pnu == 0 || !mark(x, (uint32_t)newc);
+            }
+            sync();
+            if (add) ok &= insert(x, newc);
+            sync();
+        }
+        return g.ballot(!ok) == 0;
+    }
+};
+
+// Position of the first entry of a[0, n) not below x (ascending), by all the
+// worker's lanes: each step narrows the range W-fold.
+template <int W>
+DEV int wave_lower_bound(const Grp<W> &g, const int32_t *a, int n, int32_t x) {
+    int lo = 0;
+    while (n > 0) {
+        const int st = (n + W - 1) / W;  // lane i looks at the end of piece i
+        const int i = (g.gl + 1) * st - 1;
+        const bool below = i < n && a[lo + i] < x;
+        const int full = __popcll(g.ballot(below)) * st;  // pieces wholly below x
+        if (st == 1) return lo + full;
+        lo += full;
+        n = n - full < st - 1 ? n - full : st - 1;
+    }
+    return lo;
+}
+
+// The counts of one leaf node, added to the class counters at LDS address shist_at.  (c, pmc):
+// the child of the parent's list (puid, pupm, pnu) that makes the node, its
+// mask; K = 3: the root alone, c = id[0], whose elements [lo, hi) are taken
+// as children.  lds_at: motif_leaf_fixed bytes of LDS, then `space` bytes for the table;
+// gtab: a table of 2^space slots in memory instead.  Not inlined: the node's
+// registers are then its own, not shared with the search around it.
+template <int W>
+__device__ __attribute__((noinline)) LeafSum motif_leaf(const int64_t *off, const int32_t *adj, const int64_t *ostart,
+                                                        const uint16_t *lut, const int32_t *puid, const uint8_t *pupm,
+                                                        uint32_t shist_at, uint32_t lds_at, uint32_t *gtab, uint64_t pind,
+                                                        int32_t v0, int K, int32_t c, int pmc, int pnu, int psdeg,
+                                                        int lo, int hi, int space) {
+    off = unil<W>(off), adj = unil<W>(adj), ostart = unil<W>(ostart), lut = unil<W>(lut);
+    puid = unil<W>(puid), pupm = unil<W>(pupm), gtab = unil<W>(gtab), pind = unil<W>(pind);
+    v0 = uni<W>(v0), K = uni<W>(K), c = uni<W>(c), pmc = uni<W>(pmc), pnu = uni<W>(pnu), psdeg = uni<W>(psdeg);
+    lo = uni<W>(lo), hi = uni<W>(hi), space = uni<W>(space);
+    lds_u64 *const lds = (lds_u64 *)(uintptr_t)(uint32_t)uni<W>((int)lds_at);
+    lds_u64 *const shist = (lds_u64 *)(uintptr_t)(uint32_t)uni<W>((int)shist_at);
+    Grp<W> g;
+    const bool root = K == 3;
+    const int npm = 1 << (K - 2), newc = npm >> 1;  // newc: mask of an element only N(c) holds
+    const int64_t cb = unil<W>(off[c]), ce = unil<W>(off[c + 1]);
+    const int sdeg = psdeg + (int)(ce - cb);
+    const int64_t cs = root ? unil<W>(ostart[c]) : cb + wave_lower_bound(g, adj + cb, (int)(ce - cb), v0 + 1);
+    const int32_t *nc = adj + cs;  // N(c) above id[0]
+    const int q = (int)(ce - cs);
+    const int tot = pnu + q;  // elements of U, common ones twice
+    LeafSum r{0, 0, 0};
+
+    lds_u64 *recs = lds;
+    lds_u64 *bits = recs + W;
+    lds_u64 *qs = bits + kLeafCap / 64;
+    lds_u32 *nm = (lds_u32 *)(qs + npm);
+    lds_u32 *e = nm + npm;
+    const int ne = npm * (npm + 1) / 2, copies = leaf_copies(K);
+    LeafTab<true> tl;
+    LeafTab<false> tg;
+    if (!gtab) {
+        // at least 4/3 slots per element while the space allows it
+        int b = 7;
+        while ((16 << b) <= space && 3 * (2 << b) < 5 * tot) b++;
+        tl.t = (lds_u32 *)(lds + motif_leaf_fixed(W, K) / 8);
+        tl.b = b, tl.sh = 32 - b;
+        tl.mul = 0x9E3779B1u;
+        // up to 6/7 full; a failed insertion is rare from there on down
+        if ((8 << b) > space || 7 * tot > 6 * (2 << b) || !tl.build(g, puid, pupm, pnu, c, nc, q, newc)) {
+            b = 9;
+            while ((1 << b) < tot + tot / 2) b++;
+            r.big = b;
+            return r;
+        }
+    } else {
+        tg.t = gtab;
+        tg.b = space - 1, tg.sh = 33 - space;
+        tg.mul = 0x9E3779B1u;
+        for (int tries = 0; !tg.build(g, puid, pupm, pnu, c, nc, q, newc); tries++) {
+            if (tries == 7) {
+                r.big = -1;
+                return r;
+            }
+            tg.mul = tg.mul * 0x2545F491u + 2;  // another odd multiplier
+        }
+    }
+    auto find = [&](int32_t x) { return gtab ? tg.find(x) : tl.find(x); };
+    for (int j = g.gl; j < ne * copies; j += W) e[j] = 0;
+    for (int j = g.gl; j < npm; j += W) nm[j] = 0, qs[j] = 0;
+    lsync();
+
+    // elements of U, W at a time: n_i and q_i, then their out-lists laid end
+    // to end (recs: list start and mask, by list; bits: a set bit per list
+    // start), over which the lanes stride
+    uint32_t nnew = 0, enew = 0;  // class newc / (newc, newc), counted in registers
+    unsigned long long qnew = 0, by = 0, leaves = 0, rpairs = 0;
+    lds_u32 *const ecopy = e + (g.gl & (copies - 1)) * ne;
+    for (int j0 = 0; j0 < tot; j0 += W) {
+        const int j = j0 + g.gl;
+        int32_t x = 0;
+        int code = 0;
+        if (j < tot) {
+            x = j < pnu ? puid[j] : nc[j - pnu];
+            code = find(x);
+            // a neighbour of c that an earlier list holds too is visited in
+            // the parent's list
+            if (j >= pnu && code != newc) code = 0;
+            if (root && (j < lo || j >= hi)) code = 0;
+        }
+        const int cx = code & 31;
+        int len = 0;
+        int64_t os = 0;
+        if (code) {
+            const int64_t b = off[x], en = off[x + 1];
+            os = ostart[x];
+            len = (int)(en - os);
+            if (cx) {
+                const int up = (int)(en - b) - lower_bound(adj + b, (int)(os - b), v0 + 1);
+                by += (unsigned long long)(sdeg + (int)(en - b));
+                if (cx == newc) {
+                    nnew++;
+                    qnew += (unsigned long long)up;
+                } else {
+                    ladd(nm + cx, 1u);
+                    ladd(qs + cx, (uint64_t)up);
+                }
+                if (root) rpairs += (unsigned long long)(tot - 1 - j);
+            }
+        }
+        const uint64_t mx = g.ballot(len > 0);
+        const int sc = g.iscan(len), pre = sc - len;
+        const int T = g.bcast(sc, W - 1);
+        if (len > 0) recs[g.below(mx)] = ((uint64_t)(os - pre) & 0xffffffffffffffull) | ((uint64_t)cx << 56);
+        for (int p0 = 0; p0 < T; p0 += kLeafCap) {
+            const int pe = T - p0 < kLeafCap ? T : p0 + kLeafCap;
+            for (int w = g.gl; w < kLeafCap / 64; w += W) bits[w] = 0;
+            lsync();
+            if (len > 0 && pre >= p0 && pre < pe) lor(bits + ((pre - p0) >> 6), 1ull << ((pre - p0) & 63));
+            // lists that started before this chunk
+            int own0 = __popcll(g.ballot(len > 0 && pre < p0)) - 1;
+            lsync();
+            constexpr int U = 4;
+            for (int t0 = p0; t0 < pe; t0 += U * W) {
+                int32_t ys[U];
+                int cm[U];
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const int t = t0 + u * W + g.gl;
+                    const int o = t0 + u * W - p0;
+                    uint64_t seg = o < kLeafCap ? bits[o >> 6] : 0;
+                    if constexpr (W == 64) seg = unil<W>(seg);
+                    else seg = (seg >> (o & 63)) & ((1ull << W) - 1);
+                    const int own = own0 + __popcll(seg & ((2ull << g.gl) - 1));
+                    own0 += __popcll(seg);
+                    ys[u] = v0;  // no element: v0 is never in U
+                    cm[u] = 0;
+                    if (t < pe) {
+                        const uint64_t rec = recs[own];
+                        cm[u] = (int)(rec >> 56);
+                        ys[u] = adj[((int64_t)(rec << 8) >> 8) + t];
+                    }
+                }
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const int cd = find(ys[u]);
+                    if (cd) {
+                        const int cy = cd & 31, a = cm[u] > cy ? cm[u] : cy, z = cm[u] > cy ? cy : cm[u];
+                        if (a == newc && z == newc) enew++;
+                        else ladd(ecopy + (__umul24(a, a + 1) >> 1) + z, 1u);
+                    }
+                }
+            }
+            lsync();
+        }
+    }
+    if (nnew) ladd(nm + newc, nnew);
+    if (qnew) ladd(qs + newc, (uint64_t)qnew);
+    if (enew) ladd(e + newc * (newc + 1) / 2 + newc, enew);
+    lsync();
+    if (copies > 1) {
+        for (int t = g.gl; t < ne; t += W) {
+            uint32_t sum = 0;
+            for (int k = 0; k < copies; k++) sum += e[k * ne + t];
+            e[t] = sum;
+        }
+        lsync();
+    }
+    // edges between masks i >= j (0: U \ E); the lut index of the prefix
+    // id[0..K-3] and its child's mask i
+    auto edges = [&](int i, int j) -> uint64_t { return e[i * (i + 1) / 2 + j]; };
+    const uint64_t ind = root ? 0 : pind + (K - 3 >= 2 ? (uint64_t)pmc << quick_off(K - 3) : 0);
+    auto child = [&](int i) -> uint64_t { return root ? 0 : ind + ((uint64_t)i << quick_off(K - 2)); };
+    const int o2 = quick_off(K - 1);
+    if (root) rpairs = g.lsum(rpairs);
+    for (int t = g.gl; t < npm * npm; t += W) {
+        const int i = t >> (K - 2), j = t & (npm - 1);
+        if (j == 0 || i < j) continue;
+        const uint64_t ni = nm[i], nj = nm[j];
+        const uint64_t pr = root ? rpairs : i == j ? ni * (ni - 1) / 2 : ni * nj;
+        if (pr == 0) continue;
+        const uint64_t ee = edges(i, j);
+        if (ee) ladd(shist + lut[child(i) + ((uint64_t)(j | npm) << o2)], ee);
+        if (pr != ee) ladd(shist + lut[child(i) + ((uint64_t)j << o2)], pr - ee);
+        leaves += pr;
+    }
+    for (int i = 1 + g.gl; i < npm; i += W) {
+        uint64_t nw = qs[i];
+        for (int j = 0; j < npm; j++) nw -= i == j ? 2 * edges(i, i) : i > j ? edges(i, j) : edges(j, i);
+        if (nw) ladd(shist + lut[child(i) + ((uint64_t)npm << o2)], nw);
+        leaves += nw;
+    }
+    lsync();
+    r.cnt = leaves;
+    // the node's own bytes (at k = 3 the root's are counted by the caller)
+    r.bytes = 4ull * by + 4ull * (K - 1) * leaves + (!root && g.gl == 0 ? 4ull * (unsigned long long)sdeg : 0ull);
+    return r;
 }
 
 template <int W, int MODE>
@@ -206,21 +576,6 @@ struct Worker {
     uint64_t last_poll;  // wall clock of the last donation check
     uint32_t polls;      // donation checks so far (lane 0's count)
     bool abort;
-    // motif leaf-phase scratch, reserved first in the LDS slice of each job:
-    // cs int64[B] | ic u32[B][npm] | nn u32[B] | cc i32[B] | pre i32[B + 1]
-    // | qx i32[2W] | qa i32[2W] (lookups waiting for the search of U)
-    char *lf;
-    // children per leaf batch: a full worker, capped so that the per-child
-    // mask counters (slots x 2^(K-2)) stay within 512 words
-    DEV static int leaf_slots(int K) {
-        const int cap = 512 >> (K - 2);
-        return W < cap ? W : cap;
-    }
-    DEV static int64_t leaf_scratch_bytes(int K) {
-        const int B = leaf_slots(K);
-        return (int64_t)B * 8 + (int64_t)B * (1 << (K - 2)) * 4 + (int64_t)B * 12 + 4 + 16 * W;
-    }
-
     DEV Worker(const EnumParams &p_, WorkerLDS ws_, unsigned long long *sh_, char *lds_slice,
                int wid)
         : p(p_), ws(ws_), shist(sh_) {
@@ -325,28 +680,26 @@ struct Worker {
 
     // Publishes up to P jobs for the children [cur, end) of level lvl: the
     // range is cut into np + 1 pieces of equal estimated work, np <= P as the
-    // queue allows, and all but one are queued.  The worker keeps the first
-    // piece (upper == true; returns its new end) or the last one (returns its
-    // new start).  Returns end (start) unchanged when nothing was queued.
-    DEV int push_pieces(int lvl, int cur, int end, int P, bool upper) {
+    // queue allows, and all but the first are queued.  Returns the end of the
+    // piece the worker keeps (end itself when nothing was queued).
+    DEV int push_pieces(int lvl, int cur, int end, int P) {
         uint32_t slot = 0;
         const int np = reserve_slots(P, slot);
-        if (np == 0) return upper ? end : cur;
-        const int first = upper ? 1 : 0;  // first queued piece
+        if (np == 0) return end;
         const uint64_t tag = (uint64_t)epoch << 32;
         for (int idx = g.gl; idx < np * kJobWords; idx += W) {
             const int r = idx / kJobWords, j = idx - r * kJobWords;
             int32_t v;
             if (j == 0) v = lvl;
-            else if (j == 1) v = split_at(lvl, cur, end, first + r, np + 1);
-            else if (j == 2) v = split_at(lvl, cur, end, first + r + 1, np + 1);
+            else if (j == 1) v = split_at(lvl, cur, end, 1 + r, np + 1);
+            else if (j == 2) v = split_at(lvl, cur, end, 2 + r, np + 1);
             else if (j == 3) v = qword;
             else v = (j - 4 <= lvl) ? ws.lv()[j - 4].vtx : -1;
             __hip_atomic_store(p.q[slot + r].w + j, tag | (uint32_t)v, __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_AGENT);
         }
         if (g.gl == 0) ws.st()[kStDonated] += (unsigned long long)np;
-        return split_at(lvl, cur, end, upper ? 1 : np, np + 1);
+        return split_at(lvl, cur, end, 1, np + 1);
     }
 
     // Queues the roots [lo, hi) of this worker's range job as a range job
@@ -392,8 +745,6 @@ struct Worker {
     // Donate remaining children when tickets wait for jobs: the shallowest
     // level of the job with enough children left is cut into one piece per
     // waiting ticket (at most kMaxPieces) plus the piece this worker keeps.
-    // leaf_k / leaf_lo / leaf_i describe the descending leaf-phase loop of
-    // level leaf_k (remaining children [lo, i]); leaf_k < 0 when not in it.
     static constexpr int kMaxPieces = 8;
     // Waiting tickets (at most kMaxPieces), checked at most every poll
     // period; 0 when stealing is off.  A worker takes a ticket once no
@@ -421,7 +772,7 @@ struct Worker {
 
     // min_first > 0: the job's own level may be cut down to pieces of that
     // many children (heavy children, where steal_min would leave too much)
-    DEV void maybe_donate(int top, int leaf_k, int &leaf_lo, int leaf_i, int min_first = 0) {
+    DEV void maybe_donate(int top, int min_first = 0) {
         const int want = donation_demand();
         if (want == 0) return;
         // untouched roots of a range job go first: they need no prefix
@@ -430,7 +781,7 @@ struct Worker {
             if (push_range(mid, range_hi)) range_hi = mid;
             return;
         }
-        // the last level's children are cheap: split it only in bigger pieces
+        // a clique's last level has cheap children: split it only in bigger pieces
         const int leaf_min = 4 * job_sm;
         for (int l = job_lvl; l < top; l++) {
             const int cur = ws.lv()[l].cur, end = ws.lv()[l].end;
@@ -440,18 +791,9 @@ struct Worker {
                 if (P < 1) P = 1;
                 if (P > want) P = want;
                 if (P > end - cur - 1) P = end - cur - 1;
-                if (P >= 1) ws.lv()[l].end = push_pieces(l, cur, end, P, true);
+                if (P >= 1) ws.lv()[l].end = push_pieces(l, cur, end, P);
                 return;
             }
-        }
-        const int left = leaf_i + 1 - leaf_lo;
-        if (leaf_k >= 0 && left >= leaf_min) {
-            // the leaf loop runs downward: queue the lower pieces
-            int P = left / leaf_min - 1;
-            if (P < 1) P = 1;
-            if (P > want) P = want;
-            if (P > left - 1) P = left - 1;
-            if (P >= 1) leaf_lo = push_pieces(leaf_k, leaf_lo, leaf_i + 1, P, false);
         }
     }
 
@@ -481,25 +823,21 @@ struct Worker {
         Lvl &P = ws.lv()[l];
         Lvl &N = ws.lv()[l + 1];
         const int l1 = l + 1;
-        const int32_t *nc = nbr(c);
-        const int dc = deg(c);
-        const int s0 = lower_bound(nc, dc, v0 + 1);
+        const int64_t cb = unil<W>(p.off[c]);
+        const int32_t *nc = p.adj + cb;
+        const int dc = (int)(unil<W>(p.off[c + 1]) - cb);
+        const int s0 = uni<W>(lower_bound(nc, dc, v0 + 1));
         const int q = dc - s0;
-        const int pnu = P.nu;
+        const int pnu = uni<W>(P.nu);
+        const int32_t *const puid = unil<W>(P.uid);
+        const uint8_t *const pupm = unil<W>(P.upm);
         N.mark_lds = lds_top;
         N.mark_glb = g_top;
         const int cap = pnu + q;
-        // At k >= 5 the leaf level's lists (the union of three or more
-        // neighbourhoods) go to global memory when they would take more than
-        // half the free LDS: the leaf phase reads them rarely and needs the
-        // LDS for its membership filter.  (At k = 4 they stay in LDS: short
-        // lists, and moving them measured slower.)
-        const bool lg = l1 == K - 3 && l1 >= 2 &&
-                        (int64_t)cap * 10 > (lds_lo + p.lds_per_worker - lds_top) / 2;
-        int32_t *uid = (int32_t *)(lg ? alloc_glb((int64_t)cap * 4) : alloc((int64_t)cap * 4));
-        uint8_t *upm = (uint8_t *)(lg ? alloc_glb(cap) : alloc(cap));
-        int32_t *eid = (int32_t *)(lg ? alloc_glb((int64_t)cap * 4) : alloc((int64_t)cap * 4));
-        uint8_t *epm = (uint8_t *)(lg ? alloc_glb(cap) : alloc(cap));
+        int32_t *uid = (int32_t *)alloc((int64_t)cap * 4);
+        uint8_t *upm = (uint8_t *)alloc(cap);
+        int32_t *eid = (int32_t *)alloc((int64_t)cap * 4);
+        uint8_t *epm = (uint8_t *)alloc(cap);
         char *tmark_l = lds_top, *tmark_g = g_top;
         int32_t *nw = (int32_t *)alloc((int64_t)(q > 0 ? q : 1) * 4);
         uint8_t *hit = (uint8_t *)alloc(pnu > 0 ? pnu : 1);
@@ -514,8 +852,8 @@ struct Worker {
             int32_t x = in ? nc[s0 + t] : 0;
             bool found = false;
             if (in) {
-                int pos = lower_bound(P.uid, pnu, x);
-                found = pos < pnu && P.uid[pos] == x;
+                int pos = lower_bound(puid, pnu, x);
+                found = pos < pnu && puid[pos] == x;
                 if (found) hit[pos] = 1;
             }
             uint64_t m = g.ballot(in && !found);
@@ -526,9 +864,9 @@ struct Worker {
         // merge by ranks: old elements and new ones interleave in id order
         const uint8_t bit = (uint8_t)(1u << l1);
         for (int j = g.gl; j < pnu; j += W) {
-            int32_t x = P.uid[j];
+            int32_t x = puid[j];
             int o = j + lower_bound(nw, nnew, x);
-            uint8_t pm = upm_at(P, j);
+            uint8_t pm = pupm ? pupm[j] : (uint8_t)0x81;
             if (hit[j]) pm |= bit;
             bool valid = (pm & 0x80) && x > c;
             uid[o] = x;
@@ -536,7 +874,7 @@ struct Worker {
         }
         for (int t = g.gl; t < nnew; t += W) {
             int32_t x = nw[t];
-            int o = t + lower_bound(P.uid, pnu, x);
+            int o = t + lower_bound(puid, pnu, x);
             uid[o] = x;
             upm[o] = (uint8_t)(bit | 0x80);
         }
@@ -571,196 +909,31 @@ struct Worker {
         N.ind = (l1 >= 2) ? P.ind + ((uint64_t)pmc << quick_off(l1)) : 0;
     }
 
-    // children [lo, hi) of level l = K-3, each a node of level K-2 whose
-    // leaves are counted by class without being materialised.  Children are
-    // taken in descending order, in batches of up to W; the batch's
-    // (child, neighbour) pairs are flattened across the lanes so short
-    // neighbour lists do not leave lanes idle.
-    DEV void motif_leaf_phase(int l, int lo, int hi) {
-        Lvl &P = ws.lv()[l];
-        const int npm = 1 << (l + 1);  // mask values over the lists 0..l
-        const int top = npm;           // bit of the child's own list
-        const int s = quick_off(l + 2);
-        const int o1 = quick_off(l + 1);
-        const int B = leaf_slots(K);
-        int64_t *cs = (int64_t *)lf;
-        uint32_t *ic = (uint32_t *)(cs + B);
-        uint32_t *nn = ic + B * npm;
-        int32_t *cc = (int32_t *)(nn + B);
-        int32_t *pre = cc + B;
-        int32_t *qx = pre + B + 1;
-        int32_t *qa = qx + 2 * W;
-        // ws.n_gt()[m]: valid elements of E above the current batch, by mask
-        for (int j = g.gl; j < npm; j += W) ws.n_gt()[j] = 0;
-        for (int j = g.gl; j < B * npm; j += W) ic[j] = 0;
-        for (int j = g.gl; j < B; j += W) nn[j] = 0;
-        wsync();
-        for (int j = hi + g.gl; j < P.ne; j += W) atomicAdd(&ws.n_gt()[epm_at(P, j)], 1u);
-        wsync();
-        const int pnu = P.nu;
-        // Fences of U, one per lane: fence(f) = U[f * pnu / W].  A lookup
-        // finds its fence interval by a search over the lanes' registers
-        // (cross-lane permutes, free of LDS bank conflicts), then searches
-        // only that interval of U.
-        const bool use_f = pnu >= 2 * W;
-        const int32_t fence = use_f ? P.uid[(int)(((int64_t)g.gl * pnu) / W)] : 0;
-        const int32_t flast = __shfl(fence, W - 1, W);  // read by every lane
-        // Membership filter of U in LDS: bit (x mod 32*words) is set for every
-        // x in U, with at least 8 bits per element where LDS allows.  Most
-        // neighbours of a child are not in U; a clear bit proves it with one
-        // LDS read, and only the rest go through the search of U.
-        uint32_t *bm = nullptr;
-        int32_t bmask = 0;
-        {
-            int words = 32;
-            while (words < 1024 && words * 4 < pnu) words <<= 1;
-            while (words >= 32 && lds_top + words * 4 > lds_lo + p.lds_per_worker) words >>= 1;
-            if (words >= 32) {
-                bm = (uint32_t *)alloc((int64_t)words * 4);
-                bmask = words * 32 - 1;
-                for (int j = g.gl; j < words; j += W) bm[j] = 0;
-                wsync();
-                for (int j = g.gl; j < pnu; j += W) {
-                    const int32_t u = P.uid[j] & bmask;
-                    atomicOr(&bm[u >> 5], 1u << (u & 31));
-                }
-                wsync();
-            }
-        }
-        // search of U for queued lookups (all lanes take part in the fence
-        // permutes; `act` lanes hold an entry): a hit adds to the child's
-        // class counter, a miss is a new element of the child
-        auto resolve = [&](int32_t x, int a, bool act) {
-            int flo = 0, fhi = pnu;  // interval of U holding lower_bound(x)
-            if (use_f) {
-                int c = 0;  // number of fences below x
-#pragma unroll
-                for (int st = W / 2; st >= 1; st >>= 1)
-                    if (__shfl(fence, c + st - 1, W) < x) c += st;
-                if (c == W - 1 && flast < x) c = W;
-                if (c == 0) {
-                    fhi = 0;
-                } else {
-                    flo = (int)(((int64_t)(c - 1) * pnu) / W) + 1;
-                    fhi = c < W ? (int)(((int64_t)c * pnu) / W) : pnu;
-                }
-            }
-            if (act) {
-                const int pos = flo + lower_bound(P.uid + flo, fhi - flo, x);
-                if (pos < pnu && P.uid[pos] == x) {
-                    const uint8_t pm = upm_at(P, pos);
-                    if ((pm & 0x80) && x > cc[a]) atomicAdd(&ic[a * npm + (pm & 0x7f)], 1u);
-                } else {
-                    atomicAdd(&nn[a], 1u);
-                }
-            }
+    // ---- motif leaf ------------------------------------------------------------
+    // Leaf node of child i0 of level pl = K-4 (k >= 4), or the root itself at
+    // k = 3 (pl = -1) with the elements [lo, hi) of its list as children.
+    DEV void motif_leaf_node(int pl, int i0, int lo, int hi) {
+        if (check_abort()) return;
+        const Lvl &P = ws.lv()[pl < 0 ? 0 : pl];
+        const int32_t c = pl < 0 ? v0 : P.eid[i0];
+        const int pmc = pl < 0 ? 0 : epm_at(P, i0), pnu = pl < 0 ? 0 : P.nu, sd = pl < 0 ? 0 : P.sdeg;
+        auto run = [&](uint32_t *gtab, int space) {
+            return motif_leaf<W>(p.off, p.adj, p.ostart, lut, P.uid, P.upm, lds_at(shist), lds_at(lds_lo), gtab,
+                                 P.ind, v0, K, c, pmc, pnu, sd, lo, hi, space);
         };
-        // a batch takes children (at most B) until their neighbour lists hold
-        // about `target` elements: few, large batches amortise the per-batch
-        // class bookkeeping; the bound keeps the leaf donation checks, one
-        // per batch, frequent when the children are hubs
-        const int target = 256 * W;
-        int i = hi - 1;
-        while (i >= lo) {
-            if (check_abort()) return;
-            // leaf children are cheap and a donated piece rebuilds its whole
-            // prefix: offer them only from long leaf loops
-            if (i - lo + 1 >= 512) maybe_donate(l, l, lo, i);
-            if (i < lo) break;
-            const int avail = i - lo + 1 < B ? i - lo + 1 : B;
-            int len = 0, pm_a = -1;
-            if (g.gl < avail) {
-                const int32_t c = P.eid[i - g.gl];
-                const int dc = deg(c);
-                const int s0 = lower_bound(nbr(c), dc, v0 + 1);
-                len = dc - s0;
-                cc[g.gl] = c;
-                cs[g.gl] = p.off[c] + s0;
-                pm_a = epm_at(P, i - g.gl);
-            }
-            const int sc = g.iscan(len);
-            int take = __popcll(g.ballot(g.gl < avail && sc - len < target));
-            take = take < 1 ? 1 : take;
-            if (g.gl < take) pre[g.gl + 1] = sc;
-            if (g.gl == 0) pre[0] = 0;
-            const int tot = g.bcast(sc, take - 1);
-            wsync();
-            int a = 0;
-            int qn = 0;  // queued lookups (uniform)
-            for (int t0 = 0; t0 < tot; t0 += W) {
-                const int t = t0 + g.gl;
-                int32_t x = 0x7fffffff;
-                if (t < tot) {
-                    while (pre[a + 1] <= t) a++;
-                    x = p.adj[cs[a] + (t - pre[a])];
-                }
-                bool need = t < tot;
-                if (bm && need) need = (bm[(x & bmask) >> 5] >> (x & 31)) & 1u;
-                const bool fresh = t < tot && !need;  // proven outside U
-                // new elements are the common case: count them per child with
-                // one ballot, the child's first lane in this round adding its
-                // segment's popcount (no same-address atomics)
-                const uint64_t mf = g.ballot(fresh);
-                if (t < tot) {
-                    const int s0 = pre[a] > t0 ? pre[a] - t0 : 0;
-                    if (g.gl == s0) {
-                        const int s1 = pre[a + 1] - t0 < W ? pre[a + 1] - t0 : W;
-                        const uint64_t seg = (s1 - s0 >= 64 ? ~0ull : ((1ull << (s1 - s0)) - 1)) << s0;
-                        nn[a] += (uint32_t)__popcll(mf & seg);
-                    }
-                }
-                // the rest wait in the queue until a full wave of them can be
-                // searched together
-                const uint64_t mq = g.ballot(need);
-                if (need) {
-                    const int o = qn + g.below(mq);
-                    qx[o] = x;
-                    qa[o] = a;
-                }
-                qn += __popcll(mq);
-                if (qn >= W) {
-                    wsync();
-                    qn -= W;
-                    resolve(qx[qn + g.gl], qa[qn + g.gl], true);
-                    wsync();
-                }
-            }
-            if (qn > 0) {
-                wsync();
-                const bool act = g.gl < qn;
-                resolve(act ? qx[g.gl] : 0x7fffffff, act ? qa[g.gl] : 0, act);
-            }
-            wsync();
-            // per child: slot a = lane a; valid elements above it = the
-            // batch base plus earlier slots (larger E indices) with that mask
-            const bool mine = g.gl < take;
-            const uint64_t indc = P.ind + ((mine && l + 1 >= 2) ? ((uint64_t)pm_a << o1) : 0);
-            unsigned long long leaves = 0;
-            for (int j = 0; j < npm; j++) {
-                const uint64_t mj = g.ballot(mine && pm_a == j);
-                if (mine) {
-                    const uint32_t gtj = ws.n_gt()[j] + (uint32_t)g.below(mj);
-                    const uint32_t ai = ic[g.gl * npm + j];
-                    const uint32_t bi = gtj - ai;
-                    if (ai) atomicAdd(&shist[lut[indc + ((uint64_t)(j | top) << s)]], (unsigned long long)ai);
-                    if (bi) atomicAdd(&shist[lut[indc + ((uint64_t)j << s)]], (unsigned long long)bi);
-                    ic[g.gl * npm + j] = 0;
-                    leaves += gtj;
-                }
-                wsync();
-                if (g.gl == 0) ws.n_gt()[j] += (uint32_t)__popcll(mj);
-            }
-            if (mine) {
-                const uint32_t nw = nn[g.gl];
-                if (nw) atomicAdd(&shist[lut[indc + ((uint64_t)top << s)]], (unsigned long long)nw);
-                nn[g.gl] = 0;
-                leaves += nw;
-                cnt += leaves;
-                bytes += 4ull * (unsigned long long)(P.sdeg + deg(cc[g.gl])) + 4ull * (K - 1) * leaves;
-            }
-            wsync();
-            i -= take;
+        LeafSum r = run(nullptr, p.lds_per_worker - motif_leaf_fixed(W, K));
+        if (r.big) {
+            // U does not fit the LDS table: one in the arena
+            char *const mg = g_top;
+            const int b = r.big;
+            uint32_t *const gtab = (uint32_t *)alloc_glb((int64_t)4 << b);
+            if (abort) return;
+            r = run(gtab, b);
+            g_top = mg;
+            if (r.big) fail(2);
         }
+        cnt += r.cnt;
+        bytes += r.bytes;
     }
 
     // ---- clique levels ----------------------------------------------------------
@@ -833,11 +1006,9 @@ struct Worker {
         Lvl &P = ws.lv()[l];
         for (int i = lo; i < hi; i++) {
             if (check_abort()) return;
-            int dummy_lo = 0;
-            (void)dummy_lo;
             // donation of this level's tail happens through lv[l].cur/end
             P.cur = i + 1;
-            maybe_donate(l + 1, -1, dummy_lo, 0);
+            maybe_donate(l + 1);
             hi = P.end;
             if (i >= hi) break;
             const int32_t c = P.uid[i];
@@ -1101,7 +1272,6 @@ struct Worker {
         unsigned long long by = 0;
         while (true) {
             if (check_abort()) break;
-            int dummy = 0;
             // at k >= 6 a front child with many pairs (its work grows with
             // their cube) is heavy enough to travel alone
             int front = 0;
@@ -1110,7 +1280,7 @@ struct Worker {
                 for (int w = 0; w < NW; w++) front += __popcll(rows[R.cur * NW + w]);
             }
             front = g.bcast(front, 0);
-            maybe_donate(1, -1, dummy, 0, front >= W / 2 ? 2 : 0);
+            maybe_donate(1, front >= W / 2 ? 2 : 0);
             const int cur = R.cur, end = R.end;
             if (cur >= end) break;
             // a batch holds children until it has about `target` pairs (at
@@ -1230,16 +1400,14 @@ struct Worker {
     // `hi` jobs on a prebuilt bitmap root that claim its children from the
     // root's shared cursor
     DEV void run_job(int lvl, int lo, int hi, bool first_piece, bool shared) {
-        v0 = ws.jid()[0];
+        v0 = uni<W>(ws.jid()[0]);
         job_lvl = lvl;
         lds_top = lds_lo;
         g_top = g_lo;
         cnt = 0;
         const bool motif = MODE == 2 ? qmotif : MODE == 1;
-        if (motif) {
-            lf = alloc(leaf_scratch_bytes(K));
-            if (abort) return;
-        }
+        // a motif worker's slice is its leaf scratch; its lists are in the arena
+        if (motif) lds_top = lds_lo + p.lds_per_worker;
         if (!motif && K == 2) {
             if (g.gl == 0) {
                 int d = odeg(v0);
@@ -1284,7 +1452,6 @@ struct Worker {
             else clique_forward(l - 1, pos);
         }
         if (abort) return;
-        const int leafp = K - 3;
         {
             Lvl &L = ws.lv()[lvl];
             int ne = motif ? L.ne : L.nu;
@@ -1295,8 +1462,9 @@ struct Worker {
         while (k >= lvl) {
             if (check_abort()) return;
             Lvl &L = ws.lv()[k];
-            if (k == leafp) {
-                if (motif) motif_leaf_phase(k, L.cur, L.end);
+            if (k == K - 3) {
+                // a motif job comes here only at k = 3, whose root is the leaf
+                if (motif) motif_leaf_node(-1, 0, L.cur, L.end);
                 else clique_leaf_phase(k, L.cur, L.end);
                 if (abort) return;
                 lds_top = L.mark_lds;
@@ -1304,14 +1472,18 @@ struct Worker {
                 k--;
                 continue;
             }
-            int dummy = 0;
-            maybe_donate(k + 1, -1, dummy, 0);
-            if (L.cur < L.end) {
-                const int i = L.cur;
+            maybe_donate(k + 1);
+            const int i = uni<W>(L.cur);
+            if (i < uni<W>(L.end)) {
                 L.cur = i + 1;
+                if (motif && k == K - 4) {
+                    motif_leaf_node(k, i, 0, 0x7fffffff);
+                    if (abort) return;
+                    continue;
+                }
                 if (motif) {
-                    const int32_t c = L.eid[i];
-                    const int pmc = epm_at(L, i);
+                    const int32_t c = uni<W>(L.eid[i]);
+                    const int pmc = uni<W>(epm_at(L, i));
                     motif_forward(k, c, pmc);
                     if (abort) return;
                     Lvl &N = ws.lv()[k + 1];
@@ -1643,13 +1815,13 @@ __global__ __launch_bounds__(kThreads, WAVES) void enum_kernel(EnumParams p) {
                 if (g.gl == 0) ws.st()[kStQCount] = 0;
                 const QueryDesc &Q = p.qd[jq];
                 wk.qid = jq;
-                wk.K = Q.K;
-                wk.qmotif = Q.motif != 0;
-                wk.lut = Q.lut;
+                wk.K = uni<W>(Q.K);
+                wk.qmotif = uni<W>(Q.motif) != 0;
+                wk.lut = unil<W>(Q.lut);
                 ok = (MODE == 2 || (MODE == 1) == wk.qmotif) && Q.K >= 2 && Q.K <= p.kmax;
             }
             const int lvl_max = wk.K == 2 ? 0 : wk.K - 3;
-            const int r0 = ws.jid()[0];
+            const int r0 = uni<W>(ws.jid()[0]);
             const int r1 = jh.range_end > 0 ? jh.range_end : r0 + 1;
             if (!ok || jh.lvl < 0 || jh.lvl > lvl_max || r0 < 0 || r1 > p.n || r0 >= r1) {
                 wk.fail(3);

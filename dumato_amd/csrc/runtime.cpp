@@ -258,6 +258,7 @@ int pick_shape(dm_graph *g, int K, bool motif, const dm_config &cfg, Shape &sh) 
     const int dl = max_lds_per_worker(vw, threads, launch_mode(motif, K), K, ncls, 0);
     int lds = cfg.lds_bytes > 0 ? cfg.lds_bytes : threads == 256 ? tuned_lds(g, K, motif, vw, dl) : dl;
     lds = (lds + 15) & ~15;
+    if (motif) lds = std::max(lds, motif_leaf_fixed(vw, K));
     size_t lds_total = enum_lds_bytes(vw, threads, K, ncls, 0, lds);
     int bpc = 0;
     if ((r = enum_occupancy(vw, launch_mode(motif, K), threads, lds_total, &bpc))) return r;
@@ -283,11 +284,12 @@ int64_t arena_bound_for(int32_t maxdeg, int32_t max_out_, int K, bool motif) {
     int64_t md = std::max<int64_t>(maxdeg, 1);
     int64_t b = 256;
     if (motif) {
+        // levels 1..K-4: ids and masks of U and E; level K-3: the leaf's table
+        // where LDS does not hold it (at most 9.5 B per element, 2 KB at least)
         for (int l = 1; l <= K - 3; l++) b += 10 * (int64_t)(l + 1) * md + 64;
         b += 4 * md + (int64_t)(K - 2) * md + 64;
-        // leaf-phase scratch (at most 64 slots, 512 counters, a 128-entry
-        // lookup queue)
-        b += 64 * 8 + 512 * 4 + 64 * 12 + 4 + 16 * 64 + 16;
+        b += 4372;
+        if (K == 3) b = std::max<int64_t>(b, 4096 + 10 * (int64_t)std::max(max_out_, 1));
     } else {
         int64_t mo = std::max<int64_t>(max_out_, 1);
         for (int l = 1; l <= K - 3; l++) b += 4 * mo + 16;
