@@ -547,6 +547,201 @@ __device__ __attribute__((noinline)) LeafSum motif_leaf(const int64_t *off, cons
     return r;
 }
 
+// ---------------------------------------------------------------------------
+// Cliques of a batch of second-level pairs of a root's local bitmap (rows[i *
+// NW + w] bit b: L[64w+b] in N+(L[i]), L = N+(root)): pairs 0..P-1, pair t
+// belonging to child cur + a with pre[a] <= t < pre[a+1] and being its
+// (t - pre[a])-th candidate.  The loops visit exactly the DFS children of
+// every node above the last level, so the algorithmic bytes (sum of
+// out-degrees of the children of nodes with 1..k-2 vertices) are summed in the
+// same loops from dp[] = out-degrees.
+//
+// K <= 5: a lane per pair (i, j) takes S2 = row i & row j and, at K = 5, counts
+// the edges of S2 bit by bit.  K >= 6: candidate sets are expanded breadth
+// first, sw at a time, level by level: a stage holds up to sw sets and the
+// prefix sums of their sizes; the lanes stride over the elements of a stage's
+// sets, one level finer than a lane per set, whose cost (|S| x |S & row|)
+// varies too much across a wave.  Stage K-4's elements are counted directly
+// (the edges of set & row); earlier stages fill the next one and are resumed
+// when it is done.  Bound by LDS reads of rows and by divergence in the bit
+// loops.  (K = 7 on an 8,192-vertex R-MAT: list intersection, one child at a
+// time, 174 ms; stages 1.44 ms.  R-MAT s17 K = 5 1.52 -> 1.24 ms from reading
+// the rows with LDS instructions instead of generic ones.)
+struct PairSum {
+    unsigned long long cnt, by;  // this lane's share
+};
+// bytes of one stage of sw sets: sets u64[sw * NW] | prefix u32[sw + 1], size,
+// cursor
+__host__ __device__ constexpr int stage_bytes(int sw, int NW) { return sw * NW * 8 + ((sw + 4) & ~1) * 4; }
+
+// position of the r-th set bit (0-based) of m; m has more than r bits
+DEV int select64(uint64_t m, int r) {
+    int pos = 0;
+#pragma unroll
+    for (int sh = 32; sh >= 1; sh >>= 1) {
+        const int c = __popcll(m & ((1ull << sh) - 1));
+        if (r >= c) {
+            r -= c;
+            m >>= sh;
+            pos += sh;
+        }
+    }
+    return pos;
+}
+// the r-th set bit of an NW-word set
+template <int NW, class P64>
+DEV int set_select(P64 s, int r) {
+    int w = 0;
+    uint64_t m = s[0];
+#pragma unroll
+    for (int k = 1; k < NW; k++) {
+        const int c = __popcll(m);
+        if (w == k - 1 && r >= c) {
+            r -= c;
+            w = k;
+            m = s[k];
+        }
+    }
+    return w * 64 + select64(m, r);
+}
+
+// L: everything is in LDS, at the given LDS addresses (else generic pointers)
+template <int W, int NW, bool L>
+__device__ __attribute__((noinline)) PairSum clique_pairs(uint64_t rows_at, uint64_t dp_at, uint64_t pre_at,
+                                                          uint64_t st_at, int K, int cur, int P, int sw) {
+    using P64 = std::conditional_t<L, lds_u64 *, uint64_t *>;
+    using P32 = std::conditional_t<L, lds_u32 *, uint32_t *>;
+    const P64 rows = (P64)(uintptr_t)unil<W>(rows_at);
+    const P32 dp = (P32)(uintptr_t)unil<W>(dp_at), pre = (P32)(uintptr_t)unil<W>(pre_at);
+    const P64 st = (P64)(uintptr_t)unil<W>(st_at);
+    K = uni<W>(K), cur = uni<W>(cur), P = uni<W>(P), sw = uni<W>(sw);
+    auto sync = [&]() {
+        if constexpr (L) lsync();
+        else wsync();
+    };
+    const Grp<W> g;
+    PairSum r{0, 0};
+    // edges inside s above each element; their lower ends' out-degrees to by
+    auto edges = [&](const uint64_t (&s)[NW]) {
+        int pc = 0;
+#pragma unroll
+        for (int w0 = 0; w0 < NW; w0++) {
+            uint64_t m = s[w0];
+            while (m) {
+                const int x = w0 * 64 + __builtin_ctzll(m);
+                m &= m - 1;
+                r.by += (unsigned long long)dp[x];
+#pragma unroll
+                for (int w = 0; w < NW; w++) pc += __popcll(s[w] & rows[x * NW + w]);
+            }
+        }
+        return pc;
+    };
+    int a = 0;
+    if (K <= 5) {
+        for (int t = g.gl; t < P; t += W) {
+            while ((int)pre[a + 1] <= t) a++;
+            const int i = cur + a, j = set_select<NW>(rows + i * NW, t - (int)pre[a]);
+            r.by += (unsigned long long)dp[j];
+            uint64_t s[NW];
+            int pc = 0;
+#pragma unroll
+            for (int w = 0; w < NW; w++) {
+                s[w] = rows[i * NW + w] & rows[j * NW + w];
+                if (K == 4) pc += __popcll(s[w]);
+            }
+            if (K == 5) pc = edges(s);
+            r.cnt += (unsigned long long)pc;
+        }
+        return r;
+    }
+    const int sb = stage_bytes(sw, NW) / 8;  // words of a stage
+    // lane gl's set (gl < sw, else empty) becomes element gl of stage q
+    auto fill = [&](int q, const uint64_t (&s)[NW]) {
+        int n = 0;
+#pragma unroll
+        for (int w = 0; w < NW; w++) {
+            if (g.gl < sw) st[q * sb + g.gl * NW + w] = s[w];
+            n += __popcll(s[w]);
+        }
+        const int ps = g.iscan(n);
+        const P32 pp = (P32)(st + q * sb + sw * NW);
+        if (g.gl < sw) pp[g.gl + 1] = ps;
+        if (g.gl == 0) pp[0] = 0;
+        const int T = g.bcast(ps, W - 1);
+        if (g.gl == 0) pp[sw + 1] = T, pp[sw + 2] = 0;
+        sync();
+        return T;
+    };
+    const int last = K - 6;  // stage whose elements are counted
+    for (int p0 = 0; p0 < P; p0 += sw) {
+        uint64_t s[NW];
+#pragma unroll
+        for (int w = 0; w < NW; w++) s[w] = 0;
+        const int t = p0 + g.gl;
+        if (g.gl < sw && t < P) {
+            while ((int)pre[a + 1] <= t) a++;
+            const int i = cur + a, j = set_select<NW>(rows + i * NW, t - (int)pre[a]);
+            r.by += (unsigned long long)dp[j];
+#pragma unroll
+            for (int w = 0; w < NW; w++) s[w] = rows[i * NW + w] & rows[j * NW + w];
+        }
+        int T = fill(0, s), c = 0, q = 0;
+        while (q >= 0) {
+            const P64 sets = st + q * sb;
+            const P32 pp = (P32)(sets + sw * NW);
+            if (q == last) {
+                int pa = 0;
+                for (int u = g.gl; u < T; u += W) {
+                    while ((int)pp[pa + 1] <= u) pa++;
+                    const P64 S = sets + pa * NW;
+                    const int x = set_select<NW>(S, u - (int)pp[pa]);
+                    r.by += (unsigned long long)dp[x];
+                    uint64_t n[NW];
+#pragma unroll
+                    for (int w = 0; w < NW; w++) n[w] = S[w] & rows[x * NW + w];
+                    r.cnt += (unsigned long long)edges(n);
+                }
+                c = T;
+            }
+            if (c >= T) {
+                q--;
+                if (q >= 0) {
+                    sync();
+                    const P32 up = (P32)(st + q * sb + sw * NW);
+                    T = uni<W>((int)up[sw + 1]);
+                    c = uni<W>((int)up[sw + 2]);
+                }
+                continue;
+            }
+            // the next sw elements of this stage fill the next one
+#pragma unroll
+            for (int w = 0; w < NW; w++) s[w] = 0;
+            const int u = c + g.gl;
+            if (g.gl < sw && u < T) {
+                int lo = 0, hi = sw - 1;  // last set whose prefix is <= u
+                while (lo < hi) {
+                    const int mid = (lo + hi + 1) >> 1;
+                    if ((int)pp[mid] <= u) lo = mid;
+                    else hi = mid - 1;
+                }
+                const P64 S = sets + lo * NW;
+                const int x = set_select<NW>(S, u - (int)pp[lo]);
+                r.by += (unsigned long long)dp[x];
+#pragma unroll
+                for (int w = 0; w < NW; w++) s[w] = S[w] & rows[x * NW + w];
+            }
+            c += sw;
+            if (g.gl == 0) pp[sw + 2] = (uint32_t)c;
+            q++;
+            T = fill(q, s);
+            c = 0;
+        }
+        sync();
+    }
+    return r;
+}
+
 template <int W, int MODE>
 struct Worker {
     Grp<W> g;
@@ -1020,76 +1215,6 @@ struct Worker {
     }
 
     // ---- clique, local bitmap of the root's out-neighbourhood -------------
-    // L = N+(v), d = |L| <= 64*NW.  rows[i*NW + w] bit b: L[64w+b] in N+(L[i]).
-    // Each lane takes first-level children i and walks the deeper levels as
-    // AND/popcount over rows; the loops visit exactly the DFS children of
-    // every node above the last level, so the algorithmic bytes (sum of
-    // out-degrees of the children of nodes with 1..k-2 vertices) are summed
-    // in the same loops from dp[] = out-degrees.
-    // Work of one second-level pair (i, j), j in row i: the (k-2)-level
-    // candidate set S2 = row_i & row_j, then the deeper levels by AND/popcount.
-    template <int NW>
-    DEV void bitmap_pair(const uint64_t *rows, const int32_t *dp, int i, int j, unsigned long long &c,
-                         unsigned long long &by) const {
-        uint64_t S2[NW];
-#pragma unroll
-        for (int w = 0; w < NW; w++) S2[w] = rows[i * NW + w] & rows[j * NW + w];
-        if (K == 4) {
-            int pc = 0;
-#pragma unroll
-            for (int w = 0; w < NW; w++) pc += __popcll(S2[w]);
-            c += (unsigned long long)pc;
-            return;
-        }
-#pragma unroll
-        for (int w2 = 0; w2 < NW; w2++) {
-            uint64_t m2 = S2[w2];
-            while (m2) {
-                const int k = w2 * 64 + __builtin_ctzll(m2);
-                m2 &= m2 - 1;
-                by += (unsigned long long)dp[k];
-                if (K == 5) {
-                    int pc = 0;
-#pragma unroll
-                    for (int w = 0; w < NW; w++) pc += __popcll(S2[w] & rows[k * NW + w]);
-                    c += (unsigned long long)pc;
-                    continue;
-                }
-                uint64_t S3[NW];
-#pragma unroll
-                for (int w = 0; w < NW; w++) S3[w] = S2[w] & rows[k * NW + w];
-                int pc = 0;
-#pragma unroll
-                for (int w3 = 0; w3 < NW; w3++) {
-                    uint64_t m3 = S3[w3];
-                    while (m3) {
-                        const int q = w3 * 64 + __builtin_ctzll(m3);
-                        m3 &= m3 - 1;
-                        by += (unsigned long long)dp[q];
-#pragma unroll
-                        for (int w = 0; w < NW; w++) pc += __popcll(S3[w] & rows[q * NW + w]);
-                    }
-                }
-                c += (unsigned long long)pc;
-            }
-        }
-    }
-
-    // position of the r-th set bit (0-based) of m; m has more than r bits
-    DEV static int select64(uint64_t m, int r) {
-        int pos = 0;
-#pragma unroll
-        for (int sh = 32; sh >= 1; sh >>= 1) {
-            const int c = __popcll(m & ((1ull << sh) - 1));
-            if (r >= c) {
-                r -= c;
-                m >>= sh;
-                pos += sh;
-            }
-        }
-        return pos;
-    }
-
     template <int NW>
     DEV void clique_bitmap_root(int32_t v, int lo, int hi, bool first_piece, bool shared) {
         const int d = odeg(v);
@@ -1137,14 +1262,13 @@ struct Worker {
             build_rows<NW>(v, lo, d, L, rows, dp, pre);
             if (abort) return;
         }
-        // k = 6: a round's pair staging, allocated after the build so that
-        // the build's hash gets the LDS first (both fit there together only
-        // for smaller roots)
-        uint64_t *s2 = nullptr;
-        int32_t *sp = nullptr;
-        if (K == 6) {
-            s2 = (uint64_t *)alloc((int64_t)W * NW * 8);
-            sp = (int32_t *)alloc((int64_t)(W + 1) * 4);
+        // K >= 6: the stages, allocated after the build so that the build's
+        // hash gets the LDS first; as wide as the LDS left allows
+        int sw = W;
+        char *st = nullptr;
+        if (K >= 6) {
+            while (sw > 8 && lds_top + (K - 5) * stage_bytes(sw, NW) > lds_lo + p.lds_per_worker) sw >>= 1;
+            st = alloc((int64_t)(K - 5) * stage_bytes(sw, NW));
             if (abort) return;
         }
         if (shared) {
@@ -1168,11 +1292,11 @@ struct Worker {
                 n = g.bcast(n, 0);
                 if (a >= d) break;
                 if (a == 0 && g.gl == 0) bytes += 4ull * (unsigned long long)d;
-                pair_phase<NW>(R, rows, dp, pre, s2, sp, a, a + n < d ? a + n : d);
+                pair_phase<NW>(R, rows, dp, pre, st, sw, a, a + n < d ? a + n : d);
             }
         } else {
             if (first_piece && g.gl == 0) bytes += 4ull * (unsigned long long)d;
-            pair_phase<NW>(R, rows, dp, pre, s2, sp, lo, hi);
+            pair_phase<NW>(R, rows, dp, pre, st, sw, lo, hi);
         }
         lds_top = R.mark_lds;
         g_top = R.mark_glb;
@@ -1262,11 +1386,12 @@ struct Worker {
 
     // first-level children [lo, hi) in batches of W; each batch is
     // flattened into its (i, j) pairs, which the lanes stride over
+    // (st, sw: the stages of K >= 6)
     template <int NW>
-    // s2 / sp (k = 6 only): LDS staging of a round's W pairs, W x NW words
-    // and W + 1 prefix entries
-    DEV void pair_phase(Lvl &R, const uint64_t *rows, const int32_t *dp, int32_t *pre, uint64_t *s2, int32_t *sp,
-                        int lo, int hi) {
+    DEV void pair_phase(Lvl &R, const uint64_t *rows, const int32_t *dp, int32_t *pre, char *st, int sw, int lo,
+                        int hi) {
+        auto lds = [&](const void *a) { return (const char *)a >= lds_lo && (const char *)a < lds_lo + p.lds_per_worker; };
+        const bool in_lds = lds(rows) && lds(dp) && lds(pre) && (K < 6 || lds(st));
         R.cur = lo;
         R.end = hi;
         unsigned long long by = 0;
@@ -1303,94 +1428,17 @@ struct Worker {
             if (g.gl == 0) pre[0] = 0;
             const int P = g.bcast(sc, take - 1);
             wsync();
-            if (K == 6) {
-                pair_round_k6<NW>(rows, dp, pre, s2, sp, cur, P, by);
-                continue;
-            }
-            int a = 0;
-            for (int t = g.gl; t < P; t += W) {
-                while (pre[a + 1] <= t) a++;
-                const int i = cur + a;
-                const int j = pair_second<NW>(rows, i, t - pre[a]);
-                by += (unsigned long long)dp[j];
-                bitmap_pair<NW>(rows, dp, i, j, cnt, by);
-            }
+            PairSum r;
+            if (in_lds)
+                r = clique_pairs<W, NW, true>(lds_at(rows), lds_at(dp), lds_at(pre), lds_at(st), K, cur, P, sw);
+            else
+                r = clique_pairs<W, NW, false>((uintptr_t)rows, (uintptr_t)dp, (uintptr_t)pre, (uintptr_t)st, K, cur,
+                                               P, sw);
+            cnt += r.cnt;
+            by += r.by;
             wsync();
         }
         bytes += 4ull * by;
-    }
-
-    // the second child of pair r of child i: the r-th set bit of row i
-    template <int NW>
-    DEV static int pair_second(const uint64_t *rows, int i, int r) {
-        int w = 0;
-        uint64_t m = rows[i * NW];
-        while (true) {
-            const int c = __popcll(m);
-            if (r < c || w == NW - 1) break;
-            r -= c;
-            w++;
-            m = rows[i * NW + w];
-        }
-        return w * 64 + select64(m, r);
-    }
-
-    // k = 6: the pairs of a batch, W at a time.  Each lane stages its pair's
-    // common candidates S2 = row i & row j in LDS, then the lanes stride over
-    // the round's (pair, k in S2) triples, each counting the 2-cliques of
-    // S2 & row k above k: one level finer than a lane per pair, whose cost
-    // (|S2| x |S3|) varies too much across the lanes of a wave.
-    template <int NW>
-    DEV void pair_round_k6(const uint64_t *rows, const int32_t *dp, const int32_t *pre, uint64_t *s2, int32_t *sp,
-                           int cur, int P, unsigned long long &by) {
-        int a = 0;
-        for (int t0 = 0; t0 < P; t0 += W) {
-            const int t = t0 + g.gl;
-            int s = 0;
-            if (t < P) {
-                while (pre[a + 1] <= t) a++;
-                const int i = cur + a;
-                const int j = pair_second<NW>(rows, i, t - pre[a]);
-                by += (unsigned long long)dp[j];
-#pragma unroll
-                for (int w = 0; w < NW; w++) {
-                    const uint64_t x = rows[i * NW + w] & rows[j * NW + w];
-                    s2[g.gl * NW + w] = x;
-                    s += __popcll(x);
-                }
-            }
-            const int ps = g.iscan(s);
-            sp[g.gl + 1] = ps;
-            if (g.gl == 0) sp[0] = 0;
-            const int Ts = g.bcast(ps, W - 1);
-            wsync();
-            int pa = 0;
-            unsigned long long c = 0;
-            for (int u = g.gl; u < Ts; u += W) {
-                while (sp[pa + 1] <= u) pa++;
-                const uint64_t *S2 = s2 + pa * NW;
-                const int k = pair_second<NW>(S2, 0, u - sp[pa]);
-                by += (unsigned long long)dp[k];
-                uint64_t S3[NW];
-#pragma unroll
-                for (int w = 0; w < NW; w++) S3[w] = S2[w] & rows[k * NW + w];
-                int pc = 0;
-#pragma unroll
-                for (int w3 = 0; w3 < NW; w3++) {
-                    uint64_t m3 = S3[w3];
-                    while (m3) {
-                        const int q = w3 * 64 + __builtin_ctzll(m3);
-                        m3 &= m3 - 1;
-                        by += (unsigned long long)dp[q];
-#pragma unroll
-                        for (int w = 0; w < NW; w++) pc += __popcll(S3[w] & rows[q * NW + w]);
-                    }
-                }
-                c += (unsigned long long)pc;
-            }
-            cnt += c;
-            wsync();
-        }
     }
 
     // ---- one job ------------------------------------------------------------
@@ -1416,7 +1464,7 @@ struct Worker {
             }
             return;
         }
-        if (!motif && p.bitmap && lvl == 0 && K >= 4 && K <= 6) {
+        if (!motif && p.bitmap && lvl == 0 && K >= 4) {
             const int d = odeg(v0);
             if (d <= 64) {
                 clique_bitmap_root<1>(v0, lo, hi, first_piece, shared);

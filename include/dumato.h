@@ -54,7 +54,7 @@ typedef struct dm_config {
     int32_t per_root;        /* 1: per-root subgraph counts (dm_last_root_counts) */
     int32_t root_begin;      /* enumerate roots [root_begin, root_end) only... */
     int32_t root_end;        /* ...(original vertex ids); root_end <= 0: all */
-    int32_t clique_bitmap;   /* 1: k=4..6 cliques of roots with out-degree <= 256 count
+    int32_t clique_bitmap;   /* 1: k >= 4 cliques of roots with out-degree <= 256 count
                                 on a local adjacency bitmap; 0: list intersections */
     int32_t repartition;     /* 1: compute the static partition afresh (features,
                                 inference, binning) instead of reusing the cached one */

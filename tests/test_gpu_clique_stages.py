@@ -1,0 +1,59 @@
+"""The bitmap clique path's stages (k >= 6, every k past 6 included): set
+widths of 1, 2 and 4 words, stages narrowed by small LDS slices or in the
+arena, every worker width; counts and algorithmic bytes against the oracle or
+closed forms."""
+import math
+
+import numpy as np
+import pytest
+
+import dumato_amd as dm
+from oracle import pyoracle as O
+from tests import graphs as G
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(64, 0), (64, 256), (64, 4096), (32, 0), (16, 1024), (8, 0)]
+
+
+@pytest.mark.parametrize("n,p", [(60, 0.5), (110, 0.4), (170, 0.25)])
+@pytest.mark.parametrize("w,lds", SHAPES)
+def test_random_graphs_against_the_oracle(n, p, w, lds):
+    s, d, nv = G.gnp(n, p, 300 + n)
+    g, ref = dm.Graph.from_edges(s, d, nv), O.csr_from_edges(s, d, nv)
+    _, ro = O.relabel(ref, oriented=True)
+    for k in (4, 5, 6, 7, 8, 9):
+        print("case gnp n=%d clique k=%d w=%d lds=%d" % (n, k, w, lds), flush=True)
+        assert g.clique_count(k, dm.config(vwave=w, lds_bytes=lds, watchdog_s=60.0)) == O.clique_count(ref, k)
+        assert g.last_stats()["alg_bytes"] == O.clique_bytes(ro, k)
+
+
+def bipartite_with_clique(a, b, c):
+    """Complete bipartite graph (sides a and b) plus a clique on c vertices of
+    side a: wide out-neighbourhoods (b) that hold few edges."""
+    x, y = np.meshgrid(np.arange(a), a + np.arange(b), indexing="ij")
+    i, j = np.triu_indices(c, 1)
+    src = np.concatenate([x.ravel(), a - c + i])
+    dst = np.concatenate([y.ravel(), a - c + j])
+    return src.astype(np.int32), dst.astype(np.int32), a + b
+
+
+@pytest.mark.parametrize("b", [100, 128, 129, 250, 256, 257])
+def test_wide_roots_closed_form(b):
+    # word counts 2 and 4, the last bitmap root and the first past it
+    c = 11
+    s, d, nv = bipartite_with_clique(b, b, c)
+    g = dm.Graph.from_edges(s, d, nv)
+    for k in (4, 5, 6, 7, 9, 12):
+        want = math.comb(c, k) + b * math.comb(c, k - 1)
+        for w, lds in ((64, 0), (64, 2048), (16, 0)):
+            print("case bipartite b=%d clique k=%d w=%d lds=%d" % (b, k, w, lds), flush=True)
+            assert g.clique_count(k, dm.config(vwave=w, lds_bytes=lds, watchdog_s=60.0)) == want
+
+
+def test_complete_graph_every_size():
+    s, d, n = G.complete(26)
+    g = dm.Graph.from_edges(s, d, n)
+    for k in range(3, 13):
+        print("case K26 clique k=%d" % k, flush=True)
+        assert g.clique_count(k, dm.config(watchdog_s=60.0)) == math.comb(26, k)
