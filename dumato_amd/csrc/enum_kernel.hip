@@ -352,6 +352,53 @@ DEV int wave_lower_bound(const Grp<W> &g, const int32_t *a, int n, int32_t x) {
     return lo;
 }
 
+// The lanes' lists adj[os, os + len) laid end to end, f(entry, tag of its
+// list) called for every entry, W consecutive ones at a time (U steps' loads in
+// flight; f(none, 0) where the lists end).  recs: list start and tag, by list;
+// bits: a set bit where a list starts, so the list of an entry is a popcount.
+template <int W, class F>
+DEV void stream_lists(const Grp<W> &g, lds_u64 *recs, lds_u64 *bits, const int32_t *adj, int64_t os, int len, int tag,
+                      int32_t none, F f) {
+    const uint64_t mx = g.ballot(len > 0);
+    const int sc = g.iscan(len), pre = sc - len;
+    const int T = g.bcast(sc, W - 1);
+    if (len > 0) recs[g.below(mx)] = ((uint64_t)(os - pre) & 0xffffffffffffffull) | ((uint64_t)tag << 56);
+    for (int p0 = 0; p0 < T; p0 += kLeafCap) {
+        const int pe = T - p0 < kLeafCap ? T : p0 + kLeafCap;
+        for (int w = g.gl; w < kLeafCap / 64; w += W) bits[w] = 0;
+        lsync();
+        if (len > 0 && pre >= p0 && pre < pe) lor(bits + ((pre - p0) >> 6), 1ull << ((pre - p0) & 63));
+        // lists that started before this chunk
+        int own0 = __popcll(g.ballot(len > 0 && pre < p0)) - 1;
+        lsync();
+        constexpr int U = 4;
+        for (int t0 = p0; t0 < pe; t0 += U * W) {
+            int32_t ys[U];
+            int cm[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int t = t0 + u * W + g.gl;
+                const int o = t0 + u * W - p0;
+                uint64_t seg = o < kLeafCap ? bits[o >> 6] : 0;
+                if constexpr (W == 64) seg = unil<W>(seg);
+                else seg = (seg >> (o & 63)) & ((1ull << W) - 1);
+                const int own = own0 + __popcll(seg & ((2ull << g.gl) - 1));
+                own0 += __popcll(seg);
+                ys[u] = none;
+                cm[u] = 0;
+                if (t < pe) {
+                    const uint64_t rec = recs[own];
+                    cm[u] = (int)(rec >> 56);
+                    ys[u] = adj[((int64_t)(rec << 8) >> 8) + t];
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) f(ys[u], cm[u]);
+        }
+        lsync();
+    }
+}
+
 // The counts of one leaf node, added to the class counters at LDS address shist_at.  (c, pmc):
 // the child of the parent's list (puid, pupm, pnu) that makes the node, its
 // mask; K = 3: the root alone, c = id[0], whose elements [lo, hi) are taken
@@ -420,9 +467,8 @@ __device__ __attribute__((noinline)) LeafSum motif_leaf(const int64_t *off, cons
     for (int j = g.gl; j < npm; j += W) nm[j] = 0, qs[j] = 0;
     lsync();
 
-    // elements of U, W at a time: n_i and q_i, then their out-lists laid end
-    // to end (recs: list start and mask, by list; bits: a set bit per list
-    // start), over which the lanes stride
+    // elements of U, W at a time: n_i and q_i, then their out-lists (v0, in
+    // place of an entry past their end, is never in U)
     uint32_t nnew = 0, enew = 0;  // class newc / (newc, newc), counted in registers
     unsigned long long qnew = 0, by = 0, leaves = 0, rpairs = 0;
     lds_u32 *const ecopy = e + (g.gl & (copies - 1)) * ne;
@@ -458,51 +504,14 @@ __device__ __attribute__((noinline)) LeafSum motif_leaf(const int64_t *off, cons
                 if (root) rpairs += (unsigned long long)(tot - 1 - j);
             }
         }
-        const uint64_t mx = g.ballot(len > 0);
-        const int sc = g.iscan(len), pre = sc - len;
-        const int T = g.bcast(sc, W - 1);
-        if (len > 0) recs[g.below(mx)] = ((uint64_t)(os - pre) & 0xffffffffffffffull) | ((uint64_t)cx << 56);
-        for (int p0 = 0; p0 < T; p0 += kLeafCap) {
-            const int pe = T - p0 < kLeafCap ? T : p0 + kLeafCap;
-            for (int w = g.gl; w < kLeafCap / 64; w += W) bits[w] = 0;
-            lsync();
-            if (len > 0 && pre >= p0 && pre < pe) lor(bits + ((pre - p0) >> 6), 1ull << ((pre - p0) & 63));
-            // lists that started before this chunk
-            int own0 = __popcll(g.ballot(len > 0 && pre < p0)) - 1;
-            lsync();
-            constexpr int U = 4;
-            for (int t0 = p0; t0 < pe; t0 += U * W) {
-                int32_t ys[U];
-                int cm[U];
-#pragma unroll
-                for (int u = 0; u < U; u++) {
-                    const int t = t0 + u * W + g.gl;
-                    const int o = t0 + u * W - p0;
-                    uint64_t seg = o < kLeafCap ? bits[o >> 6] : 0;
-                    if constexpr (W == 64) seg = unil<W>(seg);
-                    else seg = (seg >> (o & 63)) & ((1ull << W) - 1);
-                    const int own = own0 + __popcll(seg & ((2ull << g.gl) - 1));
-                    own0 += __popcll(seg);
-                    ys[u] = v0;  // no element: v0 is never in U
-                    cm[u] = 0;
-                    if (t < pe) {
-                        const uint64_t rec = recs[own];
-                        cm[u] = (int)(rec >> 56);
-                        ys[u] = adj[((int64_t)(rec << 8) >> 8) + t];
-                    }
-                }
-#pragma unroll
-                for (int u = 0; u < U; u++) {
-                    const int cd = find(ys[u]);
-                    if (cd) {
-                        const int cy = cd & 31, a = cm[u] > cy ? cm[u] : cy, z = cm[u] > cy ? cy : cm[u];
-                        if (a == newc && z == newc) enew++;
-                        else ladd(ecopy + (__umul24(a, a + 1) >> 1) + z, 1u);
-                    }
-                }
+        stream_lists(g, recs, bits, adj, os, len, cx, v0, [&](int32_t y, int mx) {
+            const int cd = find(y);
+            if (cd) {
+                const int cy = cd & 31, a = mx > cy ? mx : cy, z = mx > cy ? cy : mx;
+                if (a == newc && z == newc) enew++;
+                else ladd(ecopy + (__umul24(a, a + 1) >> 1) + z, 1u);
             }
-            lsync();
-        }
+        });
     }
     if (nnew) ladd(nm + newc, nnew);
     if (qnew) ladd(qs + newc, (uint64_t)qnew);
@@ -544,6 +553,55 @@ __device__ __attribute__((noinline)) LeafSum motif_leaf(const int64_t *off, cons
     r.cnt = leaves;
     // the node's own bytes (at k = 3 the root's are counted by the caller)
     r.bytes = 4ull * by + 4ull * (K - 1) * leaves + (!root && g.gl == 0 ? 4ull * (unsigned long long)sdeg : 0ull);
+    return r;
+}
+
+// Triangles of root v0 (k = 3): the edges {u, y} inside N+(v0), u one of its
+// children [lo, hi), found from the out-lists N+(u) laid end to end over the
+// lanes and tested against a table of N+(v0), as in the motif leaf.  first:
+// the call that builds the table (the root's later calls find it in place).
+// Bound by the table reads (R-MAT s18 of edge factor 16: 659 M tests a call,
+// 83 M triangles; one child at a time, each entry searched in the longer list:
+// 5.19 -> 1.81 ms).  lds_at: recs u64[W] | bits u64[kLeafCap / 64] | table.
+constexpr int kTriFixed = 64 * 8 + kLeafCap / 8;
+struct TriSum {
+    unsigned long long cnt, by;  // this lane's share; by: out-degrees of the children
+};
+template <int W>
+__device__ __attribute__((noinline)) TriSum triangles(const int64_t *off, const int32_t *adj, const int64_t *ostart,
+                                                      uint32_t at, int b, int32_t v0, int lo, int hi, bool first,
+                                                      bool &ok) {
+    off = unil<W>(off), adj = unil<W>(adj), ostart = unil<W>(ostart);
+    b = uni<W>(b), v0 = uni<W>(v0), lo = uni<W>(lo), hi = uni<W>(hi);
+    const Grp<W> g;
+    lds_u64 *const recs = (lds_u64 *)(uintptr_t)(uint32_t)uni<W>((int)at);
+    lds_u64 *const bits = recs + W;
+    LeafTab<true> tab;
+    tab.t = (lds_u32 *)(recs + kTriFixed / 8);
+    tab.b = b, tab.sh = 32 - b, tab.mul = 0x9E3779B1u;
+    const int64_t ls = unil<W>(ostart[v0]);
+    const int32_t *const L = adj + ls;
+    TriSum r{0, 0};
+    ok = true;
+    if (first) {
+        const int d = (int)(unil<W>(off[v0 + 1]) - ls);
+        ok = tab.build(g, L, nullptr, 0, v0, L, d, 1);
+        if (!ok) return r;
+    }
+    for (int j0 = lo; j0 < hi; j0 += W) {
+        const int j = j0 + g.gl;
+        int len = 0;
+        int64_t os = 0;
+        if (j < hi) {
+            const int32_t u = L[j];
+            os = ostart[u];
+            len = (int)(off[u + 1] - os);
+            r.by += (unsigned long long)len;
+        }
+        uint32_t found = 0;
+        stream_lists(g, recs, bits, adj, os, len, 0, v0, [&](int32_t y, int) { found += tab.find(y) ? 1 : 0; });
+        r.cnt += found;
+    }
     return r;
 }
 
@@ -1214,6 +1272,34 @@ struct Worker {
         }
     }
 
+    // k = 3: the root's children [lo, hi), a wave of them per donation check;
+    // false when N+(v) does not fit an LDS table
+    DEV bool triangle_root(int lo, int hi) {
+        Lvl &R = ws.lv()[0];
+        const int d = R.nu;
+        int b = 7;
+        while (3 * (2 << b) < 5 * d) b++;  // at most 3/5 full
+        if (kTriFixed + (8 << b) > p.lds_per_worker) return false;
+        R.cur = lo;
+        R.end = hi < d ? hi : d;
+        for (bool first = true;; first = false) {
+            if (check_abort()) return true;
+            maybe_donate(1);
+            const int cur = uni<W>(R.cur), end = uni<W>(R.end);
+            if (cur >= end) return true;
+            const int to = end - cur < W ? end : cur + W;
+            R.cur = to;
+            bool ok;
+            const TriSum r = triangles<W>(p.off, p.adj, p.ostart, lds_at(lds_lo), b, v0, cur, to, first, ok);
+            if (!ok) {
+                R.cur = cur;
+                return false;
+            }
+            cnt += r.cnt;
+            bytes += 4ull * r.by;
+        }
+    }
+
     // ---- clique, local bitmap of the root's out-neighbourhood -------------
     template <int NW>
     DEV void clique_bitmap_root(int32_t v, int lo, int hi, bool first_piece, bool shared) {
@@ -1510,6 +1596,7 @@ struct Worker {
         while (k >= lvl) {
             if (check_abort()) return;
             Lvl &L = ws.lv()[k];
+            if (!motif && K == 3 && triangle_root(L.cur, L.end)) return;
             if (k == K - 3) {
                 // a motif job comes here only at k = 3, whose root is the leaf
                 if (motif) motif_leaf_node(-1, 0, L.cur, L.end);
