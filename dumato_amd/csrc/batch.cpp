@@ -65,8 +65,8 @@ struct dm_batch {
     size_t sq_jobs_cap = 0;
     int32_t *d_sq_cur = nullptr;
     size_t sq_cur_cap = 0;
-    unsigned long long *d_qmask = nullptr;  // non-empty static queues (shared by the phases)
-    size_t qmask_cap = 0;
+    unsigned long long *d_mail = nullptr;  // the blocks' mailboxes (shared by the phases)
+    size_t mail_cap = 0;
     unsigned long long *d_results = nullptr;
     size_t results_cap = 0;
     dm::QueryDesc *d_qd = nullptr;
@@ -229,8 +229,7 @@ static int batch_build(dm_batch *b, const std::vector<dm_query> &qs, const dm_co
     const int sm = cfg.steal_min ? cfg.steal_min : (b->tuned_steal_min ? b->tuned_steal_min : 2);
     if (b->exec && b->plan.same(qs, cfg, vw, lds, sm, threads)) return DM_OK;
     drop_graph(b);
-    // phases: (mode, kmax, per-worker class slots) per family present; a
-    // single query keeps the batch's per-worker counters (mode 2)
+    // phases: (mode, kmax, per-worker class slots) per family present
     struct Phase {
         int mode, kmax, wslots, blocks, workers, lds;
         size_t lds_total;
@@ -244,7 +243,7 @@ static int batch_build(dm_batch *b, const std::vector<dm_query> &qs, const dm_co
         if (!has[f]) continue;
         Phase P;
         P.kmax = kmax_f[f];
-        P.mode = qs.size() == 1 ? 2 : f == 1 ? launch_mode(true, P.kmax) : 0;
+        P.mode = launch_mode(f == 1, P.kmax);
         P.wslots = f == 1 ? hslots : 0;
         for (size_t i = 0; i < qs.size(); i++)
             if ((qs[i].motif ? 1 : 0) == f) {
@@ -287,7 +286,7 @@ static int batch_build(dm_batch *b, const std::vector<dm_query> &qs, const dm_co
     if ((r = dev_grow(b->d_sq_off, b->sq_off_cap, sq_total))) return r;
     if ((r = dev_grow(b->d_sq_jobs, b->sq_jobs_cap, std::max<size_t>(jobs_total, 4)))) return r;
     if ((r = dev_grow(b->d_sq_cur, b->sq_cur_cap, (size_t)max_workers))) return r;
-    if ((r = dev_grow(b->d_qmask, b->qmask_cap, (size_t)qmask_words(max_workers, 1)))) return r;
+    if ((r = dev_grow(b->d_mail, b->mail_cap, (size_t)max_workers * kMailStride))) return r;
     if ((r = dev_grow(b->d_results, b->results_cap, b->nres))) return r;
     if ((r = dev_grow(b->d_qd, b->qd_cap, qs.size()))) return r;
     if ((r = dev_grow(b->d_done, b->done_cap, qs.size()))) return r;
@@ -332,9 +331,10 @@ static int batch_build(dm_batch *b, const std::vector<dm_query> &qs, const dm_co
         p.sq_off = b->d_sq_off + o_off;
         p.sq_jobs = b->d_sq_jobs + o_jobs;
         p.sq_cur = b->d_sq_cur;
-        p.qmask = P.mode == 1 || P.mode == 3 ? b->d_qmask : nullptr;  // motif phases only, as in single-graph calls
+        p.res_copies = 1;
         p.q = d->d_q;
         p.q_cap = (uint32_t)d->q_cap_alloc;
+        p.mail = b->d_mail;
         p.epoch = d->d_epoch;
         p.start_ticks = b->d_start;
         p.sc = b->d_sc + pi;
@@ -357,12 +357,11 @@ static int batch_build(dm_batch *b, const std::vector<dm_query> &qs, const dm_co
     for (size_t pi = 0; pi < ph.size() && !rr; pi++) {
         const Phase &P = ph[pi];
         const int64_t njobs = (int64_t)P.sq_jobs.size() / 4;
-        int queues = 0;
-        for (size_t w = 0; w + 1 < P.sq_off.size(); w++) queues += P.sq_off[w + 1] > P.sq_off[w] ? 1 : 0;
         EnumParams ip = params[pi];
         if (pi > 0) ip.start_ticks = nullptr;
-        rr = enum_init_launch(ip, (unsigned long long)njobs, queues, d->d_epoch, pi == 0 ? b->d_results : nullptr,
-                              pi == 0 ? b->nres : 0, pi == 0 ? b->d_done : nullptr, pi == 0 ? (int)qs.size() : 0, s);
+        rr = enum_init_launch(ip, (unsigned long long)njobs, d->d_epoch, pi == 0 ? b->d_results : nullptr,
+                              pi == 0 ? b->nres : 0, pi == 0 ? b->d_done : nullptr, pi == 0 ? (int)qs.size() : 0,
+                              P.blocks, s);
         if (!rr && njobs > 0) rr = enum_launch(params[pi], P.mode, vw, P.blocks, threads, P.lds_total, s);
     }
     hipError_t ce = hipStreamEndCapture(s, &b->graph);
@@ -414,10 +413,11 @@ static int batch_run(dm_batch *b, const std::vector<dm_query> &qs, const dm_conf
     HIPCHK(hipEventElapsedTime(&kms, d->ev0, d->ev1));
     // both phases' counters: sums, maxima, and the timeline of the last phase
     // measured from the first one's start
-    SchedCounters sc1 = scs[0];
+    SchedStats sc1 = sched_totals(scs[0]);
+    int error = scs[0].error;
     for (int pi = 1; pi < b->nphases; pi++) {
-        const SchedCounters &c = scs[pi];
-        if (!sc1.error) sc1.error = c.error;
+        const SchedStats c = sched_totals(scs[pi]);
+        if (!error) error = scs[pi].error;
         sc1.alg_bytes += c.alg_bytes;
         sc1.donations += c.donations;
         sc1.jobs += c.jobs;
@@ -430,7 +430,7 @@ static int batch_run(dm_batch *b, const std::vector<dm_query> &qs, const dm_conf
         sc1.t_last_job = c.t_last_job;
         sc1.t_exit = c.t_exit;
     }
-    if (sc1.error) return device_error(sc1.error, "batch kernel");
+    if (error) return device_error(error, "batch kernel");
     uint64_t total = 0;
     for (size_t i = 0; i < b->nres; i++) total += res[i];
     if (results)
@@ -623,7 +623,7 @@ int dm_batch_num_results(const dm_batch *b, const dm_query *queries, size_t nq, 
 void dm_batch_free(dm_batch *b) {
     if (!b) return;
     drop_graph(b);
-    void *bufs[] = {b->d_arena, b->d_sq_off, b->d_sq_jobs, b->d_sq_cur, b->d_qmask, b->d_results,
+    void *bufs[] = {b->d_arena, b->d_sq_off, b->d_sq_jobs, b->d_sq_cur, b->d_mail, b->d_results,
                     b->d_qd, b->d_done, b->d_start, b->d_sc};
     for (void *p : bufs)
         if (p) (void)hipFree(p);

@@ -29,11 +29,11 @@
 //     and the pair's adjacency through the class table.  One pass over the
 //     out-neighbours N+(x) of U_{K-3}'s elements finds the edges inside U_{K-3}
 //     (motif_leaf); everything else is counted in closed form.
-//   * Work: static per-worker queues of (root, lo, hi) jobs, stealing of
-//     other workers' static jobs, and donation of the lowest level's
-//     remaining children to a device queue when workers are idle (the
-//     reference's donate(), src/main/DuMatoCPU.cu:463-539, done on the device
-//     instead of by the host).
+//   * Work: static per-worker queues of (root, lo, hi) jobs.  A worker that
+//     runs out asks a random block through the block's mailbox; a busy worker
+//     there answers with half of its static jobs, or half of the remaining
+//     children of its job's lowest level (the reference's donate(),
+//     src/main/DuMatoCPU.cu:463-539, done on the device instead of by the host).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -140,6 +140,10 @@ DEV void lsync() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
 // LDS words addressed as such (ds instructions; a generic pointer takes flat ones)
 using lds_u32 = __attribute__((address_space(3))) uint32_t;
 using lds_u64 = __attribute__((address_space(3))) uint64_t;
+// The atomic that returned x has been performed before any access that
+// follows in the program (its result is waited for here).
+template <class T>
+DEV void landed(T &x) { asm volatile("" : "+v"(x)::"memory"); }
 // LDS address of a generic pointer into LDS
 DEV uint32_t lds_at(const void *a) { return (uint32_t)(uintptr_t)(lds_u32 *)a; }
 template <class P, class T>
@@ -799,13 +803,19 @@ __device__ __attribute__((noinline)) PairSum clique_pairs(uint64_t rows_at, uint
     }
     return r;
 }
+// Shared by the workers of a block.
+struct BlockLDS {
+    int32_t busy;      // workers that have a job or static jobs left
+    uint32_t pending;  // finished jobs not yet subtracted from the launch's count
+    int32_t pad[2];
+};
 
 template <int W, int MODE>
 struct Worker {
     Grp<W> g;
     const EnumParams &p;
     WorkerLDS ws;
-    unsigned long long *shist;       // class counters the leaf phase adds to
+    unsigned long long *shist;  // class counters the leaf phase adds to
     const uint16_t *lut;
     int qid;
     int32_t qword;  // the current job's query word (query index | donation threshold)
@@ -820,18 +830,19 @@ struct Worker {
     int steps;
     unsigned long long cnt;    // per-lane partial count of the current job
     unsigned long long bytes;  // per-lane partial algorithmic bytes
-    // finished jobs not yet subtracted from the shared outstanding count
-    // (lane 0's copy is the one that counts); flushed when the worker runs
-    // out of work, so the count never drops below the unfinished jobs
-    uint32_t pending;
     int range_hi;  // end of the current range job's roots (v0 + 1 otherwise)
     uint64_t t_start;
-    uint64_t last_poll;  // wall clock of the last donation check
-    uint32_t polls;      // donation checks so far (lane 0's count)
+    uint64_t last_poll;  // wall clock of the last request check
+    int poll_shift;      // the check period doubles while nobody asks
+    BlockLDS *blk;
+    // static queue: jobs [own_cur, own_end) of queue records own_base.. are
+    // this worker's; a queue shared by a group still has to be claimed
+    int64_t own_base;
+    int own_cur, own_end;
+    int own_queue;       // the queue's cursor slot, -1 once it is exhausted
     bool abort;
-    DEV Worker(const EnumParams &p_, WorkerLDS ws_, unsigned long long *sh_, char *lds_slice,
-               int wid)
-        : p(p_), ws(ws_), shist(sh_) {
+    DEV Worker(const EnumParams &p_, WorkerLDS ws_, unsigned long long *sh_, char *lds_slice, BlockLDS *blk_, int wid)
+        : p(p_), ws(ws_), shist(sh_), blk(blk_) {
         lds_lo = lds_top = lds_slice;
         g_lo = g_top = p.arena + (int64_t)wid * p.arena_per_worker;
         K = 0;
@@ -843,12 +854,11 @@ struct Worker {
         epoch = (uint32_t)*p.epoch;
         steps = 0;
         cnt = bytes = 0;
-        pending = 0;
         range_hi = 0;
         abort = false;
         t_start = now_ticks();
         last_poll = t_start;
-        polls = 0;
+        poll_shift = 0;
     }
 
     // ---- helpers -----------------------------------------------------------
@@ -902,21 +912,36 @@ struct Worker {
     }
 
     // ---- donation --------------------------------------------------------------
-    // Donated jobs are published without fences: each of a job's 16 words is
-    // one 64-bit agent-scope atomic store tagged with the launch epoch in the
-    // high half; a reader accepts the slot once all 16 tags match.
-    // Boundary j (0 <= j <= parts) when [cur, end) is cut into `parts`
-    // pieces of equal estimated work.  A clique child i of a list of n
-    // candidates roots about (n - i)^e subtrees, e = K - 3 - l; motif
+    // An idle worker asks: it writes its request into the mailbox of a random
+    // block (one line per block, kMailSlots requests) and waits for the job in
+    // its own slot (one line per worker).  A busy worker looks at its own
+    // block's mailbox now and then and divides what it has left between itself
+    // and the askers.  No line is shared by more than a block and the few
+    // workers asking it; the only word that every block updates is the launch's
+    // count of unfinished jobs, when its last worker runs out of work.
+    // (Device-scope accesses to one line serialise at about 8 ns.  With one
+    // ticket word, one count and one static-work counter polled by every idle
+    // worker, a busy worker's own accesses waited behind the polls: a 3,301-vertex
+    // sparse graph's k = 5 motifs took 13 worker-seconds with 6,144 workers, 0.8
+    // with 1,024; the mailboxes take it from 1.75 to 0.58 ms, ER 5K k = 4 from
+    // 0.91 to 0.37, Chung-Lu 18K k = 4 from 2.12 to 1.45, a mixed batch from 31
+    // to 13-17 ms.)
+    //
+    // A job is published without fences: each of its 16 words is one 64-bit
+    // agent-scope atomic store with the request's tag in the high half; the
+    // reader accepts the slot once all 16 tags match.
+
+    // Boundary j (0 <= j <= parts) when the children [cur, end) of level l are
+    // cut into `parts` pieces of equal estimated work.  A clique child i of a
+    // list of n candidates roots about (n - i)^e subtrees, e = K - 3 - l; motif
     // children and the leaf level count as equal.  Every piece keeps at least
     // one child (end - cur >= parts).
     DEV int split_at(int l, int cur, int end, int j, int parts) const {
         if (j <= 0) return cur;
         if (j >= parts) return end;
-        const bool clique = MODE == 0 || (MODE == 2 && !qmotif);
         const int e = K - 3 - l;
         int m;
-        if (!clique || e < 1) {
+        if (MODE == 1 || e < 1) {
             m = cur + (int)(((int64_t)(end - cur) * j) / parts);
         } else {
             const float n = (float)ws.lv()[l].nu;
@@ -931,107 +956,129 @@ struct Worker {
         return m;
     }
 
-    // Publishes up to P jobs for the children [cur, end) of level lvl: the
-    // range is cut into np + 1 pieces of equal estimated work, np <= P as the
-    // queue allows, and all but the first are queued.  Returns the end of the
-    // piece the worker keeps (end itself when nothing was queued).
-    DEV int push_pieces(int lvl, int cur, int end, int P) {
-        uint32_t slot = 0;
-        const int np = reserve_slots(P, slot);
-        if (np == 0) return end;
-        const uint64_t tag = (uint64_t)epoch << 32;
-        for (int idx = g.gl; idx < np * kJobWords; idx += W) {
-            const int r = idx / kJobWords, j = idx - r * kJobWords;
-            int32_t v;
-            if (j == 0) v = lvl;
-            else if (j == 1) v = split_at(lvl, cur, end, 1 + r, np + 1);
-            else if (j == 2) v = split_at(lvl, cur, end, 2 + r, np + 1);
-            else if (j == 3) v = qword;
-            else v = (j - 4 <= lvl) ? ws.lv()[j - 4].vtx : -1;
-            __hip_atomic_store(p.q[slot + r].w + j, tag | (uint32_t)v, __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
+    DEV unsigned long long *mailbox(int b) const { return p.mail + (size_t)b * kMailStride; }
+
+    // Requests waiting in this block's mailbox, looked for at most once per
+    // period, which doubles (16-fold at most) while none comes: their number;
+    // rq: lane i's own (i < kMailSlots; 0: none).
+    DEV int requests(unsigned long long &rq) {
+        const uint64_t now = now_ticks();
+        if (now - last_poll < (p.poll_ticks << poll_shift)) return 0;
+        last_poll = now;
+        rq = 0;
+        if (g.gl < kMailSlots) {
+            unsigned long long *const m = mailbox(blockIdx.x) + g.gl;
+            rq = __hip_atomic_load(m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            // (two workers' changes of state can pass each other)
+            if (rq == kMailIdle) rq = 0, (void)atomicCAS(m, kMailIdle, 0ull);
         }
-        if (g.gl == 0) ws.st()[kStDonated] += (unsigned long long)np;
-        return split_at(lvl, cur, end, 1, np + 1);
+        const int n = __popcll(g.ballot(rq != 0));
+        poll_shift = n ? 0 : poll_shift < 4 ? poll_shift + 1 : 4;
+        return n;
     }
 
-    // Queues the roots [lo, hi) of this worker's range job as a range job
-    // of their own; returns false when the queue is full.
-    DEV bool push_range(int lo, int hi) {
-        uint32_t slot = 0;
-        if (reserve_slots(1, slot) == 0) return false;
-        const uint64_t tag = (uint64_t)epoch << 32;
-        for (int j = g.gl; j < kJobWords; j += W) {
-            const int32_t v = j == 1 ? -1 : j == 2 ? hi : j == 3 ? qword : j == 4 ? lo : j == 0 ? 0 : -1;
-            __hip_atomic_store(p.q[slot].w + j, tag | (uint32_t)v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        if (g.gl == 0) ws.st()[kStDonated]++;
-        return true;
-    }
-
-    // Reserves up to P consecutive queue slots (as many as the queue has)
-    // and counts the jobs that will fill them as outstanding before they
-    // become visible, so that outstanding cannot reach zero while they wait;
-    // finished jobs not yet subtracted stand in for some of them.  Returns
-    // the number reserved (the same on every lane) and the first slot.
-    DEV int reserve_slots(int P, uint32_t &slot_out) {
-        int np = 0;
-        uint32_t slot = 0;
-        if (g.gl == 0) {
-            const uint32_t t = (uint32_t)__hip_atomic_load(&p.sc->q_ht, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (t < p.q_cap) {
-                const uint32_t t0 = (uint32_t)atomicAdd(&p.sc->q_ht, (unsigned long long)P);
-                if (t0 < p.q_cap) {
-                    np = (int)(p.q_cap - t0) < P ? (int)(p.q_cap - t0) : P;
-                    slot = t0;
-                    const uint32_t own = pending < (uint32_t)np ? pending : (uint32_t)np;
-                    pending -= own;
-                    if ((uint32_t)np > own) atomicAdd(&p.sc->outstanding, (unsigned long long)(np - own));
-                }
+    // Takes up to `most` of the requests out of the mailbox (not those that
+    // another worker of the block took first or whose asker gave up): their
+    // number; the others' lanes get rq = 0.  fresh: the answers are new jobs,
+    // counted as outstanding before they become visible, so that the count
+    // cannot reach zero while they wait (finished jobs not yet subtracted
+    // stand in for some of them).
+    DEV int accept(unsigned long long &rq, int most, bool fresh) {
+        if (g.below(g.ballot(rq != 0)) >= most) rq = 0;
+        if (rq != 0 && atomicCAS(mailbox(blockIdx.x) + g.gl, rq, 0ull) != rq) rq = 0;
+        const int n = __popcll(g.ballot(rq != 0));
+        if (fresh && n && g.gl == 0) {
+            uint32_t have = blk->pending, use = 0;
+            do {
+                use = have < (uint32_t)n ? have : (uint32_t)n;
+            } while (use && !__hip_atomic_compare_exchange_strong(&blk->pending, &have, have - use, __ATOMIC_RELAXED,
+                                                                  __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+            if (use < (uint32_t)n) {
+                unsigned long long old = atomicAdd(&p.sc->outstanding, (unsigned long long)(n - use));
+                landed(old);
             }
         }
-        np = g.bcast(np, 0);
-        slot_out = (uint32_t)g.bcast((int)slot, 0);
-        return np;
+        return n;
     }
 
-    // Donate remaining children when tickets wait for jobs: the shallowest
-    // level of the job with enough children left is cut into one piece per
-    // waiting ticket (at most kMaxPieces) plus the piece this worker keeps.
-    static constexpr int kMaxPieces = 8;
-    // Waiting tickets (at most kMaxPieces), checked at most every poll
-    // period; 0 when stealing is off.  A worker takes a ticket once no
-    // static job is left.  The check is a hint: most checks are a
-    // workgroup-scope load that may be served from this CU's cache and lag,
-    // which only delays a donation; the push itself is exact.
-    DEV int donation_demand() {
-        if (!p.steal) return 0;
-        const uint64_t now = now_ticks();
-        if (now - last_poll < p.poll_ticks) return 0;
-        last_poll = now;
-        int want = 0;
-        if (g.gl == 0) {
-            // every 4th check reads through to the device scope: a worker
-            // whose loop touches little global memory keeps the line in its
-            // CU's cache, and a cached copy could hide demand indefinitely
-            const unsigned long long ht =
-                (++polls & 3) == 0 ? __hip_atomic_load(&p.sc->q_ht, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                                   : __hip_atomic_load(&p.sc->q_ht, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            const uint32_t h = (uint32_t)(ht >> 32), t = (uint32_t)ht;
-            want = h > t ? (int)(h - t < (uint32_t)kMaxPieces ? h - t : (uint32_t)kMaxPieces) : 0;
+    // Writes answer r = 0.. to the slot of the r-th accepted asker: words
+    // f(r, 0..15).
+    template <class F>
+    DEV void answer(unsigned long long rq, F f) {
+        uint64_t left = g.ballot(rq != 0);
+        for (int r = 0; left; r++) {
+            const unsigned long long q = g.bcast64(rq, __builtin_ctzll(left));
+            left &= left - 1;
+            uint64_t *const dst = p.q[(uint32_t)q - 1].w;
+            for (int j = g.gl; j < kJobWords; j += W)
+                __hip_atomic_store(dst + j, (q & 0xffffffff00000000ull) | (uint32_t)f(r, j), __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
         }
-        return g.bcast(want, 0);
     }
 
+    // record j of a static queue (strided partition: computed)
+    DEV void static_record(int64_t base, int j, int32_t (&t)[4]) const {
+        if (p.sq_jobs) {
+            const int32_t *s = p.sq_jobs + 4 * (base + j);
+            t[0] = s[0], t[1] = s[1], t[2] = s[2], t[3] = s[3];
+        } else {
+            t[0] = p.n - 1 - (int)(base + (int64_t)j * p.nworkers);
+            t[1] = -1;
+            t[2] = t[0] + 1;
+            t[3] = 0;
+        }
+    }
+
+    // Claims up to `n` jobs of a queue shared by a group as this worker's.
+    DEV void claim_shared(int n) {
+        int j = 0;
+        const int len = (int)(p.sq_off[own_queue / p.q_group + 1] - own_base);
+        if (g.gl == 0) j = atomicAdd(&p.sq_cur[own_queue], n);
+        j = g.bcast(j, 0);
+        own_cur = j < len ? j : len;
+        own_end = j + n < len ? j + n : len;
+        if (own_end >= len) own_queue = -1;
+    }
+
+    // Answers waiting requests with equal shares of what this worker has left:
+    // of its static jobs (they need no prefix, and the worker is busy with
+    // another job), else of a range job's untouched roots, else of the children
+    // of the shallowest level of the job (below `top`) that has enough of them.
     // min_first > 0: the job's own level may be cut down to pieces of that
-    // many children (heavy children, where steal_min would leave too much)
+    // many children (heavy children, where steal_min would leave too much).
     DEV void maybe_donate(int top, int min_first = 0) {
-        const int want = donation_demand();
-        if (want == 0) return;
-        // untouched roots of a range job go first: they need no prefix
+        unsigned long long rq = 0;
+        int n = requests(rq);
+        if (n == 0) return;
+        if (own_cur >= own_end && own_queue >= 0) claim_shared(n);
+        if (own_cur < own_end) {
+            const int cur = own_cur, len = own_end - cur;
+            n = accept(rq, len, false);
+            if (n == 0) return;
+            // this worker keeps the first share (it may be empty)
+            auto cut = [&](int j) { return cur + (int)((int64_t)len * j / (n + 1)); };
+            answer(rq, [&](int r, int j) {
+                return j == 0   ? kStaticJobs
+                       : j == 1 ? cut(r + 1)
+                       : j == 2 ? cut(r + 2)
+                       : j == 4 ? (int)(uint32_t)own_base
+                       : j == 5 ? (int)(uint32_t)(own_base >> 32)
+                                : 0;
+            });
+            own_end = cut(1);
+            return;
+        }
+        if (!p.steal) return;
         if (range_hi - v0 - 1 >= 2) {
-            const int mid = v0 + 1 + ((range_hi - v0 - 1) >> 1);
-            if (push_range(mid, range_hi)) range_hi = mid;
+            const int lo = v0 + 1, len = range_hi - lo;
+            n = accept(rq, len - 1, true);
+            if (n == 0) return;
+            auto cut = [&](int j) { return lo + (int)((int64_t)len * j / (n + 1)); };
+            answer(rq, [&](int r, int j) {
+                return j == 0 ? 0 : j == 1 ? -1 : j == 2 ? cut(r + 2) : j == 3 ? qword : j == 4 ? cut(r + 1) : -1;
+            });
+            range_hi = cut(1);
+            if (g.gl == 0) ws.st()[kStDonated] += (unsigned long long)n;
             return;
         }
         // a clique's last level has cheap children: split it only in bigger pieces
@@ -1039,14 +1086,23 @@ struct Worker {
         for (int l = job_lvl; l < top; l++) {
             const int cur = ws.lv()[l].cur, end = ws.lv()[l].end;
             const int minc = (min_first > 0 && l == job_lvl) ? min_first : l == K - 3 ? leaf_min : job_sm;
-            if (end - cur >= minc) {
-                int P = (end - cur) / minc - 1;
-                if (P < 1) P = 1;
-                if (P > want) P = want;
-                if (P > end - cur - 1) P = end - cur - 1;
-                if (P >= 1) ws.lv()[l].end = push_pieces(l, cur, end, P);
-                return;
-            }
+            if (end - cur < minc) continue;
+            int most = (end - cur) / minc - 1;
+            most = most < 1 ? 1 : most > end - cur - 1 ? end - cur - 1 : most;
+            if (most < 1) return;
+            n = accept(rq, most, true);
+            if (n == 0) return;
+            answer(rq, [&](int r, int j) {
+                return j == 0   ? l
+                       : j == 1 ? split_at(l, cur, end, r + 1, n + 1)
+                       : j == 2 ? split_at(l, cur, end, r + 2, n + 1)
+                       : j == 3 ? qword
+                       : j - 4 <= l ? ws.lv()[j - 4].vtx
+                                    : -1;
+            });
+            ws.lv()[l].end = split_at(l, cur, end, 1, n + 1);
+            if (g.gl == 0) ws.st()[kStDonated] += (unsigned long long)n;
+            return;
         }
     }
 
@@ -1539,7 +1595,7 @@ struct Worker {
         lds_top = lds_lo;
         g_top = g_lo;
         cnt = 0;
-        const bool motif = MODE == 2 ? qmotif : MODE == 1;
+        constexpr bool motif = MODE == 1;
         // a motif worker's slice is its leaf scratch; its lists are in the arena
         if (motif) lds_top = lds_lo + p.lds_per_worker;
         if (!motif && K == 2) {
@@ -1658,113 +1714,134 @@ DEV int num_queues(const EnumParams &p) {
     const int gq = p.q_group > 1 ? p.q_group : 1;
     return (p.nworkers + gq - 1) / gq;
 }
-DEV int own_queue(const EnumParams &p, int wid) { return p.q_group > 1 ? wid / p.q_group : wid; }
-
-// Claims the next job of static queue w.
-template <int W>
-DEV bool take_static(const EnumParams &p, const Grp<W> &g, int w, const WorkerLDS &ws, JobHead &jh) {
-    // strided partition (no job arrays, one queue per worker): worker w
-    // holds roots n-1-w, n-1-w-nworkers, ...
-    const bool strided = p.sq_jobs == nullptr;
-    int64_t b = 0, e = 0;
-    if (strided) e = w < p.n ? (int64_t)((p.n - 1 - w) / p.nworkers) + 1 : 0;
-    else b = p.sq_off[w], e = p.sq_off[w + 1];
-    int got = 0, r = 0, lo = 0, hi = 0, q = 0;
-    // a shared queue's cursor sits at its first worker's slot, so cursors of
-    // groups of 32 or more workers never share a cache line
-    int32_t *cursor = &p.sq_cur[p.q_group > 1 ? w * p.q_group : w];
-    if (g.gl == 0 && b < e) {
-        int cur = __hip_atomic_load(cursor, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (b + cur < e) {
-            int j = atomicAdd(cursor, 1);
-            if (b + j < e) {
-                got = 1;
-                if (strided) {
-                    r = p.n - 1 - (w + j * p.nworkers);
-                    lo = -1;
-                    hi = r + 1;
-                    q = 0;
-                } else {
-                    const int32_t *t = p.sq_jobs + 4 * (b + j);
-                    r = t[0];
-                    lo = t[1];
-                    hi = t[2];
-                    q = t[3];
-                }
-                // whoever claims a queue's last job retires the queue
-                if (b + j == e - 1) {
-                    if (p.qmask) atomicAnd(&p.qmask[w >> 6], ~(1ull << (w & 63)));
-                    atomicSub(&p.sc->static_left, 1);
-                }
-            }
-        }
+// jobs of queue w, and where its records start (strided partition, no job
+// arrays, one queue per worker: worker w holds roots n-1-w, n-1-w-nworkers, ...)
+DEV int queue_jobs(const EnumParams &p, int w, int64_t &base) {
+    if (p.sq_jobs == nullptr) {
+        base = w;
+        return w < p.n ? (int)((p.n - 1 - w) / p.nworkers) + 1 : 0;
     }
-    got = g.bcast(got, 0);
-    if (!got) return false;
+    base = p.sq_off[w];
+    return (int)(p.sq_off[w + 1] - base);
+}
+
+// A static record (root, lo, hi, q) as a job head.
+template <int W>
+DEV void static_head(const Grp<W> &g, const WorkerLDS &ws, int r, int lo, int hi, int q, JobHead &jh) {
     jh.lvl = 0;
     jh.donated = false;
-    jh.shared = false;
-    lo = g.bcast(lo, 0);
-    hi = g.bcast(hi, 0);
-    jh.q = g.bcast(q, 0);
-    r = g.bcast(r, 0);
-    if (lo == -2) {  // (root, -2, jobs on the root, q): children from the shared cursor
-        jh.range_end = 0;
-        jh.shared = true;
-        jh.lo = 0;
-        jh.hi = hi;
-    } else if (lo < 0) {  // range job
-        jh.range_end = hi;
-        jh.lo = 0;
-        jh.hi = 0x7fffffff;
-    } else {
-        jh.range_end = 0;
-        jh.lo = lo;
-        jh.hi = hi;
-    }
-    ws.jid()[0] = r;
+    jh.shared = lo == -2;  // (root, -2, jobs on the root, q): children from the shared cursor
+    jh.range_end = lo == -1 ? hi : 0;
+    jh.lo = lo < 0 ? 0 : lo;
+    jh.hi = lo == -1 ? 0x7fffffff : hi;
+    jh.q = q;
+    if (g.gl == 0) ws.jid()[0] = r;
     wsync();
+}
+
+// The worker's own queue: all of it is the worker's from the start, taken
+// with one atomic (a queue whose block starts late may have lost jobs to
+// probe_queues by then); a queue shared by a group is claimed job by job.
+template <int W, int MODE>
+DEV void open_own_queue(Worker<W, MODE> &wk, int wid) {
+    const EnumParams &p = wk.p;
+    const bool shared = p.q_group > 1;
+    const int w = shared ? wid / p.q_group : wid;
+    const int len = queue_jobs(p, w, wk.own_base);
+    wk.own_cur = wk.own_end = 0;
+    wk.own_queue = shared && len > 0 ? w * p.q_group : -1;
+    if (!shared && len > 0) {
+        int j = 0;
+        if (wk.g.gl == 0) j = atomicAdd(&p.sq_cur[w], len);
+        j = wk.g.bcast(j, 0);
+        wk.own_cur = j < len ? j : len;
+        wk.own_end = len;
+    }
+}
+
+template <int W, int MODE>
+DEV bool take_own(Worker<W, MODE> &wk, JobHead &jh) {
+    if (wk.own_cur >= wk.own_end && wk.own_queue >= 0) wk.claim_shared(1);
+    if (wk.own_cur >= wk.own_end) return false;
+    int32_t t[4];
+    wk.static_record(wk.own_base, wk.own_cur++, t);
+    static_head<W>(wk.g, wk.ws, uni<W>(t[0]), uni<W>(t[1]), uni<W>(t[2]), uni<W>(t[3]), jh);
     return true;
 }
 
-// Donated jobs are served in ticket order: an idle worker takes one ticket
-// (atomicAdd on the high half of q_ht) and from then on polls only the slot of its ticket,
-// so waiting workers never contend on a shared word.  A slot is complete when
-// all its words carry this launch's epoch.  Returns true when the ticket's job
-// has arrived (and clears the ticket).
-template <int W>
-DEV bool poll_ticket(const EnumParams &p, const Grp<W> &g, const WorkerLDS &ws, JobHead &jh, bool &has_ticket,
-                     uint32_t &ticket, uint32_t ep) {
-    if (!has_ticket) {
-        uint32_t t = 0;
-        if (g.gl == 0) t = (uint32_t)(atomicAdd(&p.sc->q_ht, 1ull << 32) >> 32);
-        ticket = (uint32_t)g.bcast((int)t, 0);
-        has_ticket = true;
+// While blocks of the launch have yet to start (the grid is larger than what
+// is resident), nobody hands out their queues: an idle worker looks for a job
+// among a random run of queues.
+template <int W, int MODE>
+DEV bool probe_queues(Worker<W, MODE> &wk, uint32_t &seed, JobHead &jh) {
+    const EnumParams &p = wk.p;
+    const Grp<W> &g = wk.g;
+    const int nq = num_queues(p);
+    seed = seed * 1664525u + 1013904223u;
+    int w = (int)((seed >> 8) % (uint32_t)nq) + g.gl;
+    if (w >= nq) w -= nq;
+    int64_t base = 0;
+    int len = 0, cur = 0;
+    int32_t *const cursor = &p.sq_cur[p.q_group > 1 ? (w < nq ? w : 0) * p.q_group : (w < nq ? w : 0)];
+    if (w < nq) {
+        len = queue_jobs(p, w, base);
+        cur = __hip_atomic_load(cursor, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    if (ticket >= p.q_cap) return false;  // no slot: wait for the end
-    const uint64_t *src = p.q[ticket].w;
+    const uint64_t some = g.ballot(w < nq && cur < len);
+    if (!some) return false;
+    const int l = __builtin_ctzll(some);
+    int32_t t[4] = {0, 0, 0, 0};
+    int got = 0;
+    if (g.gl == l) {
+        const int j = atomicAdd(cursor, 1);
+        if (j < len) {
+            got = 1;
+            wk.static_record(base, j, t);
+        }
+    }
+    if (!g.bcast(got, l)) return false;
+    static_head<W>(g, wk.ws, g.bcast(t[0], l), g.bcast(t[1], l), g.bcast(t[2], l), g.bcast(t[3], l), jh);
+    return true;
+}
+
+// Reads a worker's own slot: 1 with the job its request was answered with, 2
+// with static jobs that are now its own queue, 3 when the request was turned
+// down, 0 while nothing has come.
+template <int W, int MODE>
+DEV int poll_slot(Worker<W, MODE> &wk, int wid, uint32_t tag, JobHead &jh) {
+    const Grp<W> &g = wk.g;
+    const uint64_t *src = wk.p.q[wid].w;
     int v[(kJobWords + W - 1) / W];
-    bool mine_ok = true;
+    bool mine_ok = true, none = false;
 #pragma unroll
     for (int r = 0; r < (kJobWords + W - 1) / W; r++) {
         const int j = g.gl + r * W;
         v[r] = 0;
         if (j < kJobWords) {
             uint64_t x = __hip_atomic_load(src + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if ((uint32_t)(x >> 32) != ep) mine_ok = false;
+            if ((uint32_t)(x >> 32) != tag) mine_ok = false;
             v[r] = (int32_t)(uint32_t)x;
+            if (j == 0) none = mine_ok && v[r] == kNoJob;
         }
     }
-    if (g.ballot(!mine_ok) != 0) return false;
+    if (g.ballot(none) != 0) return 3;
+    if (g.ballot(!mine_ok) != 0) return 0;
+    const int w0 = g.bcast(v[0], 0), w1 = g.bcast(v[0], 1), w2 = g.bcast(v[0], 2), w3 = g.bcast(v[0], 3);
+    if (w0 == kStaticJobs) {
+        wk.own_base = (int64_t)(((uint64_t)(uint32_t)g.bcast(v[0], 5) << 32) | (uint32_t)g.bcast(v[0], 4));
+        wk.own_cur = w1;
+        wk.own_end = w2;
+        return 2;
+    }
 #pragma unroll
     for (int r = 0; r < (kJobWords + W - 1) / W; r++) {
         const int j = g.gl + r * W;
-        if (j >= 4 && j < kJobWords) ws.jid()[j - 4] = v[r];
+        if (j >= 4 && j < kJobWords) wk.ws.jid()[j - 4] = v[r];
     }
-    jh.lvl = g.bcast(v[0], 0);
-    jh.lo = g.bcast(v[0], 1);
-    jh.hi = g.bcast(v[0], 2);
-    jh.q = g.bcast(v[0], 3);
+    jh.lvl = w0;
+    jh.lo = w1;
+    jh.hi = w2;
+    jh.q = w3;
     jh.range_end = 0;
     jh.donated = true;
     jh.shared = false;
@@ -1773,66 +1850,39 @@ DEV bool poll_ticket(const EnumParams &p, const Grp<W> &g, const WorkerLDS &ws, 
         jh.lo = 0;
         jh.hi = 0x7fffffff;
     }
-    has_ticket = false;
     wsync();
-    return true;
+    return 1;
 }
 
+// A worker has run out of work.  The last worker of a block closes its mailbox
+// and subtracts the block's finished jobs; true when no job of the launch is
+// left.
 template <int W>
-DEV bool steal_static(const EnumParams &p, const Grp<W> &g, int w, const WorkerLDS &ws, JobHead &jh,
-                      uint32_t &seed, bool &static_done) {
-    int left = 0;
-    if (g.gl == 0) left = __hip_atomic_load(&p.sc->static_left, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (g.bcast(left, 0) <= 0) {
-        static_done = true;
-        if (g.gl == 0) ws.st()[kStStatic] = wall_clock64();
-        return false;
+DEV bool go_idle(const EnumParams &p, const Grp<W> &g, BlockLDS *blk) {
+    int last = 0;
+    if (g.gl == 0) last = atomicSub(&blk->busy, 1) == 1;
+    if (!g.bcast(last, 0)) return false;
+    if (g.gl < kMailSlots) {
+        const unsigned long long rq = atomicExch(p.mail + (size_t)blockIdx.x * kMailStride + g.gl, kMailIdle);
+        if (rq != 0 && rq != kMailIdle)
+            __hip_atomic_store(p.q[(uint32_t)rq - 1].w, (rq & 0xffffffff00000000ull) | (uint32_t)kNoJob,
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    const int nq = num_queues(p);
-    if (nq <= 1) return false;  // the one queue was tried by take_static
-    if (p.qmask) {
-        // a random queue among those still holding jobs: the lanes read the
-        // mask words from a random word on, the first non-zero word (in that
-        // order) gives a random set bit.  Plain reads of rarely written
-        // words; thieves spread over the non-empty queues.
-        const int nwords = (nq + 63) >> 6;
-        for (int attempt = 0; attempt < 4; attempt++) {
-            seed = seed * 1664525u + 1013904223u;
-            const int start = (int)((seed >> 8) % (uint32_t)nwords);
-            const int rot = (int)((seed >> 20) & 63);
-            int v = -1;
-            for (int base = 0; base < nwords && v < 0; base += W) {
-                const int i = base + g.gl;
-                int wi = start + i;
-                if (wi >= nwords) wi -= nwords;
-                unsigned long long m = 0;
-                if (i < nwords) m = __hip_atomic_load(&p.qmask[wi], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                const uint64_t bal = g.ballot(m != 0);
-                if (bal) {
-                    const int l = __builtin_ctzll(bal);
-                    int q = 0;
-                    if (g.gl == l) {
-                        const unsigned long long r = rot ? (m >> rot) | (m << (64 - rot)) : m;
-                        q = wi * 64 + ((__builtin_ctzll(r) + rot) & 63);
-                    }
-                    v = g.bcast(q, l);
-                }
-            }
-            if (v < 0) return false;  // every queue retired or being retired
-            if (v != w && v < nq && take_static<W>(p, g, v, ws, jh)) return true;
-        }
-        return false;
+    int end = 0;
+    if (g.gl == 0) {
+        const unsigned long long done = atomicExch(&blk->pending, 0u);
+        end = done && atomicSub(&p.sc->outstanding, done) == done;
     }
-    // random probes: idle workers spread over the queues (a scan for the
-    // fullest queue sends them all to the same cursor, and device-scope
-    // atomics on one address slow every worker's memory traffic)
-    for (int probe = 0; probe < 8; probe++) {
-        seed = seed * 1664525u + 1013904223u;
-        int v = (int)((seed >> 8) % (uint32_t)nq);
-        if (v == w) continue;
-        if (take_static<W>(p, g, v, ws, jh)) return true;
-    }
-    return false;
+    return g.bcast(end, 0) != 0;
+}
+
+// An idle worker has work again.
+template <int W>
+DEV void go_busy(const EnumParams &p, const Grp<W> &g, BlockLDS *blk) {
+    int first = 0;
+    if (g.gl == 0) first = atomicAdd(&blk->busy, 1) == 0;
+    if (g.bcast(first, 0) && g.gl < kMailSlots)
+        (void)atomicCAS(p.mail + (size_t)blockIdx.x * kMailStride + g.gl, kMailIdle, 0ull);
 }
 
 // Adds a worker's counts for query `q` to the query's result: the clique count
@@ -1856,8 +1906,8 @@ DEV void flush_query(const EnumParams &p, const Grp<W> &g, int q, unsigned long 
     }
 }
 
-// MODE 0: cliques only, 1: motifs only, 2: mixed (batch launches); WAVES:
-// the waves per SIMD the registers are budgeted for.
+// MODE 0: cliques, 1: motifs; WAVES: the waves per SIMD the registers are
+// budgeted for.
 template <int W, int MODE, int WAVES = min_waves<W, MODE>()>
 __global__ __launch_bounds__(kThreads, WAVES) void enum_kernel(EnumParams p) {
     extern __shared__ __align__(16) char smem[];
@@ -1866,24 +1916,32 @@ __global__ __launch_bounds__(kThreads, WAVES) void enum_kernel(EnumParams p) {
     const int wpb = nthr / W;
     const int wib = uni<W>(threadIdx.x / W);
     const int wid = blockIdx.x * wpb + wib;
-    // LDS: single-query class counters of the block | per-worker records |
+    // LDS: block record | single-query class counters of the block | per-worker records |
     // per-worker class counters (batch) | per-worker stack slices
     const bool single = p.nq == 1;
     const int bslots = single && p.qd[0].motif ? (p.qd[0].ncls + 1) & ~1 : 0;
     const int wslots = single ? 0 : (p.hist_slots + 1) & ~1;
     const size_t wsb = worker_lds_bytes(p.kmax);
-    unsigned long long *bhist = (unsigned long long *)smem;
-    char *base = smem + (size_t)bslots * 8;
+    BlockLDS *const blk = (BlockLDS *)smem;
+    unsigned long long *bhist = (unsigned long long *)(smem + sizeof(BlockLDS));
+    char *base = smem + sizeof(BlockLDS) + (size_t)bslots * 8;
     const WorkerLDS ws = worker_lds(base + wib * wsb, p.kmax);
     base += wpb * wsb;
     unsigned long long *whist = (unsigned long long *)base + (size_t)wib * wslots;
     base += (size_t)wpb * wslots * 8;
     char *slice = base + (int64_t)wib * p.lds_per_worker;
     for (int i = threadIdx.x; i < bslots; i += nthr) bhist[i] = 0;
-    for (int i = threadIdx.x; i < wpb * wslots; i += nthr) ((unsigned long long *)(smem + (size_t)bslots * 8 + wpb * wsb))[i] = 0;
+    for (int i = threadIdx.x; i < wpb * wslots; i += nthr) ((unsigned long long *)(smem + sizeof(BlockLDS) + (size_t)bslots * 8 + wpb * wsb))[i] = 0;
     if (threadIdx.x == 0) {
         const unsigned long long t = wall_clock64();
-        atomicMin(&p.sc->t_start, t);
+        atomicAdd(&p.sc->started, 1);
+        const int left = p.nworkers - (int)blockIdx.x * wpb;
+        blk->busy = left < wpb ? left : wpb;
+        blk->pending = 0;
+        for (int i = 0; i < kMailSlots; i++)
+            __hip_atomic_store(p.mail + (size_t)blockIdx.x * kMailStride + i, 0ull, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+        atomicMin(&p.sc->st[blockIdx.x % kStatCopies].t_start, t);
         if (p.start_ticks) atomicMin(p.start_ticks, t);
     }
     __syncthreads();
@@ -1893,40 +1951,87 @@ __global__ __launch_bounds__(kThreads, WAVES) void enum_kernel(EnumParams p) {
         if (g.gl == 0)
             for (int i = 0; i < kStats; i++) ws.st()[i] = 0;
         wsync();
-        Worker<W, MODE> wk(p, ws, single ? bhist : whist, slice, wid);
+        Worker<W, MODE> wk(p, ws, single ? bhist : whist, slice, blk, wid);
         uint32_t seed = 0x9E3779B9u * (uint32_t)(wid + 1);
-        bool static_done = false, has_ticket = false;
-        uint32_t ticket = 0;
+        bool idle = false, all_started = false;
+        uint32_t seq = 0;  // requests of this launch
+        int asked = -1;    // mailbox word that holds this worker's request
+        int waited = 0;    // polls since it was written
         int backoff = 1;
         uint32_t spins = 0;
-        const uint64_t t0 = wk.t_start;
+        const bool can_ask = (uint32_t)wid < p.q_cap;
+        open_own_queue(wk, wid);
         while (true) {
             JobHead jh;
-            bool got = false;
-            if (!static_done) {
-                got = take_static<W>(p, g, own_queue(p, wid), ws, jh);
-                if (!got) got = steal_static<W>(p, g, own_queue(p, wid), ws, jh, seed, static_done);
-            }
-            if (!got && static_done) got = poll_ticket<W>(p, g, ws, jh, has_ticket, ticket, wk.epoch);
+            bool got = take_own(wk, jh);
             if (!got) {
-                if (wk.pending) {
-                    if (g.gl == 0) atomicSub(&p.sc->outstanding, (unsigned long long)wk.pending);
-                    wk.pending = 0;
-                }
-                // the termination words are shared by every worker: read
-                // them on every 4th empty poll only
-                if ((++spins & 3) == 0) {
-                    unsigned long long out = 0;
-                    int err = 0;
-                    if (g.gl == 0) {
-                        out = __hip_atomic_load(&p.sc->outstanding, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                        err = __hip_atomic_load(&p.sc->error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (!idle) {
+                    idle = true;
+                    if (g.gl == 0 && !ws.st()[kStStatic]) ws.st()[kStStatic] = wall_clock64();
+                    if (go_idle<W>(p, g, blk)) {
+                        // the last job is done: tell every block
+                        for (unsigned b = g.gl; b < gridDim.x; b += W)
+                            __hip_atomic_store(wk.mailbox(b) + kMailOver, (unsigned long long)wk.epoch,
+                                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        break;
                     }
-                    out = g.bcast64(out, 0);
-                    err = g.bcast(err, 0);
-                    if (out == 0 || err) break;
                 }
-                if (p.watchdog_ticks && now_ticks() - t0 > p.watchdog_ticks) {
+                // request tags: the epoch and a count, never 0
+                const uint32_t tag = (wk.epoch << 8) | (seq % 255u + 1);
+                if (asked >= 0) {
+                    const int r = poll_slot(wk, wid, tag, jh);
+                    if (r) {
+                        asked = -1;
+                        seq++;
+                    }
+                    got = r == 1;
+                    if (r == 2) got = take_own(wk, jh);
+                    // no answer for long: ask elsewhere (unless it is coming)
+                    if (r == 0 && ++waited >= 24) {
+                        int back = 0;
+                        const unsigned long long rq = ((unsigned long long)tag << 32) | (uint32_t)(wid + 1);
+                        if (g.gl == 0) back = atomicCAS(p.mail + asked, rq, 0ull) == rq;
+                        waited = 0;
+                        if (g.bcast(back, 0)) asked = -1;
+                    }
+                } else if (can_ask) {
+                    // a random word of a random block's mailbox; a block without
+                    // work, or another request there, says so at once
+                    const unsigned long long rq = ((unsigned long long)tag << 32) | (uint32_t)(wid + 1);
+                    for (int a = 0; a < 4 && asked < 0; a++) {
+                        seed = seed * 1664525u + 1013904223u;
+                        const int b = (int)((seed >> 8) % gridDim.x) * kMailStride + (int)(seed >> 29);
+                        int in = 0;
+                        if (g.gl == 0) in = atomicCAS(p.mail + b, 0ull, rq) == 0ull;
+                        if (g.bcast(in, 0)) {
+                            asked = b;
+                            waited = 0;
+                            backoff = 1;
+                        }
+                    }
+                }
+            }
+            if (!got) {
+                ++spins;
+                // the end of the launch; rarely: another worker's failure,
+                // blocks that have yet to start
+                unsigned long long over = 0;
+                int err = 0;
+                if (g.gl == 0) {
+                    over = __hip_atomic_load(wk.mailbox(blockIdx.x) + kMailOver, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    if ((spins & 63) == 0)
+                        err = __hip_atomic_load(&p.sc->error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+                if (g.bcast64(over, 0) == wk.epoch || g.bcast(err, 0)) break;
+                if (!all_started && (spins & 15) == 0) {
+                    int st = 0;
+                    if (g.gl == 0) st = __hip_atomic_load(&p.sc->started, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    all_started = g.bcast(st, 0) >= (int)gridDim.x;
+                    if (!all_started) got = probe_queues(wk, seed, jh);
+                }
+            }
+            if (!got) {
+                if (p.watchdog_ticks && now_ticks() - wk.t_start > p.watchdog_ticks) {
                     if (g.gl == 0) atomicCAS(&p.sc->error, 0, 1);
                     break;
                 }
@@ -1934,9 +2039,13 @@ __global__ __launch_bounds__(kThreads, WAVES) void enum_kernel(EnumParams p) {
                 // stalls the whole wave, including busy narrower workers
                 if (__ballot(1) == ~0ull) {
                     for (int b = 0; b < backoff; b++) __builtin_amdgcn_s_sleep(8);
-                    backoff = backoff < 32 ? backoff * 2 : 32;
+                    backoff = backoff < 16 ? backoff * 2 : 16;
                 }
                 continue;
+            }
+            if (idle) {
+                idle = false;
+                go_busy<W>(p, g, blk);
             }
             backoff = 1;
             const int jq = job_query(jh.q);
@@ -1953,7 +2062,7 @@ __global__ __launch_bounds__(kThreads, WAVES) void enum_kernel(EnumParams p) {
                 wk.K = uni<W>(Q.K);
                 wk.qmotif = uni<W>(Q.motif) != 0;
                 wk.lut = unil<W>(Q.lut);
-                ok = (MODE == 2 || (MODE == 1) == wk.qmotif) && Q.K >= 2 && Q.K <= p.kmax;
+                ok = (MODE == 1) == wk.qmotif && Q.K >= 2 && Q.K <= p.kmax;
             }
             const int lvl_max = wk.K == 2 ? 0 : wk.K - 3;
             const int r0 = uni<W>(ws.jid()[0]);
@@ -1995,8 +2104,10 @@ __global__ __launch_bounds__(kThreads, WAVES) void enum_kernel(EnumParams p) {
                     }
                 }
             }
-            if (g.gl == 0) ws.st()[kStJobs]++;
-            wk.pending++;
+            if (g.gl == 0) {
+                ws.st()[kStJobs]++;
+                atomicAdd(&blk->pending, 1u);
+            }
             if (wk.abort) break;
         }
         wsync();
@@ -2004,9 +2115,12 @@ __global__ __launch_bounds__(kThreads, WAVES) void enum_kernel(EnumParams p) {
         bytes = g.lsum(wk.bytes);
     }
     __syncthreads();
+    // a single query's results: one of res_copies copies per block, so that
+    // the blocks do not all queue up for the same words
+    unsigned long long *const out = p.qd[0].out + (size_t)(blockIdx.x % (unsigned)p.res_copies) * p.res_stride;
     if (single && bslots) {
         for (int i = threadIdx.x; i < p.qd[0].ncls; i += nthr)
-            if (bhist[i]) atomicAdd(&p.qd[0].out[i], bhist[i]);
+            if (bhist[i]) atomicAdd(&out[i], bhist[i]);
     }
     // Per-worker statistics (held by lane 0 of each worker) reduced over the
     // block, so that each block, not each worker, adds to the shared words.
@@ -2046,18 +2160,19 @@ __global__ __launch_bounds__(kThreads, WAVES) void enum_kernel(EnumParams p) {
             for (int i = 0; i < NF; i++)
                 f[i] = i < 5 || i == 10 ? f[i] + red[w][i] : (red[w][i] > f[i] ? red[w][i] : f[i]);
         }
-        if (f[0]) atomicAdd(&p.sc->alg_bytes, f[0]);
-        if (f[1]) atomicAdd(&p.sc->jobs, f[1]);
-        if (f[2]) atomicAdd(&p.sc->busy_sum, f[2]);
-        if (f[3]) atomicAdd(&p.sc->donations, f[3]);
-        if (f[4] && single && !p.qd[0].motif) atomicAdd(&p.qd[0].out[0], f[4]);
-        atomicMax(&p.sc->busy_max, f[5]);
-        atomicMax(&p.sc->t_first_job, f[6]);
-        atomicMax(&p.sc->t_static_done, f[7]);
-        atomicMax(&p.sc->t_last_job, f[8]);
-        atomicMax(&p.sc->job_max, f[9]);
-        if (f[10]) atomicAdd(&p.sc->active_workers, f[10]);
-        atomicMax(&p.sc->t_exit, (unsigned long long)wall_clock64());
+        SchedStats &st = p.sc->st[blockIdx.x % kStatCopies];
+        if (f[0]) atomicAdd(&st.alg_bytes, f[0]);
+        if (f[1]) atomicAdd(&st.jobs, f[1]);
+        if (f[2]) atomicAdd(&st.busy_sum, f[2]);
+        if (f[3]) atomicAdd(&st.donations, f[3]);
+        if (f[4] && single && !p.qd[0].motif) atomicAdd(&out[0], f[4]);
+        atomicMax(&st.busy_max, f[5]);
+        atomicMax(&st.t_first_job, f[6]);
+        atomicMax(&st.t_static_done, f[7]);
+        atomicMax(&st.t_last_job, f[8]);
+        atomicMax(&st.job_max, f[9]);
+        if (f[10]) atomicAdd(&st.active_workers, f[10]);
+        atomicMax(&st.t_exit, (unsigned long long)wall_clock64());
     }
 }
 
@@ -2170,71 +2285,51 @@ __global__ void fill_u32_kernel(uint32_t *ptr, uint32_t value, size_t count) {
 // Resets the scheduler state of a launch; graph-capturable (no memset or
 // host copies).  Bumps the epoch so queue slots of earlier launches never
 // match.
-__global__ void enum_init_kernel(SchedCounters *sc, unsigned long long njobs, int32_t queues, int32_t *epoch, int32_t *sq_cur,
+__global__ void enum_init_kernel(SchedCounters *sc, unsigned long long njobs, int32_t *epoch, int32_t *sq_cur,
                                  int nworkers, unsigned long long *results, size_t nresults,
                                  unsigned long long *done_ticks, int nq, unsigned long long *start_ticks,
-                                 unsigned long long *qmask, int nqueues, const int64_t *sq_off, int strided_n) {
+                                 unsigned long long *mail, int blocks) {
     size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     size_t stride = (size_t)gridDim.x * blockDim.x;
     if (i == 0) {
         sc->outstanding = njobs;
-        sc->static_left = queues;
-        sc->q_ht = 0;
+        sc->started = 0;
         sc->error = 0;
-        sc->donations = 0;
-        sc->jobs = 0;
-        sc->alg_bytes = 0;
-        sc->count = 0;
-        sc->busy_sum = 0;
-        sc->busy_max = 0;
-        sc->t_start = ~0ull;
-        sc->t_first_job = 0;
-        sc->t_static_done = 0;
-        sc->t_last_job = 0;
-        sc->t_exit = 0;
-        sc->job_max = 0;
-        sc->active_workers = 0;
         *epoch = *epoch + 1;
         if (start_ticks) *start_ticks = ~0ull;
     }
+    for (size_t t = i; t < kStatCopies; t += stride) {
+        SchedStats z{};
+        z.t_start = ~0ull;
+        sc->st[t] = z;
+    }
+    // no block takes requests before it has begun; the launch is not over
+    for (size_t t = i; t < (size_t)blocks * kMailStride; t += stride)
+        mail[t] = t % kMailStride < kMailSlots ? kMailIdle : 0;
     for (size_t t = i; t < (size_t)nworkers; t += stride) sq_cur[t] = 0;
     for (size_t t = i; t < nresults; t += stride) results[t] = 0;
     if (done_ticks)
         for (size_t t = i; t < (size_t)nq; t += stride) done_ticks[t] = 0;
-    // non-empty static queues (strided partition: queue w holds roots iff w
-    // < n), one queue per thread and one mask word per wave: a wave's lanes
-    // hold 64 consecutive queues (blocks of 256 threads, a stride of whole
-    // blocks), so the loop condition is uniform over the wave
-    if (qmask) {
-        const size_t nbits = ((size_t)nqueues + 63) / 64 * 64;
-        for (size_t q = i; (q & ~(size_t)63) < nbits; q += stride) {
-            bool ne = false;
-            if (q < (size_t)nqueues) ne = sq_off ? sq_off[q + 1] > sq_off[q] : (int64_t)q < strided_n;
-            const unsigned long long m = __ballot(ne);
-            if ((q & 63) == 0) qmask[q >> 6] = m;
-        }
-    }
 }
 
 // ---------------------------------------------------------------------------
 size_t enum_lds_bytes(int vwave, int threads, int kmax, int ncls_single, int hist_slots, int lds_per_worker) {
     int wpb = threads / vwave;
-    size_t b = (size_t)((ncls_single + 1) & ~1) * 8;
+    size_t b = sizeof(BlockLDS) + (size_t)((ncls_single + 1) & ~1) * 8;
     b += (size_t)wpb * worker_lds_bytes(kmax);
     b += (size_t)wpb * (size_t)((hist_slots + 1) & ~1) * 8;
     b += (size_t)wpb * lds_per_worker;
     return b;
 }
 
-// launch modes: 0 cliques, 1 motifs, 2 mixed, 3 motifs of size >= 5 (the
+// launch modes: 0 cliques, 1 motifs, 2 motifs of size >= 5 (the
 // full-wave motif kernel at kDeepMotifWaves; narrower widths keep mode 1's)
 template <int W>
 static const void *kernel_mode(int mode) {
     switch (mode) {
         case 0: return (const void *)enum_kernel<W, 0>;
         case 1: return (const void *)enum_kernel<W, 1>;
-        case 2: return (const void *)enum_kernel<W, 2>;
-        case 3:
+        case 2:
             if constexpr (W == 64) return (const void *)enum_kernel<W, 1, kDeepMotifWaves>;
             else return (const void *)enum_kernel<W, 1>;
         default: return nullptr;
@@ -2296,19 +2391,35 @@ int enum_launch(const EnumParams &p, int mode, int vwave, int blocks, int thread
     return DM_OK;
 }
 
-int enum_init_launch(const EnumParams &p, unsigned long long njobs, int queues, int32_t *epoch,
-                     unsigned long long *results, size_t nresults, unsigned long long *done_ticks, int nq,
-                     void *stream) {
+int enum_init_launch(const EnumParams &p, unsigned long long njobs, int32_t *epoch, unsigned long long *results,
+                     size_t nresults, unsigned long long *done_ticks, int nq, int launch_blocks, void *stream) {
     size_t work = std::max<size_t>({(size_t)p.nworkers, nresults, (size_t)nq, (size_t)1});
     int blocks = (int)std::min<size_t>((work + 255) / 256, 1024);
-    const int g = p.q_group > 1 ? p.q_group : 1;
-    const int nqueues = p.sq_jobs ? (p.nworkers + g - 1) / g : p.nworkers;
-    hipLaunchKernelGGL(enum_init_kernel, dim3(blocks), dim3(256), 0, (hipStream_t)stream, p.sc, njobs, queues, epoch,
-                       p.sq_cur, p.nworkers, results, nresults, done_ticks, nq, p.start_ticks, p.qmask, nqueues,
-                       p.sq_jobs ? p.sq_off : (const int64_t *)nullptr, p.n);
+    hipLaunchKernelGGL(enum_init_kernel, dim3(blocks), dim3(256), 0, (hipStream_t)stream, p.sc, njobs, epoch, p.sq_cur,
+                       p.nworkers, results, nresults, done_ticks, nq, p.start_ticks, p.mail, launch_blocks);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return set_error(DM_ERR_HIP, "init launch: %s", hipGetErrorString(e));
     return DM_OK;
+}
+
+SchedStats sched_totals(const SchedCounters &c) {
+    SchedStats t = c.st[0];
+    for (int i = 1; i < kStatCopies; i++) {
+        const SchedStats &s = c.st[i];
+        t.donations += s.donations;
+        t.jobs += s.jobs;
+        t.alg_bytes += s.alg_bytes;
+        t.busy_sum += s.busy_sum;
+        t.active_workers += s.active_workers;
+        t.busy_max = std::max(t.busy_max, s.busy_max);
+        t.job_max = std::max(t.job_max, s.job_max);
+        t.t_start = std::min(t.t_start, s.t_start);
+        t.t_first_job = std::max(t.t_first_job, s.t_first_job);
+        t.t_static_done = std::max(t.t_static_done, s.t_static_done);
+        t.t_last_job = std::max(t.t_last_job, s.t_last_job);
+        t.t_exit = std::max(t.t_exit, s.t_exit);
+    }
+    return t;
 }
 
 int fill_u32_launch(void *ptr, uint32_t value, size_t count, void *stream) {

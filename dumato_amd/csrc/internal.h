@@ -2,6 +2,7 @@
 #ifndef DM_INTERNAL_H
 #define DM_INTERNAL_H
 
+#include <algorithm>
 #include <cstddef>
 #include <cstdint>
 #include <string>
@@ -71,40 +72,56 @@ struct Rng {
 
 // ---- device-side structures (identical layout on host and device) ----------
 // A donated job: children [lo, hi) of the node with prefix ids[0..lvl] in
-// query q.  Word j holds (launch epoch << 32 | value): words 0..3 = lvl, lo,
-// hi, q; words 4.. = ids.
+// query q.  Word j holds (tag << 32 | value): words 0..3 = lvl, lo, hi, q;
+// words 4.. = ids.
 constexpr int kJobWords = 4 + kJobIds;
 struct Job {
     uint64_t w[kJobWords];
 };
 
-// Scheduler counters.  Fields that idle and busy workers poll or update
-// concurrently each sit on their own 128-byte line, so traffic on one never
-// stalls the others.
-struct SchedCounters {
-    unsigned long long outstanding;  // unfinished jobs (static + donated)
-    char pad0[120];
-    int32_t static_left;             // worker queues whose last job is not yet claimed
-    char pad2[124];
-    // donated-job queue: next ticket (high 32 bits) and next free slot (low
-    // 32 bits) in one word, so one load tells whether tickets wait for jobs
-    unsigned long long q_ht;
-    char pad3[120];
-    int32_t error;                   // 1 watchdog, 2 arena overflow, 3 bad job
-    char pad5[124];
+// Scheduler words that workers update while a launch runs, each on its own
+// 128-byte line, so that traffic on one never stalls the others.
+struct SchedStats {
     unsigned long long donations;
     unsigned long long jobs;
     unsigned long long alg_bytes;
-    unsigned long long count;        // clique count / motif subgraph total
     unsigned long long busy_sum;     // sum over workers of cycles spent in jobs
     unsigned long long busy_max;     // largest per-worker busy cycles
     // timeline (wall-clock ticks): first block start, then the latest worker
-    // to start its first job, to find static work exhausted, to end its last
-    // job and to exit
+    // to start its first job, to find its static queue exhausted, to end its
+    // last job and to exit
     unsigned long long t_start, t_first_job, t_static_done, t_last_job, t_exit;
-    unsigned long long job_max;  // cycles of the longest single job
+    unsigned long long job_max;         // cycles of the longest single job
     unsigned long long active_workers;  // workers that ran at least one job
+    unsigned long long pad[4];
 };
+static_assert(sizeof(SchedStats) == 128, "one line per copy of the statistics");
+// Every block adds its statistics once, when it ends: to one of these copies,
+// which the host sums (one copy: 13 same-line atomics of 768 blocks took the
+// last 50 us of every clique launch, of 1,536 blocks 125 us of a k >= 5 motif's).
+constexpr int kStatCopies = 32;
+struct SchedCounters {
+    unsigned long long outstanding;  // unfinished jobs (static + donated)
+    char pad0[120];
+    int32_t started;                 // blocks that have begun to run
+    char pad2[124];
+    int32_t error;                   // 1 watchdog, 2 arena overflow, 3 bad job
+    char pad5[124];
+    SchedStats st[kStatCopies];
+};
+SchedStats sched_totals(const SchedCounters &c);
+// Word 0 of a job in a worker's slot is its level, or kStaticJobs: the records
+// [word 1, word 2) of the static queue that starts at record (or, strided, at
+// worker) word 4 | word 5 << 32; or kNoJob: the request was not taken.
+constexpr int32_t kStaticJobs = 0x100;
+constexpr int32_t kNoJob = 0x200;
+// A block's mailbox, a line: kMailSlots words that hold 0 (open), a request
+// (asking worker + 1, its tag in the high half) or kMailIdle (no worker of the
+// block has work); word kMailOver is the epoch of a launch that is over.
+constexpr int kMailStride = 16;
+constexpr int kMailSlots = 8;
+constexpr int kMailOver = 8;
+constexpr unsigned long long kMailIdle = 0xffffffffull;
 
 // One counting query of a launch.  A single-graph call has one; a batch
 // has one per (graph, pattern, k).
@@ -142,10 +159,12 @@ struct EnumParams {
     const int64_t *sq_off;
     const int32_t *sq_jobs;
     int32_t *sq_cur;
-    // donated jobs
+    // a slot per worker for the jobs it is given (workers past q_cap never
+    // ask), and a mailbox per block
     Job *q;
     uint32_t q_cap;
     int32_t pad2;
+    unsigned long long *mail;
     const int32_t *epoch;             // launch epoch in device memory (set by the init kernel)
     unsigned long long *start_ticks;  // wall clock of the first block start
     SchedCounters *sc;
@@ -157,7 +176,7 @@ struct EnumParams {
     unsigned long long *root_cost;    // nullable, per vertex
     unsigned long long *root_count;   // nullable
     int32_t steal, steal_min, bitmap, pad4;
-    uint64_t poll_ticks;              // wall-clock ticks between a worker's donation checks
+    uint64_t poll_ticks;              // wall-clock ticks between a worker's looks at its mailbox
     uint64_t watchdog_ticks;          // wall-clock ticks
     // local bitmaps prebuilt for some roots (cliques, k = 4..6): pre_roots
     // ascending (npre entries), root pre_roots[i]'s rows (d x NW uint64) and
@@ -172,20 +191,16 @@ struct EnumParams {
     int32_t npre;
     // workers per static queue (0 or 1: one queue per worker): worker w
     // claims from queue w / q_group of the (nworkers + q_group - 1) / q_group
-    // queues, and an idle worker probes the other queues
+    // queues
     int32_t q_group;
+    // copies of a single query's results that the blocks add to (summed by
+    // the host), and the words from one copy to the next
+    int32_t res_copies, res_stride;
     int32_t pad6;
-    // nullable: one bit per static queue, set while the queue holds an
-    // unclaimed job (set by the init kernel, cleared by the claimer of the
-    // queue's last job); idle workers steal from a set bit's queue
-    unsigned long long *qmask;
 };
-
-// 64-bit words of the non-empty-queue mask of a launch with these workers
-inline int qmask_words(int nworkers, int q_group) {
-    const int g = q_group > 1 ? q_group : 1;
-    return ((nworkers + g - 1) / g + 63) / 64;
-}
+// One copy per block, 32 at most, in at most 8 KB unless one copy is larger.
+inline int result_stride(size_t nres) { return (int)((nres + 15) & ~(size_t)15); }
+inline int result_copies(size_t nres) { return std::max(1, std::min(32, 1024 / result_stride(nres))); }
 
 // A static or donated job's query word: bits 0..15 the query index, bits
 // 16..23 the job's own donation threshold (0: the launch's steal_min).
@@ -195,9 +210,9 @@ constexpr int job_steal_min(int32_t q) { return (q >> kQueryBits) & 0xff; }
 constexpr int32_t make_job_query(int q, int steal_min) { return q | (steal_min << kQueryBits); }
 
 // kernels (enum_kernel.hip)
-// mode: 0 cliques only, 1 motifs only, 2 mixed (batch), 3 motifs of size >= 5
-// (a motif kernel budgeted for one more wave per SIMD)
-inline int launch_mode(bool motif, int K) { return motif ? (K >= 5 ? 3 : 1) : 0; }
+// mode: 0 cliques, 1 motifs, 2 motifs of size >= 5 (a motif kernel budgeted
+// for more waves per SIMD)
+inline int launch_mode(bool motif, int K) { return motif ? (K >= 5 ? 2 : 1) : 0; }
 // The motif leaf's LDS without its table, per worker of W lanes: recs u64[W] |
 // bits u64[kLeafCap / 64] | qs u64[npm] | n u32[npm] | e u32[copies][npm (npm + 1) / 2],
 // npm = 2^(K-2) mask values.  A motif launch gives each worker at least this.
@@ -211,10 +226,8 @@ int enum_occupancy(int vwave, int mode, int threads, size_t lds, int *blocks_per
 int enum_launch(const EnumParams &p, int mode, int vwave, int blocks, int threads, size_t lds,
                 void *stream);
 // resets the scheduler state of a launch (graph-capturable: kernels only)
-// queues: worker queues holding at least one static job
-int enum_init_launch(const EnumParams &p, unsigned long long njobs, int queues, int32_t *epoch,
-                     unsigned long long *results, size_t nresults, unsigned long long *done_ticks, int nq,
-                     void *stream);
+int enum_init_launch(const EnumParams &p, unsigned long long njobs, int32_t *epoch, unsigned long long *results,
+                     size_t nresults, unsigned long long *done_ticks, int nq, int launch_blocks, void *stream);
 int fill_u32_launch(void *ptr, uint32_t value, size_t count, void *stream);
 // builds the local bitmaps of p.pre_roots into p.pre (one block per root)
 int prebuild_launch(const EnumParams &p, void *stream);

@@ -36,22 +36,23 @@ static __device__ __align__(256) char scratch[kScratchBytes];
 
 // layout of the array (byte offsets)
 constexpr size_t kSoSc = 0;                           // SchedCounters
-constexpr size_t kSoEpoch = 1024;                     // int32 launch epoch
-constexpr size_t kSoQd = 1280;                        // QueryDesc
-constexpr size_t kSoRes = 2048;                       // result slots
+constexpr size_t kSoEpoch = 6144;                     // int32 launch epoch
+constexpr size_t kSoQd = 6400;                        // QueryDesc
+constexpr size_t kSoRes = 8192;                       // result slots
 constexpr size_t kResSlots = 2048;
 constexpr size_t kSoLut = 32 << 10;                   // class table (uint16)
 constexpr size_t kLutBytes = (size_t)2 << 20;         // 2^20 entries: k <= 7
 constexpr size_t kSoCur = kSoLut + kLutBytes;         // static-queue cursors
 constexpr size_t kMaxWorkers = 65536;
-constexpr size_t kSoQmask = kSoRes + kResSlots * 8;    // non-empty static queues (1 bit per worker)
-constexpr size_t kSoQueue = kSoCur + kMaxWorkers * 4;  // donated-job queue
-constexpr uint32_t kQueueSlots = 16384;
-constexpr size_t kSoArena = kSoQueue + (size_t)kQueueSlots * sizeof(Job);
+constexpr size_t kSoQueue = kSoCur + kMaxWorkers * 4;  // the workers' job slots
+constexpr uint32_t kQueueSlots = 8192;
+constexpr size_t kSoMail = kSoQueue + (size_t)kQueueSlots * sizeof(Job);  // the blocks' mailboxes
+constexpr size_t kMaxBlocks = 8192;
+constexpr size_t kSoArena = kSoMail + kMaxBlocks * kMailStride * 8;
 constexpr size_t kArenaBytes = kScratchBytes - kSoArena;
 static_assert(sizeof(SchedCounters) <= kSoEpoch - kSoSc, "counters overlap the epoch");
 static_assert(sizeof(QueryDesc) <= kSoRes - kSoQd, "query descriptor overlaps the results");
-static_assert(kSoQmask + kMaxWorkers / 8 <= kSoLut, "queue mask overlaps the class table");
+static_assert(kSoRes + kResSlots * 8 <= kSoLut, "results overlap the class table");
 static_assert(kSoQueue % 256 == 0 && kSoArena % 256 == 0, "misaligned scratch regions");
 
 // Device address of `scratch` per device, taken once per device with the
@@ -126,7 +127,7 @@ static int noalloc_count(dm_graph *g, bool motif, int K, const dm_config &cfg, u
     if ((r = pick_shape(g, K, motif, cfg, sh))) return r;
     const int wpb = sh.threads / sh.vwave;
     const int64_t fit_blocks = (int64_t)kArenaBytes / (arena * wpb);
-    const int64_t fit_workers = std::min<int64_t>(fit_blocks * wpb, (int64_t)kMaxWorkers);
+    const int64_t fit_workers = std::min<int64_t>(std::min<int64_t>(fit_blocks, kMaxBlocks) * wpb, (int64_t)kMaxWorkers);
     if (fit_workers < wpb)
         return set_error(DM_ERR_ARG, "dm_count_noalloc: one block of %d workers needs %lld bytes of stack arena, "
                                      "beyond the %zu bytes of the static scratch", wpb, (long long)(arena * wpb),
@@ -171,9 +172,10 @@ static int noalloc_count(dm_graph *g, bool motif, int K, const dm_config &cfg, u
     p.sq_off = nullptr;
     p.sq_jobs = nullptr;  // strided static partition
     p.sq_cur = (int32_t *)(sp + kSoCur);
-    p.qmask = motif ? (unsigned long long *)(sp + kSoQmask) : nullptr;  // motifs only, as in dm_count
+    p.res_copies = 1;
     p.q = (Job *)(sp + kSoQueue);
     p.q_cap = kQueueSlots;
+    p.mail = (unsigned long long *)(sp + kSoMail);
     p.epoch = (const int32_t *)(sp + kSoEpoch);
     p.sc = (SchedCounters *)(sp + kSoSc);
     p.arena = sp + kSoArena;
@@ -185,20 +187,20 @@ static int noalloc_count(dm_graph *g, bool motif, int K, const dm_config &cfg, u
     p.bitmap = cfg.clique_bitmap ? 1 : 0;
     p.watchdog_ticks = cfg.watchdog_s > 0 ? (uint64_t)(cfg.watchdog_s * d->wall_khz * 1000.0) : 0;
     const unsigned long long njobs = (unsigned long long)n;
-    const int queues = (int)std::min<int64_t>(n, sh.workers);
-    if ((r = enum_init_launch(p, njobs, queues, (int32_t *)(sp + kSoEpoch), res, nres, nullptr, 0, s))) return r;
+    if ((r = enum_init_launch(p, njobs, (int32_t *)(sp + kSoEpoch), res, nres, nullptr, 0, sh.blocks, s))) return r;
     if ((e = hipEventRecord(d->ev0, s)) != hipSuccess) return set_error(DM_ERR_HIP, "event: %s", hipGetErrorString(e));
     if (njobs > 0 && (r = enum_launch(p, launch_mode(motif, K), sh.vwave, sh.blocks, sh.threads, sh.lds_total, s)))
         return r;
     if ((e = hipEventRecord(d->ev1, s)) != hipSuccess) return set_error(DM_ERR_HIP, "event: %s", hipGetErrorString(e));
-    SchedCounters sc1;
-    e = hipMemcpyAsync(&sc1, sp + kSoSc, sizeof(sc1), hipMemcpyDeviceToHost, s);
+    SchedCounters sc;
+    e = hipMemcpyAsync(&sc, sp + kSoSc, sizeof(sc), hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipMemcpyAsync(out, res, nres * 8, hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e != hipSuccess) return set_error(DM_ERR_HIP, "result copy: %s", hipGetErrorString(e));
     float kms = 0;
     (void)hipEventElapsedTime(&kms, d->ev0, d->ev1);
-    if (sc1.error) return device_error(sc1.error, "enumeration kernel");
+    if (sc.error) return device_error(sc.error, "enumeration kernel");
+    const SchedStats sc1 = sched_totals(sc);
     uint64_t total = 0;
     for (size_t i = 0; i < nres; i++) total += out[i];
     if (total_out) *total_out = total;

@@ -117,8 +117,8 @@ int device_ctx(DeviceCtx **out) {
     HIPCHK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
     HIPCHK(hipEventCreate(&c->ev0));
     HIPCHK(hipEventCreate(&c->ev1));
-    // donated-job queue: 2^20 slots; epoch 0 never matches a launch
-    const size_t qcap = (size_t)1 << 20;
+    // job slots, one per worker; epoch 0 never matches a launch
+    const size_t qcap = (size_t)1 << 16;
     int r = dev_grow(c->d_q, c->q_cap_alloc, qcap);
     if (r) return r;
     HIPCHK(hipMemset(c->d_q, 0, qcap * sizeof(Job)));
@@ -501,10 +501,13 @@ int run_enum(dm_graph *g, int K, bool motif, const dm_config &cfg, uint64_t *his
     if ((r = dev_grow(d->d_sq_off, d->sq_off_cap, sq_off.size()))) return r;
     if ((r = dev_grow(d->d_sq_jobs, d->sq_jobs_cap, std::max<size_t>(sq_jobs.size(), 4)))) return r;
     if ((r = dev_grow(d->d_sq_cur, d->sq_cur_cap, (size_t)sh.workers))) return r;
-    if ((r = dev_grow(d->d_qmask, d->qmask_cap, (size_t)qmask_words(sh.workers, part->group)))) return r;
+    if ((r = dev_grow(d->d_mail, d->mail_cap, (size_t)sh.blocks * kMailStride))) return r;
     const size_t ncls = tab ? (size_t)tab->ncls : 0;
     const size_t nres = motif ? ncls : 1;
-    if ((r = dev_grow(d->d_results, d->results_cap, std::max<size_t>(nres, 1)))) return r;
+    // the blocks add to copies of the results, summed below
+    const int copies = result_copies(nres), stride = result_stride(nres);
+    const size_t nslots = (size_t)copies * stride;
+    if ((r = dev_grow(d->d_results, d->results_cap, nslots))) return r;
     const uint16_t *lut = nullptr;
     if (tab && (r = device_lut(d, K, &lut))) return r;
     const bool want_cost = cfg.record_costs != 0, want_cnt = cfg.per_root != 0;
@@ -527,7 +530,7 @@ int run_enum(dm_graph *g, int K, bool motif, const dm_config &cfg, uint64_t *his
     }
 
     // pinned staging for the counters and results read back after the launch
-    const size_t stage_need = sizeof(SchedCounters) + std::max<size_t>(nres, 1) * 8;
+    const size_t stage_need = sizeof(SchedCounters) + nslots * 8;
     if (stage_need > d->stage_cap) {
         if (d->h_stage) (void)hipHostFree(d->h_stage);
         d->h_stage = nullptr;
@@ -575,6 +578,7 @@ int run_enum(dm_graph *g, int K, bool motif, const dm_config &cfg, uint64_t *his
     p.sq_cur = d->d_sq_cur;
     p.q = d->d_q;
     p.q_cap = (uint32_t)d->q_cap_alloc;
+    p.mail = d->d_mail;
     p.epoch = d->d_epoch;
     p.start_ticks = nullptr;
     p.sc = d->d_sc;
@@ -594,14 +598,9 @@ int run_enum(dm_graph *g, int K, bool motif, const dm_config &cfg, uint64_t *his
     p.pre = npre ? d->d_pre : nullptr;
     p.pre_cursor = npre ? d->d_pre_cursor : nullptr;
     p.q_group = part->group;
-    // mask-guided steals for motifs only (motif k=4 on Chung-Lu 18K: 4.74 ->
-    // 4.65 ms).  A clique launch's makespan is a few long jobs, which run
-    // faster beside idle workers that sleep than beside thieves that always
-    // find a light job (R-MAT s17 k=5: 1.43 -> 1.54 ms with the mask).
-    p.qmask = motif ? d->d_qmask : nullptr;
-    int queues = 0;
-    for (size_t w = 0; w + 1 < sq_off.size(); w++) queues += sq_off[w + 1] > sq_off[w] ? 1 : 0;
-    if ((r = enum_init_launch(p, (unsigned long long)njobs, queues, d->d_epoch, d->d_results, nres, nullptr, 0, s)))
+    p.res_copies = copies;
+    p.res_stride = stride;
+    if ((r = enum_init_launch(p, (unsigned long long)njobs, d->d_epoch, d->d_results, nslots, nullptr, 0, sh.blocks, s)))
         return r;
 
     // the kernel time includes the bitmap pre-pass of a learned partition
@@ -611,15 +610,17 @@ int run_enum(dm_graph *g, int K, bool motif, const dm_config &cfg, uint64_t *his
         return r;
     HIPCHK(hipEventRecord(d->ev1, s));
     HIPCHK(hipMemcpyAsync(d->h_stage, d->d_sc, sizeof(SchedCounters), hipMemcpyDeviceToHost, s));
-    HIPCHK(hipMemcpyAsync(d->h_stage + sizeof(SchedCounters), d->d_results, nres * 8, hipMemcpyDeviceToHost, s));
+    HIPCHK(hipMemcpyAsync(d->h_stage + sizeof(SchedCounters), d->d_results, nslots * 8, hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));
-    SchedCounters sc1;
-    memcpy(&sc1, d->h_stage, sizeof(sc1));
-    std::vector<unsigned long long> h(nres);
-    if (nres) memcpy(h.data(), d->h_stage + sizeof(SchedCounters), nres * 8);
+    const SchedCounters &sc = *(const SchedCounters *)d->h_stage;
+    const SchedStats sc1 = sched_totals(sc);
+    std::vector<unsigned long long> h(nres, 0);
+    const unsigned long long *hc = (const unsigned long long *)(d->h_stage + sizeof(SchedCounters));
+    for (int c = 0; c < copies; c++)
+        for (size_t i = 0; i < nres; i++) h[i] += hc[(size_t)c * stride + i];
     float kms = 0;
     HIPCHK(hipEventElapsedTime(&kms, d->ev0, d->ev1));
-    if (sc1.error) return device_error(sc1.error, "enumeration kernel");
+    if (sc.error) return device_error(sc.error, "enumeration kernel");
     uint64_t total = 0;
     if (motif) {
         for (size_t i = 0; i < ncls; i++) total += h[i];

@@ -16,8 +16,8 @@ namespace dm {
 
 // State of one GPU, created on first use and kept until the process ends.
 // Every counting launch on the device goes to its one stream, so launches run
-// one after another on the GPU; that is what lets them share the donated-job
-// queue (slots are tagged with the launch epoch) and the workspaces.  `mu` is
+// one after another on the GPU; that is what lets them share the workers' job
+// slots (tagged with the launch epoch) and the workspaces.  `mu` is
 // held for the whole of a call that uses the stream or the workspaces (it is
 // recursive: a learned partition runs a k=3 count inside a counting call).
 struct DeviceCtx {
@@ -28,7 +28,7 @@ struct DeviceCtx {
     std::recursive_mutex mu;
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
-    // donated-job queue (fixed size, never reallocated: batches capture it)
+    // the workers' job slots (fixed size, never reallocated: batches capture it)
     Job *d_q = nullptr;
     size_t q_cap_alloc = 0;
     int32_t *d_epoch = nullptr;
@@ -43,10 +43,10 @@ struct DeviceCtx {
     size_t sq_jobs_cap = 0;
     int32_t *d_sq_cur = nullptr;
     size_t sq_cur_cap = 0;
-    unsigned long long *d_qmask = nullptr;  // non-empty static queues
-    size_t qmask_cap = 0;
+    unsigned long long *d_mail = nullptr;  // the blocks' mailboxes
+    size_t mail_cap = 0;
     SchedCounters *d_sc = nullptr;
-    unsigned long long *d_results = nullptr;  // clique count or motif histogram
+    unsigned long long *d_results = nullptr;  // clique count or motif histogram, in copies
     size_t results_cap = 0;
     QueryDesc *d_qd = nullptr;
     size_t qd_cap = 0;
