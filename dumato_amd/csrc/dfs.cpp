@@ -204,7 +204,7 @@ static int dfs_reset(dm_dfs *s) {
 static int dfs_launch(dm_dfs *s, const void *kernel) {
     dm_dfs_data d = s->d;
     void *args[] = {&d};
-    const size_t lds = s->motif ? (size_t)s->ncls * 8 : 0;
+    const size_t lds = (s->motif ? (size_t)s->ncls * 8 : 0) + (size_t)(256 / s->vw) * DM_DFS_ROW_BYTES;
     hipError_t e = hipLaunchKernel(kernel, dim3(s->blocks), dim3(256), args, lds, s->ctx->stream);
     if (e != hipSuccess) return set_error(DM_ERR_HIP, "step-API kernel launch: %s", hipGetErrorString(e));
     s->last.launches++;

@@ -242,6 +242,7 @@ void dm_batch_free(dm_batch *b);
 /* Per-worker DFS state in device memory, passed by value to the kernel.
  * Vertex ids are the graph's degree ranks (ascending (degree, id)). */
 #define DM_DFS_MAXK 16
+#define DM_DFS_ROW_BYTES (DM_DFS_MAXK * 20) /* a worker's rows in LDS while a kernel runs */
 typedef struct dm_dfs_data {
     const int64_t *off;       /* symmetric CSR: off[n+1], adj, each list ascending */
     const int32_t *adj;
