@@ -237,6 +237,18 @@ constexpr int64_t prebuilt_bytes(int32_t d) {
     return nw ? (((int64_t)d * nw * 8 + (int64_t)d * 4 + 15) & ~(int64_t)15) : 0;
 }
 
+// step-API state kernels (dfs_kernels.hip)
+struct DfsMove {  // a job moved to another worker's queue
+    int64_t slot;
+    uint64_t ind;
+    int32_t level;
+    int32_t id[DM_DFS_MAXK];
+    int32_t pad;
+};
+int dfs_reset_launch(const dm_dfs_data &d, const int32_t *roots, int nroots, void *stream);
+int dfs_gather_launch(const dm_dfs_data &d, const int64_t *at, int32_t *out, void *stream);
+int dfs_scatter_launch(const dm_dfs_data &d, const DfsMove *mv, int n, void *stream);
+
 }  // namespace dm
 
 #endif
