@@ -94,12 +94,24 @@ struct Grp {
         else return __shfl(x, src, W);
     }
     DEV int iscan(int x) const {  // inclusive prefix sum over the worker's lanes
+        if constexpr (W == 64) {
+            // within rows of 16 lanes (row_shr 1, 2, 4, 8), then the row ends
+            // added to the rows above them (row_bcast 15, 31)
+            x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);
+            x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);
+            x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);
+            x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);
+            x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);
+            x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);
+            return x;
+        } else {
 #pragma unroll
-        for (int o = 1; o < W; o <<= 1) {
-            int y = __shfl_up(x, o, W);
-            if (gl >= o) x += y;
+            for (int o = 1; o < W; o <<= 1) {
+                int y = __shfl_up(x, o, W);
+                if (gl >= o) x += y;
+            }
+            return x;
         }
-        return x;
     }
     DEV unsigned long long bcast64(unsigned long long x, int src) const {
         if constexpr (W == 64) {
@@ -140,6 +152,14 @@ DEV void lsync() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
 // LDS words addressed as such (ds instructions; a generic pointer takes flat ones)
 using lds_u32 = __attribute__((address_space(3))) uint32_t;
 using lds_u64 = __attribute__((address_space(3))) uint64_t;
+// global memory addressed as such: a generic pointer takes flat loads, which
+// the LDS counter waits for too, so LDS reads between them end their overlap
+using glb_i32 = const __attribute__((address_space(1))) int32_t;
+using glb_i64 = const __attribute__((address_space(1))) int64_t;
+using glb_u8 = const __attribute__((address_space(1))) uint8_t;
+using glb_u16 = const __attribute__((address_space(1))) uint16_t;
+using glb_u32 = __attribute__((address_space(1))) uint32_t;
+using glb_u64 = __attribute__((address_space(1))) uint64_t;
 // The atomic that returned x has been performed before any access that
 // follows in the program (its result is waited for here).
 template <class T>
@@ -154,7 +174,8 @@ template <class P>
 DEV void lor(P *a, uint64_t v) {
     (void)__hip_atomic_fetch_or(a, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
 }
-DEV int lower_bound(const int32_t *a, int n, int32_t x) {
+template <class P>
+DEV int lower_bound(P a, int n, int32_t x) {
     int lo = 0, hi = n;
     while (lo < hi) {
         int mid = (lo + hi) >> 1;
@@ -228,15 +249,17 @@ DEV WorkerLDS worker_lds(char *base, int K) {
 // fewer (over the leaf nodes of Chung-Lu 18K k = 4: 305 M against 1,116 M;
 // Barabasi-Albert 100K k = 4: 678 M against 3,557 M).  Calls against the
 // leaf that streamed every child's N(c): Chung-Lu 18K k = 4 4.76 -> 2.12 ms,
-// Barabasi-Albert 100K k = 4 16.5 -> 5.9 ms, 12K k = 5 167 -> 43 ms.
+// Barabasi-Albert 100K k = 4 16.5 -> 5.9 ms, 12K k = 5 167 -> 43 ms, before the
+// steps described below.
 //
 // U is held in a hash table for these tests: buckets of two 32-bit slots, two
-// buckets per element, so a test is two 8-byte LDS reads and no loop.  A slot
-// holds the bits of the element's hash that its bucket does not determine
-// (32 - b), whether it sits in its second bucket, and its 6-bit code ^ 63
-// (code: its mask if valid, 32 if not; 63 marks an empty slot); together they
-// identify any 31-bit id once b >= 7.  The table is in LDS, or in the worker's
-// arena where U is too large for that.
+// buckets per element, so a test is two 8-byte LDS reads and no loop.  With h =
+// id * odd (a bijection of 32 bits) the top b bits of h name the first bucket;
+// a slot holds the other 32 - b bits in place (h << b), whether it sits in its
+// second bucket (the first one xor the next b bits of h), and its 6-bit code
+// ^ 63 (code: its mask if valid, 32 if not; 63 marks an empty slot), which
+// fits from b = 7 on.  The table is in LDS, or in the worker's arena where U is
+// too large for that.
 constexpr uint32_t kEmpty = 63;
 
 struct LeafSum {
@@ -247,64 +270,50 @@ struct LeafSum {
 // The table's b and hash split; slots are reached through lds (LDS) or glb.
 template <bool LDS>
 struct LeafTab {
-    using P32 = std::conditional_t<LDS, lds_u32 *, uint32_t *>;
-    using P64 = std::conditional_t<LDS, lds_u64 *, uint64_t *>;
+    using P32 = std::conditional_t<LDS, lds_u32 *, glb_u32 *>;
+    using P64 = std::conditional_t<LDS, lds_u64 *, glb_u64 *>;
     P32 t;
     int b, sh;     // 2^b buckets, sh = 32 - b
-    uint32_t mul;  // odd: the hash is a bijection
-    DEV uint32_t other(uint32_t bk, uint32_t r) const { return bk ^ (((r >> (sh - b)) ^ (r >> 1)) & ((1u << b) - 1)); }
+    uint32_t mul;  // odd
     // code of x (0: not in U)
     DEV int find(int32_t x) const {
-        const uint32_t h = (uint32_t)x * mul;
-        const uint32_t b1 = h >> sh, r = h & ((1u << sh) - 1), b2 = other(b1, r);
-        const uint32_t k1 = r << 7, k2 = k1 | 64;
+        const uint32_t h = (uint32_t)x * mul, b1 = h >> sh, k1 = h << b, b2 = b1 ^ (k1 >> sh);
         const uint64_t s1 = ((P64)t)[b1], s2 = ((P64)t)[b2];
         const uint32_t a0 = (uint32_t)s1 ^ k1, a1 = (uint32_t)(s1 >> 32) ^ k1;
-        const uint32_t a2 = (uint32_t)s2 ^ k2, a3 = (uint32_t)(s2 >> 32) ^ k2;
+        const uint32_t a2 = (uint32_t)s2 ^ (k1 | 64), a3 = (uint32_t)(s2 >> 32) ^ (k1 | 64);
         const uint32_t m0 = a0 < a1 ? a0 : a1, m1 = a2 < a3 ? a2 : a3;
         const uint32_t m = m0 < m1 ? m0 : m1;
         return m < 63 ? (int)(m ^ 63) : 0;
     }
-    // adds mask bit `bit` to x if it is in U and valid; false: not in U
-    DEV bool mark(int32_t x, uint32_t bit) const {
-        const uint32_t h = (uint32_t)x * mul;
-        const uint32_t b1 = h >> sh, r = h & ((1u << sh) - 1), b2 = other(b1, r);
-        const uint32_t k1 = r << 7;
+    // adds mask bit `bit` to x, which is in U, if it is valid
+    DEV void mark(int32_t x, uint32_t bit) const {
+        const uint32_t h = (uint32_t)x * mul, b1 = h >> sh, k1 = h << b, b2 = b1 ^ (k1 >> sh);
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             P32 s = t + 2 * (i < 2 ? b1 : b2) + (i & 1);
             const uint32_t v = *s, a = v ^ (k1 | (i < 2 ? 0 : 64));
-            if (a < 63) {
-                if (a != (32 ^ 63)) *s = v ^ bit;
-                return true;
-            }
+            if (a < 63 && a != (32 ^ 63)) *s = v ^ bit;
         }
-        return false;
     }
-    // inserts x (not present); false when no slot was found: a full bucket's
-    // element is moved on to its other bucket, which one by a mixed bit (a
-    // fixed order runs into cycles from half load on)
+    // inserts x (not present); false when no slot was found.  Every step is one
+    // exchange: what it displaces goes to the bucket's other slot, what that
+    // displaces to its own other bucket.  (At most 45% full, a wave needs 2-5
+    // steps of 9 instructions; compare-and-swap probes of the four slots took
+    // 70 instructions a round, 3 rounds a wave.)
     DEV bool insert(int32_t x, int code) const {
         const uint32_t h = (uint32_t)x * mul;
-        uint32_t bk = h >> sh, v = ((h & ((1u << sh) - 1)) << 7) | (uint32_t)(code ^ 63);
-        for (uint32_t it = 0; it < 256; it++) {
-            P32 s = t + 2 * bk;
-            if (cas(s, v) || cas(s + 1, v)) return true;
-            if (it == 0) {
-                P32 o = t + 2 * other(bk, v >> 7);
-                if (cas(o, v ^ 64) || cas(o + 1, v ^ 64)) return true;
+        uint32_t bk = h >> sh, v = (h << b) | (uint32_t)(code ^ 63);
+        for (int it = 0; it < 256; it++) {
+            v = __hip_atomic_exchange(t + 2 * bk + (it & 1), v, __ATOMIC_RELAXED, kScope);
+            if (v == kEmpty) return true;
+            if (it & 1) {
+                bk ^= v >> sh;
+                v ^= 64;
             }
-            v = __hip_atomic_exchange(s + (((v + it) * 0x85EBCA6Bu) >> 31), v, __ATOMIC_RELAXED, kScope);
-            bk = other(bk, v >> 7);
-            v ^= 64;
         }
         return false;
     }
     static constexpr int kScope = LDS ? __HIP_MEMORY_SCOPE_WAVEFRONT : __HIP_MEMORY_SCOPE_AGENT;
-    DEV static bool cas(P32 s, uint32_t v) {
-        uint32_t e = kEmpty;
-        return __hip_atomic_compare_exchange_strong(s, &e, v, __ATOMIC_RELAXED, __ATOMIC_RELAXED, kScope);
-    }
     DEV static void sync() {
         if constexpr (LDS) lsync();
         else wsync();
@@ -312,9 +321,11 @@ struct LeafTab {
     // U of the leaf: the parent's list (masks pm, nullptr: all 1) with the
     // order rule x > c, then nc[0, q), whose new elements get mask newc
     template <int W>
-    DEV bool build(const Grp<W> &g, const int32_t *puid, const uint8_t *pupm, int pnu, int32_t c, const int32_t *nc,
-                   int q, int newc) const {
-        for (int j = g.gl; j < (1 << b); j += W) ((P64)t)[j] = ((uint64_t)kEmpty << 32) | kEmpty;
+    DEV bool build(const Grp<W> &g, glb_i32 *puid, glb_u8 *pupm, int pnu, int32_t c, glb_i32 *nc, int q,
+                   int newc) const {
+        using V4 = uint32_t __attribute__((ext_vector_type(4)));
+        using P128 = std::conditional_t<LDS, __attribute__((address_space(3))) V4 *, __attribute__((address_space(1))) V4 *>;
+        for (int j = g.gl; j < (1 << (b - 1)); j += W) ((P128)t)[j] = V4{kEmpty, kEmpty, kEmpty, kEmpty};
         sync();
         bool ok = true;
         for (int j = g.gl; j < pnu; j += W) {
@@ -329,7 +340,8 @@ struct LeafTab {
             int32_t x = 0;
             if (j < q) {
                 x = nc[j];
-                add = pnu == 0 || !mark(x, (uint32_t)newc);
+                add = pnu == 0 || find(x) == 0;
+                if (!add) mark(x, (uint32_t)newc);
             }
             sync();
             if (add) ok &= insert(x, newc);
@@ -342,7 +354,7 @@ struct LeafTab {
 // Position of the first entry of a[0, n) not below x (ascending), by all the
 // worker's lanes: each step narrows the range W-fold.
 template <int W>
-DEV int wave_lower_bound(const Grp<W> &g, const int32_t *a, int n, int32_t x) {
+DEV int wave_lower_bound(const Grp<W> &g, glb_i32 *a, int n, int32_t x) {
     int lo = 0;
     while (n > 0) {
         const int st = (n + W - 1) / W;  // lane i looks at the end of piece i
@@ -356,49 +368,67 @@ DEV int wave_lower_bound(const Grp<W> &g, const int32_t *a, int n, int32_t x) {
     return lo;
 }
 
-// The lanes' lists adj[os, os + len) laid end to end, f(entry, tag of its
-// list) called for every entry, W consecutive ones at a time (U steps' loads in
-// flight; f(none, 0) where the lists end).  recs: list start and tag, by list;
-// bits: a set bit where a list starts, so the list of an entry is a popcount.
+// The lanes' lists (len entries at `list`) laid end to end, f(entry, tag of its
+// list) called for every entry, W consecutive ones at a time, U of those steps'
+// loads in flight (f(none, 0) past the lists' end).  recs: list address and
+// tag, by list; bits: a set bit where a list starts, so the list of an entry is
+// a popcount.  VALU-bound once the loads overlap: about 35 instructions a step
+// with the table test, against 104 with generic pointers, 64-bit index
+// arithmetic and a bounds check per step (with the insertions by exchange:
+// Chung-Lu 18K k = 4 1.44 -> 1.26 ms, Barabasi-Albert 12K k = 5 38.8 -> 33.3 ms,
+// triangles of R-MAT s18 1.63 -> 1.32 ms).
 template <int W, class F>
-DEV void stream_lists(const Grp<W> &g, lds_u64 *recs, lds_u64 *bits, const int32_t *adj, int64_t os, int len, int tag,
-                      int32_t none, F f) {
+DEV void stream_lists(const Grp<W> &g, lds_u64 *recs, lds_u64 *bits, glb_i32 *list, int len, int tag, int32_t none,
+                      F f) {
     const uint64_t mx = g.ballot(len > 0);
     const int sc = g.iscan(len), pre = sc - len;
     const int T = g.bcast(sc, W - 1);
-    if (len > 0) recs[g.below(mx)] = ((uint64_t)(os - pre) & 0xffffffffffffffull) | ((uint64_t)tag << 56);
+    // addresses have 48 bits (the first `pre` entries before a list may lie
+    // outside the array: they are not read)
+    if (len > 0) recs[g.below(mx)] = ((uint64_t)(list - pre) & 0xffffffffffffull) | ((uint64_t)tag << 56);
+    constexpr int U = 4;
     for (int p0 = 0; p0 < T; p0 += kLeafCap) {
         const int pe = T - p0 < kLeafCap ? T : p0 + kLeafCap;
-        for (int w = g.gl; w < kLeafCap / 64; w += W) bits[w] = 0;
+        for (int w = g.gl; w < kLeafCap / 64 + U; w += W) bits[w] = 0;
         lsync();
         if (len > 0 && pre >= p0 && pre < pe) lor(bits + ((pre - p0) >> 6), 1ull << ((pre - p0) & 63));
         // lists that started before this chunk
         int own0 = __popcll(g.ballot(len > 0 && pre < p0)) - 1;
         lsync();
-        constexpr int U = 4;
-        for (int t0 = p0; t0 < pe; t0 += U * W) {
+        // U * W positions from t0; the last ones (full = false) may end early
+        auto step = [&](int t0, auto full) {
+            uint64_t rec[U], seg[U];
             int32_t ys[U];
-            int cm[U];
+            int tg[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) seg[u] = bits[(t0 + u * W - p0) >> 6];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                if constexpr (W == 64) seg[u] = unil<W>(seg[u]);
+                else seg[u] = (seg[u] >> ((t0 + u * W - p0) & 63)) & ((1ull << W) - 1);
+                rec[u] = recs[own0 + __popcll(seg[u] & ((2ull << g.gl) - 1))];
+                own0 += __popcll(seg[u]);
+            }
 #pragma unroll
             for (int u = 0; u < U; u++) {
                 const int t = t0 + u * W + g.gl;
-                const int o = t0 + u * W - p0;
-                uint64_t seg = o < kLeafCap ? bits[o >> 6] : 0;
-                if constexpr (W == 64) seg = unil<W>(seg);
-                else seg = (seg >> (o & 63)) & ((1ull << W) - 1);
-                const int own = own0 + __popcll(seg & ((2ull << g.gl) - 1));
-                own0 += __popcll(seg);
-                ys[u] = none;
-                cm[u] = 0;
-                if (t < pe) {
-                    const uint64_t rec = recs[own];
-                    cm[u] = (int)(rec >> 56);
-                    ys[u] = adj[((int64_t)(rec << 8) >> 8) + t];
+                tg[u] = (int)(rec[u] >> 56);
+                glb_i32 *const a = (glb_i32 *)(rec[u] & 0xffffffffffffull) + t;
+                if constexpr (full) {
+                    ys[u] = *a;
+                } else {
+                    ys[u] = none;
+                    if (t < pe) ys[u] = *a;
+                    else tg[u] = 0;
                 }
             }
 #pragma unroll
-            for (int u = 0; u < U; u++) f(ys[u], cm[u]);
-        }
+            for (int u = 0; u < U; u++)
+                if (full || t0 + u * W < pe) f(ys[u], tg[u]);
+        };
+        int t0 = p0;
+        for (; t0 + U * W <= pe; t0 += U * W) step(t0, std::true_type{});
+        if (t0 < pe) step(t0, std::false_type{});
         lsync();
     }
 }
@@ -410,13 +440,16 @@ DEV void stream_lists(const Grp<W> &g, lds_u64 *recs, lds_u64 *bits, const int32
 // gtab: a table of 2^space slots in memory instead.  Not inlined: the node's
 // registers are then its own, not shared with the search around it.
 template <int W>
-__device__ __attribute__((noinline)) LeafSum motif_leaf(const int64_t *off, const int32_t *adj, const int64_t *ostart,
-                                                        const uint16_t *lut, const int32_t *puid, const uint8_t *pupm,
-                                                        uint32_t shist_at, uint32_t lds_at, uint32_t *gtab, uint64_t pind,
-                                                        int32_t v0, int K, int32_t c, int pmc, int pnu, int psdeg,
-                                                        int lo, int hi, int space) {
-    off = unil<W>(off), adj = unil<W>(adj), ostart = unil<W>(ostart), lut = unil<W>(lut);
-    puid = unil<W>(puid), pupm = unil<W>(pupm), gtab = unil<W>(gtab), pind = unil<W>(pind);
+__device__ __attribute__((noinline)) LeafSum motif_leaf(const int64_t *off_, const int32_t *adj_, const int64_t *ostart_,
+                                                        const uint16_t *lut_, const int32_t *puid_,
+                                                        const uint8_t *pupm_, uint32_t shist_at, uint32_t lds_at,
+                                                        uint32_t *gtab, uint64_t pind, int32_t v0, int K, int32_t c,
+                                                        int pmc, int pnu, int psdeg, int lo, int hi, int space) {
+    glb_i64 *const off = (glb_i64 *)unil<W>(off_), *const ostart = (glb_i64 *)unil<W>(ostart_);
+    glb_i32 *const adj = (glb_i32 *)unil<W>(adj_), *const puid = (glb_i32 *)unil<W>(puid_);
+    glb_u16 *const lut = (glb_u16 *)unil<W>(lut_);
+    glb_u8 *const pupm = (glb_u8 *)unil<W>(pupm_);
+    gtab = unil<W>(gtab), pind = unil<W>(pind);
     v0 = uni<W>(v0), K = uni<W>(K), c = uni<W>(c), pmc = uni<W>(pmc), pnu = uni<W>(pnu), psdeg = uni<W>(psdeg);
     lo = uni<W>(lo), hi = uni<W>(hi), space = uni<W>(space);
     lds_u64 *const lds = (lds_u64 *)(uintptr_t)(uint32_t)uni<W>((int)lds_at);
@@ -427,23 +460,25 @@ __device__ __attribute__((noinline)) LeafSum motif_leaf(const int64_t *off, cons
     const int64_t cb = unil<W>(off[c]), ce = unil<W>(off[c + 1]);
     const int sdeg = psdeg + (int)(ce - cb);
     const int64_t cs = root ? unil<W>(ostart[c]) : cb + wave_lower_bound(g, adj + cb, (int)(ce - cb), v0 + 1);
-    const int32_t *nc = adj + cs;  // N(c) above id[0]
+    glb_i32 *const nc = adj + cs;  // N(c) above id[0]
     const int q = (int)(ce - cs);
     const int tot = pnu + q;  // elements of U, common ones twice
     LeafSum r{0, 0, 0};
 
     lds_u64 *recs = lds;
     lds_u64 *bits = recs + W;
-    lds_u64 *qs = bits + kLeafCap / 64;
+    lds_u64 *qs = bits + kLeafCap / 64 + 4;
     lds_u32 *nm = (lds_u32 *)(qs + npm);
     lds_u32 *e = nm + npm;
-    const int ne = npm * (npm + 1) / 2, copies = leaf_copies(K);
+    // counters of a pair: npm x npm, several copies, up to k = 6; triangular at 7
+    const bool sq = K <= 6;
+    const int ne = sq ? npm * npm : npm * (npm + 1) / 2, copies = leaf_copies(K);
     LeafTab<true> tl;
     LeafTab<false> tg;
     if (!gtab) {
-        // at least 4/3 slots per element while the space allows it
+        // at most 45% full while the space allows it
         int b = 7;
-        while ((16 << b) <= space && 3 * (2 << b) < 5 * tot) b++;
+        while ((16 << b) <= space && 9 * (2 << b) < 20 * tot) b++;
         tl.t = (lds_u32 *)(lds + motif_leaf_fixed(W, K) / 8);
         tl.b = b, tl.sh = 32 - b;
         tl.mul = 0x9E3779B1u;
@@ -455,7 +490,7 @@ __device__ __attribute__((noinline)) LeafSum motif_leaf(const int64_t *off, cons
             return r;
         }
     } else {
-        tg.t = gtab;
+        tg.t = (glb_u32 *)gtab;
         tg.b = space - 1, tg.sh = 33 - space;
         tg.mul = 0x9E3779B1u;
         for (int tries = 0; !tg.build(g, puid, pupm, pnu, c, nc, q, newc); tries++) {
@@ -466,7 +501,6 @@ __device__ __attribute__((noinline)) LeafSum motif_leaf(const int64_t *off, cons
             tg.mul = tg.mul * 0x2545F491u + 2;  // another odd multiplier
         }
     }
-    auto find = [&](int32_t x) { return gtab ? tg.find(x) : tl.find(x); };
     for (int j = g.gl; j < ne * copies; j += W) e[j] = 0;
     for (int j = g.gl; j < npm; j += W) nm[j] = 0, qs[j] = 0;
     lsync();
@@ -474,15 +508,17 @@ __device__ __attribute__((noinline)) LeafSum motif_leaf(const int64_t *off, cons
     // elements of U, W at a time: n_i and q_i, then their out-lists (v0, in
     // place of an entry past their end, is never in U)
     uint32_t nnew = 0, enew = 0;  // class newc / (newc, newc), counted in registers
+    const int lw = K - 2;
     unsigned long long qnew = 0, by = 0, leaves = 0, rpairs = 0;
     lds_u32 *const ecopy = e + (g.gl & (copies - 1)) * ne;
-    for (int j0 = 0; j0 < tot; j0 += W) {
+    auto scan = [&](const auto &tab) {
+        for (int j0 = 0; j0 < tot; j0 += W) {
         const int j = j0 + g.gl;
         int32_t x = 0;
         int code = 0;
         if (j < tot) {
             x = j < pnu ? puid[j] : nc[j - pnu];
-            code = find(x);
+            code = tab.find(x);
             // a neighbour of c that an earlier list holds too is visited in
             // the parent's list
             if (j >= pnu && code != newc) code = 0;
@@ -508,18 +544,27 @@ __device__ __attribute__((noinline)) LeafSum motif_leaf(const int64_t *off, cons
                 if (root) rpairs += (unsigned long long)(tot - 1 - j);
             }
         }
-        stream_lists(g, recs, bits, adj, os, len, cx, v0, [&](int32_t y, int mx) {
-            const int cd = find(y);
-            if (cd) {
-                const int cy = cd & 31, a = mx > cy ? mx : cy, z = mx > cy ? cy : mx;
-                if (a == newc && z == newc) enew++;
-                else ladd(ecopy + (__umul24(a, a + 1) >> 1) + z, 1u);
+        stream_lists(g, recs, bits, adj + os, len, cx, v0, [&](int32_t y, int mx) {
+            const int cd = tab.find(y);
+            const bool nn = mx == newc && cd == newc;
+            enew += nn ? 1u : 0u;
+            if (cd && !nn) {
+                const int cy = cd & 31;
+                if (sq) {
+                    ladd(ecopy + ((mx << lw) + cy), 1u);
+                } else {
+                    const int a = mx > cy ? mx : cy, z = mx > cy ? cy : mx;
+                    ladd(ecopy + (__umul24(a, a + 1) >> 1) + z, 1u);
+                }
             }
         });
-    }
+        }
+    };
+    if (gtab) scan(tg);
+    else scan(tl);
     if (nnew) ladd(nm + newc, nnew);
     if (qnew) ladd(qs + newc, (uint64_t)qnew);
-    if (enew) ladd(e + newc * (newc + 1) / 2 + newc, enew);
+    if (enew) ladd(e + (sq ? (newc << lw) + newc : newc * (newc + 1) / 2 + newc), enew);
     lsync();
     if (copies > 1) {
         for (int t = g.gl; t < ne; t += W) {
@@ -531,7 +576,10 @@ __device__ __attribute__((noinline)) LeafSum motif_leaf(const int64_t *off, cons
     }
     // edges between masks i >= j (0: U \ E); the lut index of the prefix
     // id[0..K-3] and its child's mask i
-    auto edges = [&](int i, int j) -> uint64_t { return e[i * (i + 1) / 2 + j]; };
+    auto edges = [&](int i, int j) -> uint64_t {
+        if (!sq) return e[i * (i + 1) / 2 + j];
+        return i == j ? (uint64_t)e[(i << lw) + i] : (uint64_t)e[(i << lw) + j] + e[(j << lw) + i];
+    };
     const uint64_t ind = root ? 0 : pind + (K - 3 >= 2 ? (uint64_t)pmc << quick_off(K - 3) : 0);
     auto child = [&](int i) -> uint64_t { return root ? 0 : ind + ((uint64_t)i << quick_off(K - 2)); };
     const int o2 = quick_off(K - 1);
@@ -566,16 +614,17 @@ __device__ __attribute__((noinline)) LeafSum motif_leaf(const int64_t *off, cons
 // the call that builds the table (the root's later calls find it in place).
 // Bound by the table reads (R-MAT s18 of edge factor 16: 659 M tests a call,
 // 83 M triangles; one child at a time, each entry searched in the longer list:
-// 5.19 -> 1.81 ms).  lds_at: recs u64[W] | bits u64[kLeafCap / 64] | table.
-constexpr int kTriFixed = 64 * 8 + kLeafCap / 8;
+// 5.19 -> 1.81 ms).  lds_at: recs u64[W] | bits u64[kLeafCap / 64 + 4] | table.
+constexpr int kTriFixed = 64 * 8 + kLeafCap / 8 + 32;
 struct TriSum {
     unsigned long long cnt, by;  // this lane's share; by: out-degrees of the children
 };
 template <int W>
-__device__ __attribute__((noinline)) TriSum triangles(const int64_t *off, const int32_t *adj, const int64_t *ostart,
-                                                      uint32_t at, int b, int32_t v0, int lo, int hi, bool first,
+__device__ __attribute__((noinline)) TriSum triangles(const int64_t *off_, const int32_t *adj_,
+                                                      const int64_t *ostart_, uint32_t at, int b, int32_t v0, int lo, int hi, bool first,
                                                       bool &ok) {
-    off = unil<W>(off), adj = unil<W>(adj), ostart = unil<W>(ostart);
+    glb_i64 *const off = (glb_i64 *)unil<W>(off_), *const ostart = (glb_i64 *)unil<W>(ostart_);
+    glb_i32 *const adj = (glb_i32 *)unil<W>(adj_);
     b = uni<W>(b), v0 = uni<W>(v0), lo = uni<W>(lo), hi = uni<W>(hi);
     const Grp<W> g;
     lds_u64 *const recs = (lds_u64 *)(uintptr_t)(uint32_t)uni<W>((int)at);
@@ -584,12 +633,12 @@ __device__ __attribute__((noinline)) TriSum triangles(const int64_t *off, const 
     tab.t = (lds_u32 *)(recs + kTriFixed / 8);
     tab.b = b, tab.sh = 32 - b, tab.mul = 0x9E3779B1u;
     const int64_t ls = unil<W>(ostart[v0]);
-    const int32_t *const L = adj + ls;
+    glb_i32 *const L = adj + ls;
     TriSum r{0, 0};
     ok = true;
     if (first) {
         const int d = (int)(unil<W>(off[v0 + 1]) - ls);
-        ok = tab.build(g, L, nullptr, 0, v0, L, d, 1);
+        ok = tab.build(g, L, (glb_u8 *)nullptr, 0, v0, L, d, 1);
         if (!ok) return r;
     }
     for (int j0 = lo; j0 < hi; j0 += W) {
@@ -603,7 +652,7 @@ __device__ __attribute__((noinline)) TriSum triangles(const int64_t *off, const 
             r.by += (unsigned long long)len;
         }
         uint32_t found = 0;
-        stream_lists(g, recs, bits, adj, os, len, 0, v0, [&](int32_t y, int) { found += tab.find(y) ? 1 : 0; });
+        stream_lists(g, recs, bits, adj + os, len, 0, v0, [&](int32_t y, int) { found += tab.find(y) ? 1 : 0; });
         r.cnt += found;
     }
     return r;
@@ -1334,7 +1383,8 @@ struct Worker {
         Lvl &R = ws.lv()[0];
         const int d = R.nu;
         int b = 7;
-        while (3 * (2 << b) < 5 * d) b++;  // at most 3/5 full
+        while (9 * (2 << b) < 20 * d) b++;  // at most 45% full
+        while (b > 7 && kTriFixed + (8 << b) > p.lds_per_worker && 7 * d <= 6 * (1 << b)) b--;
         if (kTriFixed + (8 << b) > p.lds_per_worker) return false;
         R.cur = lo;
         R.end = hi < d ? hi : d;

@@ -214,12 +214,14 @@ constexpr int32_t make_job_query(int q, int steal_min) { return q | (steal_min <
 // for more waves per SIMD)
 inline int launch_mode(bool motif, int K) { return motif ? (K >= 5 ? 2 : 1) : 0; }
 // The motif leaf's LDS without its table, per worker of W lanes: recs u64[W] |
-// bits u64[kLeafCap / 64] | qs u64[npm] | n u32[npm] | e u32[copies][npm (npm + 1) / 2],
-// npm = 2^(K-2) mask values.  A motif launch gives each worker at least this.
+// bits u64[kLeafCap / 64 + 4] | qs u64[npm] | n u32[npm] | e u32[copies][npm * npm]
+// (k = 7: [npm (npm + 1) / 2]), npm = 2^(K-2) mask values.  A motif launch gives
+// each worker at least this.
 constexpr int kLeafCap = 2048;  // stream positions per chunk
 constexpr int leaf_copies(int K) { return K <= 4 ? 8 : K == 5 ? 2 : 1; }
 constexpr int motif_leaf_fixed(int W, int K) {
-    return (W * 8 + kLeafCap / 8 + (1 << (K - 2)) * (12 + leaf_copies(K) * ((1 << (K - 2)) + 1) * 2) + 15) & ~15;
+    return (W * 8 + kLeafCap / 8 + 32 + (1 << (K - 2)) * 12 +
+            (K <= 6 ? leaf_copies(K) * (4 << (2 * (K - 2))) : (1 << (K - 2)) * ((1 << (K - 2)) + 1) * 2) + 15) & ~15;
 }
 size_t enum_lds_bytes(int vwave, int threads, int kmax, int ncls_single, int hist_slots, int lds_per_worker);
 int enum_occupancy(int vwave, int mode, int threads, size_t lds, int *blocks_per_cu);
