@@ -1094,8 +1094,9 @@ struct Worker {
     // another job), else of a range job's untouched roots, else of the children
     // of the shallowest level of the job (below `top`) that has enough of them.
     // min_first > 0: the job's own level may be cut down to pieces of that
-    // many children (heavy children, where steal_min would leave too much).
-    DEV void maybe_donate(int top, int min_first = 0) {
+    // many children (heavy children, where steal_min would leave too much);
+    // min_pairs > 0: the same for the pairs of a bitmap root's child (level 1).
+    DEV void maybe_donate(int top, int min_first = 0, int min_pairs = 0) {
         unsigned long long rq = 0;
         int n = requests(rq);
         if (n == 0) return;
@@ -1134,7 +1135,10 @@ struct Worker {
         const int leaf_min = 4 * job_sm;
         for (int l = job_lvl; l < top; l++) {
             const int cur = ws.lv()[l].cur, end = ws.lv()[l].end;
-            const int minc = (min_first > 0 && l == job_lvl) ? min_first : l == K - 3 ? leaf_min : job_sm;
+            const int minc = min_pairs > 0 && l == 1                ? min_pairs
+                             : min_first > 0 && l == job_lvl ? min_first
+                             : l == K - 3                    ? leaf_min
+                                                             : job_sm;
             if (end - cur < minc) continue;
             int most = (end - cur) / minc - 1;
             most = most < 1 ? 1 : most > end - cur - 1 ? end - cur - 1 : most;
@@ -1408,7 +1412,7 @@ struct Worker {
 
     // ---- clique, local bitmap of the root's out-neighbourhood -------------
     template <int NW>
-    DEV void clique_bitmap_root(int32_t v, int lo, int hi, bool first_piece, bool shared) {
+    DEV void clique_bitmap_root(int32_t v, int lvl, int lo, int hi, bool first_piece, bool shared) {
         const int d = odeg(v);
         const int32_t *L = onbr(v);
         Lvl &R = ws.lv()[0];
@@ -1422,6 +1426,9 @@ struct Worker {
             lo = 0;
             hi = d;
         }
+        // level 1: pairs [lo, hi) of one child, at `child`
+        const int p0 = lo, p1 = hi, child = lvl ? uni<W>(lower_bound(L, d, ws.jid()[1])) : 0;
+        if (lvl) lo = child, hi = child + 1;
         if (hi > d) hi = d;
         if (lo >= hi) return;
         // pair-phase data first, so that it gets the LDS
@@ -1463,7 +1470,10 @@ struct Worker {
             st = alloc((int64_t)(K - 5) * stage_bytes(sw, NW));
             if (abort) return;
         }
-        if (shared) {
+        if (lvl) {
+            R.cur = R.end = hi;
+            pairs_of_child<NW>(R, rows, dp, pre, st, sw, child, p0, p1);
+        } else if (shared) {
             // guided self-scheduling with the root's other jobs: each claim
             // takes about 1 / (2 x jobs on the root) of the children left, at
             // least one, so the root's last children are spread thinly
@@ -1579,25 +1589,76 @@ struct Worker {
     // first-level children [lo, hi) in batches of W; each batch is
     // flattened into its (i, j) pairs, which the lanes stride over
     // (st, sw: the stages of K >= 6)
+    // a batch of the pairs described by pre, from child cur on
+    template <int NW>
+    DEV PairSum pairs(const uint64_t *rows, const int32_t *dp, const int32_t *pre, const char *st, int sw, int cur,
+                      int P) {
+        auto lds = [&](const void *a) { return (const char *)a >= lds_lo && (const char *)a < lds_lo + p.lds_per_worker; };
+        if (lds(rows) && lds(dp) && lds(pre) && (K < 6 || lds(st)))
+            return clique_pairs<W, NW, true>(lds_at(rows), lds_at(dp), lds_at(pre), lds_at(st), K, cur, P, sw);
+        return clique_pairs<W, NW, false>((uintptr_t)rows, (uintptr_t)dp, (uintptr_t)pre, (uintptr_t)st, K, cur, P, sw);
+    }
+
+    // k >= 6: the pairs [lo, hi) of child i alone, a chunk at a time, so that a
+    // heavy child's pairs are given away too: its work grows with the square
+    // (k = 6) of its pairs or faster, and one worker's share of a dense root
+    // would otherwise be the launch (8,192-vertex R-MAT k = 7: 1.90 ms with whole
+    // children, 1.28 ms with their pairs divided, 0.95 ms with batches of W / 2
+    // pairs instead of 2 W as well)
+    template <int NW>
+    DEV void pairs_of_child(Lvl &R, const uint64_t *rows, const int32_t *dp, int32_t *pre, char *st, int sw, int i,
+                            int lo, int hi) {
+        Lvl &C = ws.lv()[1];
+        int n = 0;
+#pragma unroll
+        for (int w = 0; w < NW; w++) n += __popcll(rows[i * NW + w]);
+        n = uni<W>(n);
+        C.vtx = R.uid[i];
+        C.nu = n;
+        C.cur = lo;
+        C.end = hi < n ? hi : n;
+        const int chunk = K >= 7 ? W / 4 : W;
+        while (true) {
+            if (check_abort()) return;
+            maybe_donate(2, 2, K >= 7 ? 4 : 32);
+            const int cur = uni<W>(C.cur), end = uni<W>(C.end);
+            if (cur >= end) return;
+            const int P = end - cur < chunk ? end - cur : chunk;
+            C.cur = cur + P;
+            if (g.gl == 0) pre[0] = -cur, pre[1] = P;
+            wsync();
+            const PairSum r = pairs<NW>(rows, dp, pre, st, sw, i, P);
+            cnt += r.cnt;
+            bytes += 4ull * r.by;
+            wsync();
+        }
+    }
+
     template <int NW>
     DEV void pair_phase(Lvl &R, const uint64_t *rows, const int32_t *dp, int32_t *pre, char *st, int sw, int lo,
                         int hi) {
-        auto lds = [&](const void *a) { return (const char *)a >= lds_lo && (const char *)a < lds_lo + p.lds_per_worker; };
-        const bool in_lds = lds(rows) && lds(dp) && lds(pre) && (K < 6 || lds(st));
+        // a front child with this many pairs is heavy enough to travel alone,
+        // with twice as many its pairs are divided too
+        const int heavy = K >= 7 ? 4 : W / 2;
         R.cur = lo;
         R.end = hi;
         unsigned long long by = 0;
         while (true) {
             if (check_abort()) break;
-            // at k >= 6 a front child with many pairs (its work grows with
-            // their cube) is heavy enough to travel alone
             int front = 0;
             if (K >= 6 && g.gl == 0 && R.cur < R.end) {
 #pragma unroll
                 for (int w = 0; w < NW; w++) front += __popcll(rows[R.cur * NW + w]);
             }
             front = g.bcast(front, 0);
-            maybe_donate(1, front >= W / 2 ? 2 : 0);
+            maybe_donate(1, front >= heavy ? 2 : 0);
+            if (front >= 2 * heavy && R.cur < R.end) {
+                const int i = R.cur;
+                R.cur = i + 1;
+                if (g.gl == 0) by += (unsigned long long)dp[i];
+                pairs_of_child<NW>(R, rows, dp, pre, st, sw, i, 0, 0x7fffffff);
+                continue;
+            }
             const int cur = R.cur, end = R.end;
             if (cur >= end) break;
             // a batch holds children until it has about `target` pairs (at
@@ -1609,7 +1670,7 @@ struct Worker {
                 for (int w = 0; w < NW; w++) np += __popcll(rows[(cur + g.gl) * NW + w]);
             }
             const int sc = g.iscan(np);
-            const int target = K == 4 ? 16 * W : 2 * W;
+            const int target = K == 4 ? 16 * W : K >= 7 ? W / 2 : 2 * W;
             int take = __popcll(g.ballot(g.gl < avail && sc - np < target));
             take = take < 1 ? 1 : take;
             R.cur = cur + take;
@@ -1620,12 +1681,7 @@ struct Worker {
             if (g.gl == 0) pre[0] = 0;
             const int P = g.bcast(sc, take - 1);
             wsync();
-            PairSum r;
-            if (in_lds)
-                r = clique_pairs<W, NW, true>(lds_at(rows), lds_at(dp), lds_at(pre), lds_at(st), K, cur, P, sw);
-            else
-                r = clique_pairs<W, NW, false>((uintptr_t)rows, (uintptr_t)dp, (uintptr_t)pre, (uintptr_t)st, K, cur,
-                                               P, sw);
+            const PairSum r = pairs<NW>(rows, dp, pre, st, sw, cur, P);
             cnt += r.cnt;
             by += r.by;
             wsync();
@@ -1656,18 +1712,18 @@ struct Worker {
             }
             return;
         }
-        if (!motif && p.bitmap && lvl == 0 && K >= 4) {
+        if (!motif && p.bitmap && K >= 4 && (lvl == 0 || (lvl == 1 && K >= 6))) {
             const int d = odeg(v0);
             if (d <= 64) {
-                clique_bitmap_root<1>(v0, lo, hi, first_piece, shared);
+                clique_bitmap_root<1>(v0, lvl, lo, hi, first_piece, shared);
                 return;
             }
             if (d <= 128) {
-                clique_bitmap_root<2>(v0, lo, hi, first_piece, shared);
+                clique_bitmap_root<2>(v0, lvl, lo, hi, first_piece, shared);
                 return;
             }
             if (d <= 256) {
-                clique_bitmap_root<4>(v0, lo, hi, first_piece, shared);
+                clique_bitmap_root<4>(v0, lvl, lo, hi, first_piece, shared);
                 return;
             }
         }

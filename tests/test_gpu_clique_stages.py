@@ -57,3 +57,22 @@ def test_complete_graph_every_size():
     for k in range(3, 13):
         print("case K26 clique k=%d" % k, flush=True)
         assert g.clique_count(k, dm.config(watchdog_s=60.0)) == math.comb(26, k)
+
+
+@pytest.mark.parametrize("n,p", [(64, 0.8), (120, 0.6), (220, 0.35)])
+def test_pairs_of_a_child_given_away(n, p):
+    # few dense roots, many idle workers, the smallest pieces: children's pairs
+    # travel as jobs of their own; with a learned partition too
+    s, d, nv = G.gnp(n, p, 70 + n)
+    ref = O.csr_from_edges(s, d, nv)
+    _, ro = O.relabel(ref, oriented=True)
+    for k in (6, 7):
+        want, by = O.clique_count(ref, k), O.clique_bytes(ro, k)
+        g = dm.Graph.from_edges(s, d, nv)
+        g.sched_train(False, 4, epochs=3, seed=1)
+        for w, kw in ((64, {}), (16, {}), (64, dict(sched=dm.DM_SCHED_LEARNED))):
+            print("case gnp n=%d clique k=%d w=%d %s" % (n, k, w, kw), flush=True)
+            cfg = dm.config(vwave=w, blocks=64, steal_min=2, steal_period=0, watchdog_s=60.0, **kw)
+            for _ in range(2):
+                assert g.clique_count(k, cfg) == want
+                assert g.last_stats()["alg_bytes"] == by
