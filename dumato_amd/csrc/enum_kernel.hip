@@ -150,6 +150,7 @@ DEV void wsync() { __threadfence_block(); }
 DEV void lsync() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
 
 // LDS words addressed as such (ds instructions; a generic pointer takes flat ones)
+using lds_u8 = __attribute__((address_space(3))) uint8_t;
 using lds_u32 = __attribute__((address_space(3))) uint32_t;
 using lds_u64 = __attribute__((address_space(3))) uint64_t;
 // global memory addressed as such: a generic pointer takes flat loads, which
@@ -285,6 +286,18 @@ struct LeafTab {
         const uint32_t m = m0 < m1 ? m0 : m1;
         return m < 63 ? (int)(m ^ 63) : 0;
     }
+    // where x lies, of a table whose codes are all 1 (-1: not in it)
+    DEV int slot(int32_t x) const {
+        const uint32_t h = (uint32_t)x * mul, b1 = h >> sh, k1 = h << b, b2 = b1 ^ (k1 >> sh);
+        const uint64_t s1 = ((P64)t)[b1], s2 = ((P64)t)[b2];
+        const uint32_t w = k1 | (1 ^ 63);
+        int at = -1;
+        at = (uint32_t)s1 == w ? 2 * (int)b1 : at;
+        at = (uint32_t)(s1 >> 32) == w ? 2 * (int)b1 + 1 : at;
+        at = (uint32_t)s2 == (w | 64) ? 2 * (int)b2 : at;
+        at = (uint32_t)(s2 >> 32) == (w | 64) ? 2 * (int)b2 + 1 : at;
+        return at;
+    }
     // adds mask bit `bit` to x, which is in U, if it is valid
     DEV void mark(int32_t x, uint32_t bit) const {
         const uint32_t h = (uint32_t)x * mul, b1 = h >> sh, k1 = h << b, b2 = b1 ^ (k1 >> sh);
@@ -376,8 +389,10 @@ DEV int wave_lower_bound(const Grp<W> &g, glb_i32 *a, int n, int32_t x) {
 // with the table test, against 104 with generic pointers, 64-bit index
 // arithmetic and a bounds check per step (with the insertions by exchange:
 // Chung-Lu 18K k = 4 1.44 -> 1.26 ms, Barabasi-Albert 12K k = 5 38.8 -> 33.3 ms,
-// triangles of R-MAT s18 1.63 -> 1.32 ms).
-template <int W, class F>
+// triangles of R-MAT s18 1.63 -> 1.32 ms).  U = 4 in the motif leaf, whose
+// registers allow no more, 8 in the clique kernel at 3 waves per SIMD
+// (triangles of R-MAT s18 of edge factor 8 1.05 -> 1.00 ms).
+template <int U, int W, class F>
 DEV void stream_lists(const Grp<W> &g, lds_u64 *recs, lds_u64 *bits, glb_i32 *list, int len, int tag, int32_t none,
                       F f) {
     const uint64_t mx = g.ballot(len > 0);
@@ -386,7 +401,6 @@ DEV void stream_lists(const Grp<W> &g, lds_u64 *recs, lds_u64 *bits, glb_i32 *li
     // addresses have 48 bits (the first `pre` entries before a list may lie
     // outside the array: they are not read)
     if (len > 0) recs[g.below(mx)] = ((uint64_t)(list - pre) & 0xffffffffffffull) | ((uint64_t)tag << 56);
-    constexpr int U = 4;
     for (int p0 = 0; p0 < T; p0 += kLeafCap) {
         const int pe = T - p0 < kLeafCap ? T : p0 + kLeafCap;
         for (int w = g.gl; w < kLeafCap / 64 + U; w += W) bits[w] = 0;
@@ -544,7 +558,7 @@ __device__ __attribute__((noinline)) LeafSum motif_leaf(const int64_t *off_, con
                 if (root) rpairs += (unsigned long long)(tot - 1 - j);
             }
         }
-        stream_lists(g, recs, bits, adj + os, len, cx, v0, [&](int32_t y, int mx) {
+        stream_lists<4>(g, recs, bits, adj + os, len, cx, v0, [&](int32_t y, int mx) {
             const int cd = tab.find(y);
             const bool nn = mx == newc && cd == newc;
             enew += nn ? 1u : 0u;
@@ -614,8 +628,8 @@ __device__ __attribute__((noinline)) LeafSum motif_leaf(const int64_t *off_, con
 // the call that builds the table (the root's later calls find it in place).
 // Bound by the table reads (R-MAT s18 of edge factor 16: 659 M tests a call,
 // 83 M triangles; one child at a time, each entry searched in the longer list:
-// 5.19 -> 1.81 ms).  lds_at: recs u64[W] | bits u64[kLeafCap / 64 + 4] | table.
-constexpr int kTriFixed = 64 * 8 + kLeafCap / 8 + 32;
+// 5.19 -> 1.81 ms).  lds_at: recs u64[W] | bits u64[kLeafCap / 64 + 8] | table.
+constexpr int kTriFixed = 64 * 8 + kLeafCap / 8 + 64;
 struct TriSum {
     unsigned long long cnt, by;  // this lane's share; by: out-degrees of the children
 };
@@ -652,7 +666,7 @@ __device__ __attribute__((noinline)) TriSum triangles(const int64_t *off_, const
             r.by += (unsigned long long)len;
         }
         uint32_t found = 0;
-        stream_lists(g, recs, bits, adj + os, len, 0, v0, [&](int32_t y, int) { found += tab.find(y) ? 1 : 0; });
+        stream_lists<8>(g, recs, bits, adj + os, len, 0, v0, [&](int32_t y, int) { found += tab.find(y) ? 1 : 0; });
         r.cnt += found;
     }
     return r;
@@ -681,11 +695,144 @@ __device__ __attribute__((noinline)) TriSum triangles(const int64_t *off_, const
 struct PairSum {
     unsigned long long cnt, by;  // this lane's share
 };
+// Rows lo..d-1 of the bitmap of root v0's out-neighbourhood L (two or more
+// words a row, d <= 64 NW): the out-lists N+(L[i]) laid end to end over the
+// lanes, each entry looked up in a table of L, whose slots' positions are a
+// byte array.  False when the table could not be filled.  Latency-bound: three
+// dependent loads a child batch, then a list step's loads; eight of those are in
+// flight.  (R-MAT s17 of edge factor 8, a root of 100 children with its pairs
+// at k = 5: 155 -> 98 us against build_rows' linear probes through generic
+// pointers.)
+// at: recs u64[W] | bits u64[kLeafCap / 64 + 8] | table | positions.
+constexpr int rows_bits(int NW) { return NW == 4 ? 8 : 7; }
+constexpr int rows_scratch(int NW) { return kTriFixed + 10 * (1 << rows_bits(NW)); }
+template <int W, int NW>
+__device__ __attribute__((noinline)) bool root_rows(const int64_t *off_, const int32_t *adj_, const int64_t *ostart_,
+                                                    uint32_t at, uint32_t rows_at, uint32_t dp_at, int32_t v0, int lo,
+                                                    int d) {
+    glb_i64 *const off = (glb_i64 *)unil<W>(off_), *const ostart = (glb_i64 *)unil<W>(ostart_);
+    glb_i32 *const adj = (glb_i32 *)unil<W>(adj_);
+    v0 = uni<W>(v0), lo = uni<W>(lo), d = uni<W>(d);
+    const Grp<W> g;
+    lds_u64 *const recs = (lds_u64 *)(uintptr_t)(uint32_t)uni<W>((int)at);
+    lds_u64 *const bits = recs + 64;
+    lds_u64 *const rows = (lds_u64 *)(uintptr_t)(uint32_t)uni<W>((int)rows_at);
+    lds_u32 *const dp = (lds_u32 *)(uintptr_t)(uint32_t)uni<W>((int)dp_at);
+    constexpr int b = rows_bits(NW);
+    LeafTab<true> tab;
+    tab.t = (lds_u32 *)(recs + kTriFixed / 8);
+    tab.b = b, tab.sh = 32 - b, tab.mul = 0x9E3779B1u;
+    lds_u8 *const val = (lds_u8 *)(tab.t + (2 << b));
+    glb_i32 *const L = adj + unil<W>(ostart[v0]);
+    for (int t = g.gl; t < (2 << b); t += W) tab.t[t] = kEmpty;
+    for (int t = lo * NW + g.gl; t < d * NW; t += W) rows[t] = 0;
+    lsync();
+    // only children above lo can be set in rows lo.. (lists are sorted)
+    bool ok = true;
+    for (int j = lo + 1 + g.gl; j < d; j += W) ok &= tab.insert(L[j], 1);
+    lsync();
+    if (g.ballot(!ok)) return false;
+    for (int j = lo + 1 + g.gl; j < d; j += W) val[tab.slot(L[j])] = (uint8_t)j;
+    lsync();
+    for (int j0 = lo; j0 < d; j0 += W) {
+        const int j = j0 + g.gl;
+        int len = 0;
+        int64_t os = 0;
+        if (j < d) {
+            const int32_t u = L[j];
+            os = ostart[u];
+            len = (int)(off[u + 1] - os);
+            dp[j] = (uint32_t)len;
+            if (j == d - 1) len = 0;  // no child above the last
+        }
+        stream_lists<8>(g, recs, bits, adj + os, len, g.gl, v0, [&](int32_t y, int i) {
+            const int s = tab.slot(y);
+            if (s >= 0) {
+                const int k = val[s];
+                lor(rows + (j0 + i) * NW + (k >> 6), 1ull << (k & 63));
+            }
+        });
+    }
+    return true;
+}
+
+// One bitmap over the out-neighbourhoods of several light roots (lane's root v
+// with d children, sum of the d's T <= W): child i of the r-th root is position
+// pre_r + i, and a row holds positions of its own root only, so the cliques in
+// it are those of all the roots.  Rows and out-degrees as for one root; an
+// out-list's entries are searched among their root's children above it.
+// A root of 8 children leaves most lanes idle and waits for the same chain of
+// loads as a full one; together they share it.  The search in LDS (1 to 5
+// steps) costs 10-25 instructions an entry, about as much as a table's probe,
+// and needs no table.  (Barabasi-Albert 100K k = 4 0.41 -> 0.12 ms, Chung-Lu 50K
+// k = 4 0.27 -> 0.12, uniform random of 2 M edges k = 3 0.39 -> 0.22, R-MAT s18
+// of edge factor 8 k = 4 1.47 -> 0.82.)
+// at: recs u64[W] | bits u64[kLeafCap / 64 + 8] | children i32[W] | spans u32[W].
+constexpr int kLightScratch = kTriFixed + 2 * 64 * 4;
+template <int W>
+__device__ __attribute__((noinline)) void light_rows(const int64_t *off_, const int32_t *adj_, const int64_t *ostart_,
+                                                     uint32_t at, uint32_t rows_at, uint32_t dp_at, int32_t v, int d,
+                                                     int lo) {
+    glb_i64 *const off = (glb_i64 *)unil<W>(off_), *const ostart = (glb_i64 *)unil<W>(ostart_);
+    glb_i32 *const adj = (glb_i32 *)unil<W>(adj_);
+    const Grp<W> g;
+    lds_u64 *const recs = (lds_u64 *)(uintptr_t)(uint32_t)uni<W>((int)at);
+    lds_u64 *const bits = recs + 64;
+    lds_u32 *const kid = (lds_u32 *)(recs + kTriFixed / 8), *const span = kid + 64;
+    lds_u64 *const rows = (lds_u64 *)(uintptr_t)(uint32_t)uni<W>((int)rows_at);
+    lds_u32 *const dp = (lds_u32 *)(uintptr_t)(uint32_t)uni<W>((int)dp_at);
+    const int sc = g.iscan(d), T = g.bcast(sc, W - 1);
+    // the lane's position: its root's first and one past its last
+    span[g.gl] = 0;
+    lsync();
+    if (d > 0) span[sc - d] = (uint32_t)g.gl + 1;
+    lsync();
+    const uint64_t first = g.ballot(span[g.gl] != 0), upto = (2ull << g.gl) - 1;
+    const int s = 63 - __builtin_clzll(first & upto | 1);
+    const int e = first & ~upto ? __builtin_ctzll(first & ~upto) : T;
+    const int r = (int)span[s] - 1;
+    const int64_t ls = __shfl(d > 0 ? (long long)ostart[v] : 0ll, r < 0 ? 0 : r, W);
+    int most = d;
+    for (int o = W / 2; o; o >>= 1) {
+        const int x = __shfl_xor(most, o, W);
+        most = x > most ? x : most;
+    }
+    most = uni<W>(most);
+    int32_t u = 0x7fffffff;
+    int len = 0;
+    int64_t os = 0;
+    if (g.gl < T) {
+        u = adj[ls + g.gl - s];
+        os = ostart[u];
+        len = (int)(off[u + 1] - os);
+        dp[g.gl] = (uint32_t)len;
+        rows[g.gl] = 0;
+        if (g.gl < lo || g.gl + 1 == e) len = 0;  // no child above the last
+    }
+    lsync();
+    kid[g.gl] = (uint32_t)u;
+    span[g.gl] = (uint32_t)e;
+    lsync();
+    const int top = most > 1 ? 1 << (31 - __builtin_clz(most - 1)) : 0;
+    stream_lists<8>(g, recs, bits, adj + os, len, g.gl, -1, [&](int32_t y, int i) {
+        // the last child <= y of (i, e)
+        const int e = (int)span[i];
+        int a = i;
+        for (int o = top; o; o >>= 1) {
+            const int32_t x = (int32_t)kid[a + o];  // past the children: in span
+            a += a + o < e && x <= y ? o : 0;
+        }
+        if (a > i && (int32_t)kid[a] == y) lor(rows + i, 1ull << a);
+    });
+}
+
 // bytes of one stage of sw sets: sets u64[sw * NW] | prefix u32[sw + 1], size,
 // cursor
 __host__ __device__ constexpr int stage_bytes(int sw, int NW) { return sw * NW * 8 + ((sw + 4) & ~1) * 4; }
 // a child's own bitmap: rows u64[64], the set of all its elements, dp i32[64]
 constexpr int kChildBytes = 65 * 8 + 64 * 4;
+// a light batch: rows, out-degrees and the larger of its scratch and its prefix
+constexpr int kLightRoots = 64 * 8 + 64 * 4 + kLightScratch;
 
 // position of the r-th set bit (0-based) of m; m has more than r bits
 DEV int select64(uint64_t m, int r) {
@@ -741,14 +888,14 @@ __device__ __attribute__((noinline)) PairSum clique_pairs(uint64_t rows_at, uint
         int pc = 0;
         uint32_t by = 0;
 #pragma unroll
-        for (int w0 = 0; w0 < NW; w0++) {
+        for (int w0 = 0; w0 < NW; w0++) {  // a row's bits lie above its own
             uint64_t m = s[w0];
             while (m) {
                 const int x = w0 * 64 + __builtin_ctzll(m);
                 m &= m - 1;
                 by += dp[x];
 #pragma unroll
-                for (int w = 0; w < NW; w++) pc += __popcll(s[w] & rows[x * NW + w]);
+                for (int w = w0; w < NW; w++) pc += __popcll(s[w] & rows[x * NW + w]);
             }
         }
         r.by += by;
@@ -858,6 +1005,14 @@ __device__ __attribute__((noinline)) PairSum clique_pairs(uint64_t rows_at, uint
     }
     return r;
 }
+// A job's head, in registers; its prefix ids go to the worker's LDS record (jid).
+struct JobHead {
+    int lvl, lo, hi, q;
+    int range_end;  // > 0: a static range job over roots [jid[0], range_end)
+    bool donated;
+    bool shared;    // one of hi jobs that claim the root's children from its shared cursor
+};
+
 // Shared by the workers of a block.
 struct BlockLDS {
     int32_t busy;      // workers that have a job or static jobs left
@@ -1419,7 +1574,7 @@ struct Worker {
     // ---- clique, local bitmap of the root's out-neighbourhood -------------
     template <int NW>
     DEV void clique_bitmap_root(int32_t v, int lvl, int lo, int hi, bool first_piece, bool shared) {
-        const int d = odeg(v);
+        const int d = uni<W>(odeg(v));
         const int32_t *L = onbr(v);
         Lvl &R = ws.lv()[0];
         R.uid = const_cast<int32_t *>(L);
@@ -1440,7 +1595,7 @@ struct Worker {
         // pair-phase data first, so that it gets the LDS
         uint64_t *rows = (uint64_t *)alloc((int64_t)d * NW * 8);
         int32_t *dp = (int32_t *)alloc((int64_t)d * 4);
-        int32_t *pre = (int32_t *)alloc((int64_t)(d + 1) * 4);
+        int32_t *pre = nullptr;
         if (abort) return;
         // a root whose bitmap the launch prebuilt (a heavy root cut into
         // many pieces): copy its rows instead of building them
@@ -1463,16 +1618,20 @@ struct Worker {
         } else if (shared) {
             fail(3);  // the host gives a shared cursor only to prebuilt roots
             return;
-        } else {
+        } else if (!stream_rows<NW>(v, lo, d, rows, dp)) {
+            pre = (int32_t *)alloc((int64_t)(d + 1) * 4);
+            if (abort) return;
             build_rows<NW>(v, lo, d, L, rows, dp, pre);
             if (abort) return;
         }
+        if (!pre) pre = (int32_t *)alloc((int64_t)(d + 1) * 4);
+        if (abort) return;
         // K >= 6: the stages, allocated after the build so that the build's
         // hash gets the LDS first; as wide as the LDS left allows
         int sw = W;
         char *st = nullptr, *cu = nullptr;
+        if (NW > 1 && K >= 6 && lds_top + kChildBytes <= lds_lo + p.lds_per_worker) cu = alloc(kChildBytes);
         if (K >= 6) {
-            if (NW > 1 && lds_top + kChildBytes <= lds_lo + p.lds_per_worker) cu = alloc(kChildBytes);
             while (sw > 8 && lds_top + (K - 5) * stage_bytes(sw, NW) > lds_lo + p.lds_per_worker) sw >>= 1;
             st = alloc((int64_t)(K - 5) * stage_bytes(sw, NW));
             if (abort) return;
@@ -1509,6 +1668,63 @@ struct Worker {
         }
         lds_top = R.mark_lds;
         g_top = R.mark_glb;
+    }
+
+    // Rows lo..d-1 of root v's bitmap by root_rows / light_rows; false when
+    // they or the scratch are not in LDS
+    template <int NW>
+    DEV bool stream_rows(int32_t v, int lo, int d, uint64_t *rows, int32_t *dp) {
+        char *const at = lds_top;
+        if ((char *)rows < lds_lo || (char *)rows >= at || (char *)dp < lds_lo || (char *)dp >= at) return false;
+        char *const end = lds_lo + p.lds_per_worker;
+        if (d <= W) {
+            if (at + kLightScratch > end) return false;
+            light_rows<W>(p.off, p.adj, p.ostart, lds_at(at), lds_at(rows), lds_at(dp), v, g.gl == 0 ? d : 0, lo);
+            wsync();
+            return true;
+        }
+        if constexpr (NW > 1) {
+            if (at + rows_scratch(NW) > end) return false;
+            const bool ok = root_rows<W, NW>(p.off, p.adj, p.ostart, lds_at(at), lds_at(rows), lds_at(dp), v, lo, d);
+            wsync();
+            return ok;
+        }
+        return false;
+    }
+
+    // Several light roots at once (lane's root v with d children, sum <= W):
+    // one bitmap, enumerated as one root's; pieces of it are not given away.
+    DEV void light_roots(int32_t v, int d) {
+        job_lvl = 2;
+        lds_top = lds_lo;
+        g_top = g_lo;
+        cnt = 0;
+        const int T = uni<W>(g.bcast(g.iscan(d), W - 1));
+        uint64_t *rows = (uint64_t *)alloc(64 * 8);
+        int32_t *dp = (int32_t *)alloc(64 * 4);
+        light_rows<W>(p.off, p.adj, p.ostart, lds_at(lds_top), lds_at(rows), lds_at(dp), v, d, 0);
+        wsync();
+        bytes += 4ull * (unsigned long long)d;
+        if (K == 3) {
+            if (g.gl < T) {
+                cnt += (unsigned long long)__popcll(rows[g.gl]);
+                bytes += 4ull * (unsigned long long)dp[g.gl];
+            }
+            return;
+        }
+        int32_t *pre = (int32_t *)alloc((int64_t)(T + 1) * 4);
+        int sw = W;
+        char *st = nullptr;
+        if (K >= 6) {
+            while (sw > 8 && lds_top + (K - 5) * stage_bytes(sw, 1) > lds_lo + p.lds_per_worker) sw >>= 1;
+            st = alloc((int64_t)(K - 5) * stage_bytes(sw, 1));
+        }
+        if (abort) return;
+        Lvl &R = ws.lv()[0];
+        R.uid = (int32_t *)dp;  // ids are only read for jobs given away
+        R.nu = T;
+        R.vtx = v0;
+        pair_phase<1>(R, rows, dp, pre, st, sw, nullptr, 0, T);
     }
 
     // Rows lo..d-1 of the local bitmap of root v (L = N+(v), d = |L|): row i
@@ -1734,6 +1950,43 @@ struct Worker {
     // root node's own bytes are counted once, by that job); shared: one of
     // `hi` jobs on a prebuilt bitmap root that claim its children from the
     // root's shared cursor
+    // Light roots that can be run together from `root` on (each with at most
+    // half the lanes' children, a quarter at k >= 7, where one lane's share of a
+    // dense one could outlast the launch): of a range job, then
+    // of the worker's own queue.  False when there is only one; else lane's
+    // root v with d children (d = 0 past the last), the job's root and the
+    // queue moved on to the last of them, `merged` the queue's jobs taken.
+    DEV bool collect_light(const JobHead &jh, int &root, int &merged, int32_t &v, int &d) {
+        const int most = K <= 6 ? W / 2 : W / 4;
+        if (K < 3 || (K > 3 && !p.bitmap) || p.root_cost || p.root_count || p.lds_per_worker < kLightRoots) return false;
+        if (jh.lvl || jh.shared || jh.donated || (!jh.range_end && (jh.lo != 0 || jh.hi != 0x7fffffff))) return false;
+        if (odeg(root) > most) return false;
+        const int m = range_hi - root;
+        // a queue shared by a group: light roots are claimed many at a time
+        if (m == 1 && own_cur >= own_end && own_queue >= 0) claim_shared(W / 8);
+        v = root + g.gl;
+        bool ok = g.gl < m;
+        if (!ok && own_cur + g.gl - m < own_end) {
+            int32_t t[4];
+            static_record(own_base, own_cur + g.gl - m, t);
+            v = t[0];
+            ok = t[3] == jh.q && (t[1] == -1 ? t[2] == v + 1 : t[1] == 0 && t[2] == 0x7fffffff);
+        }
+        d = ok ? odeg(v) : W + 1;
+        const bool light = d <= most;
+        const int sc = g.iscan(light ? d : W + 1);
+        const uint64_t no = g.ballot(!light || sc > W);
+        const int n = no ? __builtin_ctzll(no) : W;
+        if (n < 2) return false;
+        if (g.gl >= n) d = 0;
+        root += (n < m ? n : m) - 1;
+        const int taken = n > m ? n - m : 0;
+        own_cur += taken;
+        merged += taken;
+        v0 = root;
+        return true;
+    }
+
     DEV void run_job(int lvl, int lo, int hi, bool first_piece, bool shared) {
         v0 = uni<W>(ws.jid()[0]);
         job_lvl = lvl;
@@ -1845,14 +2098,7 @@ struct Worker {
 };
 
 // ---------------------------------------------------------------------------
-// work acquisition.  A job head comes back in registers; its prefix ids go to
-// the worker's LDS record (jid).
-struct JobHead {
-    int lvl, lo, hi, q;
-    int range_end;  // > 0: a static range job over roots [jid[0], range_end)
-    bool donated;
-    bool shared;    // one of hi jobs that claim the root's children from its shared cursor
-};
+// work acquisition
 
 // static queues: one per q_group workers (one per worker when q_group <= 1)
 DEV int num_queues(const EnumParams &p) {
@@ -2195,6 +2441,7 @@ __global__ __launch_bounds__(kThreads, WAVES) void enum_kernel(EnumParams p) {
             backoff = 1;
             const int jq = job_query(jh.q);
             bool ok = jh.q >= 0 && jq < p.nq;
+            int merged = 0;  // further jobs done with this one
             // the job's own donation threshold travels with its query word
             // to every piece it gives away
             wk.qword = jh.q;
@@ -2228,13 +2475,20 @@ __global__ __launch_bounds__(kThreads, WAVES) void enum_kernel(EnumParams p) {
                         ws.jid()[0] = root;
                         wsync();
                     }
+                    int32_t lv = 0;
+                    int ld = 0;
+                    bool light = false;
+                    if constexpr (MODE == 0) {
+                        light = wk.collect_light(jh, root, merged, lv, ld);
+                    }
                     // the job's start time goes through LDS: nothing of the
                     // bookkeeping stays live in registers across the DFS
                     if (g.gl == 0) {
                         if (!ws.st()[kStFirst]) ws.st()[kStFirst] = wall_clock64();
                         ws.st()[kStT0] = __builtin_amdgcn_s_memtime();
                     }
-                    wk.run_job(jh.lvl, jh.lo, jh.hi,
+                    if (light) wk.light_roots(lv, ld);
+                    else wk.run_job(jh.lvl, jh.lo, jh.hi,
                                !jh.shared && (jh.range_end > 0 || (!jh.donated && jh.lvl == 0 && jh.lo == 0)),
                                jh.shared);
                     unsigned long long jc = g.lsum(wk.cnt);
@@ -2250,8 +2504,8 @@ __global__ __launch_bounds__(kThreads, WAVES) void enum_kernel(EnumParams p) {
                 }
             }
             if (g.gl == 0) {
-                ws.st()[kStJobs]++;
-                atomicAdd(&blk->pending, 1u);
+                ws.st()[kStJobs] += 1 + merged;
+                atomicAdd(&blk->pending, 1u + (unsigned)merged);
             }
             if (wk.abort) break;
         }
