@@ -161,6 +161,8 @@ using glb_u8 = const __attribute__((address_space(1))) uint8_t;
 using glb_u16 = const __attribute__((address_space(1))) uint16_t;
 using glb_u32 = __attribute__((address_space(1))) uint32_t;
 using glb_u64 = __attribute__((address_space(1))) uint64_t;
+// waits until the wave's memory operations have been performed
+DEV void stores_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 // The atomic that returned x has been performed before any access that
 // follows in the program (its result is waited for here).
 template <class T>
@@ -826,6 +828,49 @@ __device__ __attribute__((noinline)) void light_rows(const int64_t *off_, const 
     });
 }
 
+// A root's rows [lo, d) and out-degrees to (publish) or from (fetch) a buffer
+// that workers of other compute units read: device-scope words, several loads
+// in flight.  Rows of nw words at rows_at, out-degrees at dp_at, both in LDS.
+template <int W, bool OUT>
+__device__ __attribute__((noinline)) void copy_rows(uint64_t *buf_, uint32_t rows_at, uint32_t dp_at, int nw, int lo,
+                                                    int d) {
+    using glb_w64 = __attribute__((address_space(1))) uint64_t;
+    glb_w64 *const buf = (glb_w64 *)unil<W>((uint64_t)buf_);
+    lds_u64 *const rows = (lds_u64 *)(uintptr_t)(uint32_t)uni<W>((int)rows_at);
+    lds_u32 *const dp = (lds_u32 *)(uintptr_t)(uint32_t)uni<W>((int)dp_at);
+    nw = uni<W>(nw), lo = uni<W>(lo), d = uni<W>(d);
+    const Grp<W> g;
+    const int n = d * nw;
+    // words [0, n): rows; then two out-degrees a word
+    const int end = n + (d + 1) / 2;
+    if constexpr (OUT) {
+        for (int t = lo * nw + g.gl; t < end; t += W) {
+            const int i = 2 * (t - n);
+            const uint64_t x = t < n ? rows[t] : (uint64_t)dp[i] | (i + 1 < d ? (uint64_t)dp[i + 1] << 32 : 0);
+            __hip_atomic_store(buf + t, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        stores_done();
+    } else {
+        for (int t0 = lo * nw; t0 < end; t0 += 4 * W) {
+            uint64_t x[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const int t = t0 + u * W + g.gl;
+                x[u] = __hip_atomic_load(buf + (t < end ? t : end - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const int t = t0 + u * W + g.gl, i = 2 * (t - n);
+                if (t < n) rows[t] = x[u];
+                else if (t < end) {
+                    dp[i] = (uint32_t)x[u];
+                    if (i + 1 < d) dp[i + 1] = (uint32_t)(x[u] >> 32);
+                }
+            }
+        }
+    }
+}
+
 // bytes of one stage of sw sets: sets u64[sw * NW] | prefix u32[sw + 1], size,
 // cursor
 __host__ __device__ constexpr int stage_bytes(int sw, int NW) { return sw * NW * 8 + ((sw + 4) & ~1) * 4; }
@@ -1043,7 +1088,11 @@ struct Worker {
     int range_hi;  // end of the current range job's roots (v0 + 1 otherwise)
     uint64_t t_start;
     uint64_t last_poll;  // wall clock of the last request check
-    int poll_shift;      // the check period doubles while nobody asks
+    int poll_shift;      // the check period doubles when nobody asked
+    int pub;          // words a row | lo << 4 | d << 16 of the running bitmap root
+                      // (0: its rows cannot be published)
+    uint32_t pub_no;  // publications so far << 1 | this root's rows are published
+    int from;         // worker + 1 that published a job's rows (0: nobody)
     BlockLDS *blk;
     // static queue: jobs [own_cur, own_end) of queue records own_base.. are
     // this worker's; a queue shared by a group still has to be claimed
@@ -1069,6 +1118,54 @@ struct Worker {
         t_start = now_ticks();
         last_poll = t_start;
         poll_shift = 0;
+        pub = from = 0;
+        pub_no = 0;
+    }
+    // The word that says which of a worker's publications its arena holds.
+    DEV unsigned long long *pub_word(int w) const {
+        const int wpb = (int)blockDim.x / W;
+        return mailbox(w / wpb) + kMailPub + w % wpb;
+    }
+    DEV unsigned long long pub_tag(uint32_t no) const { return ((unsigned long long)epoch << 32) | no; }
+    DEV int me() const { return (int)blockIdx.x * ((int)blockDim.x / W) + uni<W>((int)threadIdx.x / W); }
+    DEV void set_pub_word(unsigned long long tag) {
+        if (g.gl == 0) __hip_atomic_store(pub_word(me()), tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        stores_done();
+    }
+    // Out-degrees follow a root's rows, which are first in the worker's slice.
+    DEV char *dp_of(int nw, int d) const { return lds_lo + ((d * nw * 8 + 15) & ~15); }
+    // The running root's rows to the start of this worker's arena, which holds
+    // nothing else while they are in LDS.  A job on some of the root's children
+    // then starts with a copy (3-8 KB, one round of loads) instead of building
+    // the rows again, which took longer than most pieces: 5-cliques of R-MAT
+    // s17 of edge factor 8 0.79 -> 0.73 ms, 6-cliques (plain queues) 3.14 -> 2.79,
+    // 7-cliques of s13 0.97 -> 0.77.  The word says which root the arena holds:
+    // it is taken back before the arena is used for anything else, and read
+    // after the copy, so a copy that a later root may have overwritten is known
+    // and the rows are built after all.
+    DEV void publish() {
+        if (!pub || (pub_no & 1)) return;
+        const int nw = pub & 15, lo = pub >> 4 & 0xfff, d = pub >> 16;
+        copy_rows<W, true>((uint64_t *)g_lo, lds_at(lds_lo), lds_at(dp_of(nw, d)), nw, lo, d);
+        pub_no += 3;  // the next number, live
+        set_pub_word(pub_tag(pub_no));
+    }
+    // The arena is about to be used for something else.
+    DEV void unpublish() {
+        pub = 0;
+        if (!(pub_no & 1)) return;
+        pub_no--;
+        set_pub_word(0);
+    }
+    // Rows from where the job's giver published them; false when it has moved on.
+    DEV bool fetch_rows(int nw, int lo, int d) {
+        if (from <= 0 || from > p.nworkers) return false;
+        copy_rows<W, false>((uint64_t *)(p.arena + (int64_t)(from - 1) * p.arena_per_worker), lds_at(lds_lo),
+                            lds_at(dp_of(nw, d)), nw, lo, d);
+        stores_done();
+        unsigned long long tag = 0;
+        if (g.gl == 0) tag = __hip_atomic_load(pub_word(from - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return g.bcast64(tag, 0) == pub_tag((uint32_t)uni<W>(ws.jid()[kJobPub - 3]));
     }
 
     // ---- helpers -----------------------------------------------------------
@@ -1183,7 +1280,7 @@ struct Worker {
             if (rq == kMailIdle) rq = 0, (void)atomicCAS(m, kMailIdle, 0ull);
         }
         const int n = __popcll(g.ballot(rq != 0));
-        poll_shift = n ? 0 : poll_shift < 4 ? poll_shift + 1 : 4;
+        poll_shift = n ? 0 : 1;
         return n;
     }
 
@@ -1306,8 +1403,11 @@ struct Worker {
             if (most < 1) return;
             n = accept(rq, most, true);
             if (n == 0) return;
+            publish();
             answer(rq, [&](int r, int j) {
                 return j == 0   ? l
+                       : j == kJobPub && l <= 1     ? (pub_no & 1 ? me() + 1 : 0)
+                       : j == kJobPub + 1 && l <= 1 ? (int)pub_no
                        : j == 1 ? split_at(l, cur, end, r + 1, n + 1)
                        : j == 2 ? split_at(l, cur, end, r + 2, n + 1)
                        : j == 3 ? qword
@@ -1600,6 +1700,7 @@ struct Worker {
         // a root whose bitmap the launch prebuilt (a heavy root cut into
         // many pieces): copy its rows instead of building them
         int slot = -1;
+        const bool in_lds = (char *)dp >= lds_lo && (char *)dp < lds_top && (char *)rows >= lds_lo && (char *)rows < lds_top;
         if (p.npre > 0) {
             int a = 0, b = p.npre;
             while (a < b) {
@@ -1618,7 +1719,7 @@ struct Worker {
         } else if (shared) {
             fail(3);  // the host gives a shared cursor only to prebuilt roots
             return;
-        } else if (!stream_rows<NW>(v, lo, d, rows, dp)) {
+        } else if (!(in_lds && from && fetch_rows(NW, lo, d)) && !stream_rows<NW>(v, lo, d, rows, dp)) {
             pre = (int32_t *)alloc((int64_t)(d + 1) * 4);
             if (abort) return;
             build_rows<NW>(v, lo, d, L, rows, dp, pre);
@@ -1626,6 +1727,7 @@ struct Worker {
         }
         if (!pre) pre = (int32_t *)alloc((int64_t)(d + 1) * 4);
         if (abort) return;
+        wsync();
         // K >= 6: the stages, allocated after the build so that the build's
         // hash gets the LDS first; as wide as the LDS left allows
         int sw = W;
@@ -1636,6 +1738,9 @@ struct Worker {
             st = alloc((int64_t)(K - 5) * stage_bytes(sw, NW));
             if (abort) return;
         }
+        if (in_lds && slot < 0 && g_top == g_lo && (int)blockDim.x / W <= kMailPubs &&
+            p.arena_per_worker >= (int64_t)d * (NW * 8 + 4) + 8)
+            pub = NW | lo << 4 | d << 16;
         if (lvl) {
             R.cur = R.end = hi;
             pairs_of_child<NW>(R, rows, dp, pre, st, sw, cu, child, p0, p1);
@@ -1696,6 +1801,7 @@ struct Worker {
     // one bitmap, enumerated as one root's; pieces of it are not given away.
     DEV void light_roots(int32_t v, int d) {
         job_lvl = 2;
+        unpublish();
         lds_top = lds_lo;
         g_top = g_lo;
         cnt = 0;
@@ -1989,6 +2095,7 @@ struct Worker {
 
     DEV void run_job(int lvl, int lo, int hi, bool first_piece, bool shared) {
         v0 = uni<W>(ws.jid()[0]);
+        if constexpr (MODE == 0) unpublish();
         job_lvl = lvl;
         lds_top = lds_lo;
         g_top = g_lo;
@@ -2430,7 +2537,7 @@ __global__ __launch_bounds__(kThreads, WAVES) void enum_kernel(EnumParams p) {
                 // stalls the whole wave, including busy narrower workers
                 if (__ballot(1) == ~0ull) {
                     for (int b = 0; b < backoff; b++) __builtin_amdgcn_s_sleep(8);
-                    backoff = backoff < 16 ? backoff * 2 : 16;
+                    backoff = backoff < 4 ? backoff * 2 : 4;
                 }
                 continue;
             }
@@ -2445,6 +2552,7 @@ __global__ __launch_bounds__(kThreads, WAVES) void enum_kernel(EnumParams p) {
             // the job's own donation threshold travels with its query word
             // to every piece it gives away
             wk.qword = jh.q;
+            wk.from = jh.donated && jh.lvl <= 1 && !jh.range_end ? uni<W>(ws.jid()[kJobPub - 4]) : 0;
             wk.job_sm = job_steal_min(jh.q) >= 2 ? job_steal_min(jh.q) : p.steal_min;
             if (ok && jq != wk.qid) {
                 if (!single) flush_query<W>(p, g, wk.qid, ws.st()[kStQCount], whist, ws.st()[kStLast]);

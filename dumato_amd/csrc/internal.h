@@ -73,8 +73,10 @@ struct Rng {
 // ---- device-side structures (identical layout on host and device) ----------
 // A donated job: children [lo, hi) of the node with prefix ids[0..lvl] in
 // query q.  Word j holds (tag << 32 | value): words 0..3 = lvl, lo, hi, q;
-// words 4.. = ids.
+// words 4.. = ids; of a job on a root's children or their pairs, the last two
+// = where the root's rows are published (worker + 1, number; 0: nowhere).
 constexpr int kJobWords = 4 + kJobIds;
+constexpr int kJobPub = kJobWords - 2;
 struct Job {
     uint64_t w[kJobWords];
 };
@@ -121,6 +123,10 @@ constexpr int32_t kNoJob = 0x200;
 constexpr int kMailStride = 16;
 constexpr int kMailSlots = 8;
 constexpr int kMailOver = 8;
+// words kMailPub..: which publication of its root's rows each worker's arena
+// holds (blocks of at most kMailPubs workers)
+constexpr int kMailPub = 9;
+constexpr int kMailPubs = kMailStride - kMailPub;
 constexpr unsigned long long kMailIdle = 0xffffffffull;
 
 // One counting query of a launch.  A single-graph call has one; a batch
