@@ -874,8 +874,9 @@ __device__ __attribute__((noinline)) void copy_rows(uint64_t *buf_, uint32_t row
 // bytes of one stage of sw sets: sets u64[sw * NW] | prefix u32[sw + 1], size,
 // cursor
 __host__ __device__ constexpr int stage_bytes(int sw, int NW) { return sw * NW * 8 + ((sw + 4) & ~1) * 4; }
-// a child's own bitmap: rows u64[64], the set of all its elements, dp i32[64]
-constexpr int kChildBytes = 65 * 8 + 64 * 4;
+// a child's own bitmap: rows u64[64], the set of all its elements, dp i32[64],
+// columns u64[64]
+constexpr int kChildBytes = 65 * 8 + 64 * 4 + 64 * 8;
 // a light batch: rows, out-degrees and the larger of its scratch and its prefix
 constexpr int kLightRoots = 64 * 8 + 64 * 4 + kLightScratch;
 
@@ -932,15 +933,16 @@ __device__ __attribute__((noinline)) PairSum clique_pairs(uint64_t rows_at, uint
     auto edges = [&](const uint64_t (&s)[NW]) {
         int pc = 0;
         uint32_t by = 0;
+        // a row's bits lie above its own: half a word at a time, the words from
+        // there on
 #pragma unroll
-        for (int w0 = 0; w0 < NW; w0++) {  // a row's bits lie above its own
-            uint64_t m = s[w0];
-            while (m) {
-                const int x = w0 * 64 + __builtin_ctzll(m);
-                m &= m - 1;
+        for (int h = 0; h < 2 * NW; h++) {
+            for (uint32_t m = (uint32_t)(s[h >> 1] >> (h & 1) * 32); m; m &= m - 1) {
+                const int x = h * 32 + __builtin_ctz(m);
                 by += dp[x];
+                const P32 row = (P32)(rows + x * NW);
 #pragma unroll
-                for (int w = w0; w < NW; w++) pc += __popcll(s[w] & rows[x * NW + w]);
+                for (int w = h; w < 2 * NW; w++) pc += __popc((uint32_t)(s[w >> 1] >> (w & 1) * 32) & row[w]);
             }
         }
         r.by += by;
@@ -1050,6 +1052,64 @@ __device__ __attribute__((noinline)) PairSum clique_pairs(uint64_t rows_at, uint
     }
     return r;
 }
+// k = 6 below a child with a bitmap of its own: its elements [cur, cur + P) as
+// the third vertex x; the second, j, runs over x's predecessors (col), the
+// fourth and fifth are counted in the common successors.  Taken by x, not by j,
+// lanes side by side have sets of like size: by j they fall from |N(j)| to
+// nothing along one j's elements.  VALU-bound in the inner loop, 13 instructions
+// a bit of the lower half and 9 of the upper.  (6-cliques of R-MAT s17 of edge
+// factor 8, learned queues: 2.23 ms by j, 2.02 by x, 1.93 with the halves
+// apart.)  pp: u32[65].
+template <int W>
+__device__ __attribute__((noinline)) PairSum child_quads(uint32_t rows_at, uint32_t cols_at, uint32_t dp_at,
+                                                         uint32_t pp_at, int cur, int P) {
+    lds_u64 *const rows = (lds_u64 *)(uintptr_t)(uint32_t)uni<W>((int)rows_at);
+    lds_u64 *const cols = (lds_u64 *)(uintptr_t)(uint32_t)uni<W>((int)cols_at);
+    lds_u32 *const dp = (lds_u32 *)(uintptr_t)(uint32_t)uni<W>((int)dp_at);
+    lds_u32 *const pp = (lds_u32 *)(uintptr_t)(uint32_t)uni<W>((int)pp_at);
+    cur = uni<W>(cur), P = uni<W>(P);
+    const Grp<W> g;
+    PairSum r{0, 0};
+    int n = 0;
+    if (g.gl < P) {
+        const int x = cur + g.gl, d = (int)dp[x];
+        const int p = __popcll(cols[x]);
+        r.by += (unsigned long long)d * (unsigned)(p + 1);
+        n = rows[x] ? p : 0;
+    }
+    const int sc = g.iscan(n);
+    const int T = g.bcast(sc, W - 1);
+    pp[g.gl] = (uint32_t)(sc - n);
+    if (g.gl == 0) pp[W] = (uint32_t)T;
+    lsync();
+    int pa = 0;
+    for (int u = g.gl; u < T; u += W) {
+        while ((int)pp[pa + 1] <= u) pa++;
+        const int x = cur + pa;
+        const int j = select64(cols[x], u - (int)pp[pa]);
+        const uint64_t s = rows[x] & rows[j];
+        uint32_t by = 0, pc = 0;
+        // a row's bits lie above its own: the upper half needs its upper words only
+        const uint32_t s0 = (uint32_t)s, s1 = (uint32_t)(s >> 32);
+        for (uint32_t m = s0; m; m &= m - 1) {
+            const int y = __builtin_ctz(m);
+            const uint64_t row = rows[y];
+            by += dp[y];
+            pc += (uint32_t)__popc(s0 & (uint32_t)row) + (uint32_t)__popc(s1 & (uint32_t)(row >> 32));
+        }
+        const lds_u32 *const up = (lds_u32 *)(rows + 32) + 1;
+        for (uint32_t m = s1; m; m &= m - 1) {
+            const int y = __builtin_ctz(m);
+            by += dp[32 + y];
+            pc += (uint32_t)__popc(s1 & up[2 * y]);
+        }
+        r.cnt += pc;
+        r.by += by;
+    }
+    lsync();
+    return r;
+}
+
 // A job's head, in registers; its prefix ids go to the worker's LDS record (jid).
 struct JobHead {
     int lvl, lo, hi, q;
@@ -1952,16 +2012,20 @@ struct Worker {
         // takes 21 instructions a bit instead of 44, and almost all of k = 6's
         // bits lie under such children of wide roots: R-MAT s17 of edge factor
         // 8, 2.97 -> 2.45 ms.  Below `alone` pairs a child is better off in a
-        // batch of several: 16 / 24 / 40 measured 2.54 / 2.45 / 2.79 ms.)
+        // batch of several: 16 / 24 / 40 measured 2.54 / 2.45 / 2.79 ms, and
+        // with child_quads 16 / 24 / 32 2.11 / 2.04 / 2.04.)  At k = 6 a full
+        // wave then takes child_quads, whose order keeps its lanes level.
         const bool own = NW > 1 && cu && n <= 64;
         uint64_t *const crow = (uint64_t *)cu;
         int32_t *const cdp = (int32_t *)(crow + 65);
+        uint64_t *const ccol = (uint64_t *)(cdp + 64);
+        const bool quads = W == 64 && K == 6 && own && st >= lds_lo && st < lds_lo + p.lds_per_worker;
         int sw1 = sw;
         if (own) {
             while (sw1 < W && stage_bytes(2 * sw1, 1) <= stage_bytes(sw, NW)) sw1 *= 2;
             for (int x = g.gl; x < n; x += W) {
                 const int at = set_select<NW>(rows + i * NW, x);
-                uint64_t out = 0;
+                uint64_t out = 0, col = 0;
                 int e = 0;
 #pragma unroll
                 for (int w = 0; w < NW; w++) {
@@ -1970,10 +2034,16 @@ struct Worker {
                     while (m) {
                         const int b = __builtin_ctzll(m);
                         m &= m - 1;
-                        out |= ((in >> b) & 1) << e;
+                        const uint64_t bit = (in >> b) & 1;
+                        out |= bit << e;
+                        if constexpr (W == 64) {
+                            const uint64_t pred = __ballot(bit != 0);
+                            if (e == g.gl) col = pred;
+                        }
                         e++;
                     }
                 }
+                ccol[x] = col;
                 crow[x] = out;
                 cdp[x] = dp[at];
             }
@@ -1988,7 +2058,8 @@ struct Worker {
             C.cur = cur + P;
             if (g.gl == 0) pre[0] = -cur, pre[1] = P;
             wsync();
-            const PairSum r = own ? pairs<1>(crow, cdp, pre, st, sw1, 64, P) : pairs<NW>(rows, dp, pre, st, sw, i, P);
+            const PairSum r = quads ? child_quads<W>(lds_at(crow), lds_at(ccol), lds_at(cdp), lds_at(st), cur, P)
+                              : own ? pairs<1>(crow, cdp, pre, st, sw1, 64, P) : pairs<NW>(rows, dp, pre, st, sw, i, P);
             cnt += r.cnt;
             bytes += 4ull * r.by;
             wsync();
