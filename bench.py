@@ -30,10 +30,9 @@ times (a cached partition's gain on repeated queries).
 roofline: the resource that bounds the headline kernel.  Its shader counters
 (profiles/counters.json, from the rocprofv3 runs summarised in
 profiles/enum_kernel_motif4_chunglu18k.md) show VALU issue as the most used
-unit (latency-bound otherwise: waves wait about two thirds of their cycles),
+unit (waves wait half of their cycles),
 so achieved = VALU wave-instructions per launch (profile) / kernel time (HIP
-events on the library's stream, this run; frac_enumeration leaves out the idle
-workers' steal loop, 9% of the count), against the MI355X issue peak of
+events on the library's stream, this run), against the MI355X issue peak of
 256 CUs x 4 SIMDs x 2.4 GHz / 4 cycles per wave64 instruction.  Beside it:
 traffic = HBM bytes per launch (rocprofv3 FETCH_SIZE + WRITE_SIZE, calibrated
 on a copy of known size) and the algorithmic bytes of the enumeration
@@ -325,8 +324,8 @@ def roofline(st, kern_ms, total):
     t = kern_ms / 1e3
     achieved = valu / t / 1e9 if valu else None
     alg = st["alg_bytes"]
-    # frac counts every VALU instruction issued, the idle workers' steal
-    # loop included; frac_enumeration leaves that loop's share out
+    # frac counts every VALU instruction issued; frac_enumeration leaves out
+    # the idle workers' loop where the profile has its share
     return {"bound": "valu", "achieved": achieved, "peak": VALU_PEAK_GINST, "unit": "Ginst/s",
             "frac": achieved / VALU_PEAK_GINST if achieved else None, "traffic": traffic,
             "frac_enumeration": (valu - steal) / t / 1e9 / VALU_PEAK_GINST if valu else None,

@@ -6,7 +6,7 @@
 // degree rank inside its own id range, so cliques and motifs never cross
 // graphs); every (graph, pattern, k) query gets a descriptor with its class
 // table and result slots, and static range jobs over its graph's roots.  The
-// kernel switches query per job; donation and counting are the single-graph
+// kernel switches query per job; sharing and counting are the single-graph
 // kernel's.
 #include <hip/hip_runtime_api.h>
 

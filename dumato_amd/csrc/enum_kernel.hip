@@ -31,7 +31,7 @@
 //     (motif_leaf); everything else is counted in closed form.
 //   * Work: static per-worker queues of (root, lo, hi) jobs.  A worker that
 //     runs out asks a random block through the block's mailbox; a busy worker
-//     there answers with half of its static jobs, or half of the remaining
+//     there answers with a share of its static jobs, or of the remaining
 //     children of its job's lowest level (the reference's donate(),
 //     src/main/DuMatoCPU.cu:463-539, done on the device instead of by the host).
 #include <hip/hip_runtime.h>
@@ -49,13 +49,12 @@ namespace dm {
 // Largest block (4 waves); a launch may use 1, 2 or 4 waves per block.
 constexpr int kThreads = 256;
 // Waves per SIMD each instantiation is compiled for: 3 (168 VGPRs) for the
-// clique and mixed kernels, 4 (128 VGPRs) for the full-wave motif kernel.
-// Motif sizes k >= 5 get a second full-wave motif kernel at 6 waves (80
-// VGPRs, more of them spilled): their deeper searches wait on more loads, and
-// the extra waves hide them (Barabasi-Albert k = 5: 5.16 s at 4 waves, 4.73 s
-// at 5, 4.53 s at 6, 4.54 s at 7, 5.52 s at 8), while k = 4 is faster at 4
-// (Chung-Lu 18K: 4.66 ms at 4, 4.96 ms at 5).  The clique kernel is slower
-// at 4 than at 3 (R-MAT k = 5: 1.42 -> 1.66 ms).
+// clique kernel, whose bitmap roots need the LDS of three blocks a CU, 4 (128
+// VGPRs) for the full-wave motif kernel.  Motif sizes k >= 5 get a second
+// full-wave motif kernel at 6 waves (80 VGPRs; what is spilled belongs to the
+// levels above the leaf, whose own registers fit).  k = 4 has larger tables,
+// which 4 waves leave room for: at 5 / 6 waves Chung-Lu 18K 1.225 -> 1.193 /
+// 1.199 ms, Barabasi-Albert 100K 4.82 -> 5.19 / 5.20.
 template <int W, int MODE>
 constexpr int min_waves() { return W == 64 && MODE == 1 ? 4 : 3; }
 constexpr int kDeepMotifWaves = 6;
@@ -252,8 +251,8 @@ DEV WorkerLDS worker_lds(char *base, int K) {
 // fewer (over the leaf nodes of Chung-Lu 18K k = 4: 305 M against 1,116 M;
 // Barabasi-Albert 100K k = 4: 678 M against 3,557 M).  Calls against the
 // leaf that streamed every child's N(c): Chung-Lu 18K k = 4 4.76 -> 2.12 ms,
-// Barabasi-Albert 100K k = 4 16.5 -> 5.9 ms, 12K k = 5 167 -> 43 ms, before the
-// steps described below.
+// Barabasi-Albert 100K k = 4 16.5 -> 5.9 ms, 12K k = 5 167 -> 43 ms; with the
+// steps described at their places now 1.25, 4.79 and 34 ms.
 //
 // U is held in a hash table for these tests: buckets of two 32-bit slots, two
 // buckets per element, so a test is two 8-byte LDS reads and no loop.  With h =

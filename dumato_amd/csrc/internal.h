@@ -71,7 +71,7 @@ struct Rng {
 };
 
 // ---- device-side structures (identical layout on host and device) ----------
-// A donated job: children [lo, hi) of the node with prefix ids[0..lvl] in
+// A job given away: children [lo, hi) of the node with prefix ids[0..lvl] in
 // query q.  Word j holds (tag << 32 | value): words 0..3 = lvl, lo, hi, q;
 // words 4.. = ids; of a job on a root's children or their pairs, the last two
 // = where the root's rows are published (worker + 1, number; 0: nowhere).

@@ -5,10 +5,10 @@
 // stream capture, serving loops, harnesses that forbid hipMalloc).  Every
 // device buffer the enumeration kernel needs beyond the graph (its input) and
 // the result (its output) -- scheduler counters, launch epoch, query
-// descriptor, result slots, class table, static-queue cursors, donated-job
-// queue and the per-worker stack arenas -- is carved from one file-scope
-// device array of kScratchBytes.  Static work uses the kernel's strided
-// partition (root r goes to worker (n-1-r) mod workers, highest degree rank
+// descriptor, result slots, class table, static-queue cursors, the workers'
+// job slots, the blocks' mailboxes and the per-worker stack arenas -- is carved
+// from one file-scope device array of kScratchBytes.  Static work uses the
+// kernel's strided partition (root r goes to worker (n-1-r) mod workers, highest degree rank
 // first), which needs no job arrays.  The number of workers is capped so that
 // their arenas fit; a graph whose arena does not fit one block is rejected.
 //
