@@ -2041,7 +2041,10 @@ struct Worker {
         uint64_t *const crow = (uint64_t *)cu;
         int32_t *const cdp = (int32_t *)(crow + 65);
         uint64_t *const ccol = (uint64_t *)(cdp + 64);
-        const bool quads = W == 64 && K == 6 && own && st >= lds_lo && st < lds_lo + p.lds_per_worker;
+        // (the quads' prefix takes the stage's place, which a narrow one is too
+        // small for)
+        const bool quads = W == 64 && K == 6 && own && st >= lds_lo && st < lds_lo + p.lds_per_worker &&
+                           stage_bytes(sw, NW) >= 4 * (W + 1);
         int sw1 = sw;
         if (own) {
             while (sw1 < W && stage_bytes(2 * sw1, 1) <= stage_bytes(sw, NW)) sw1 *= 2;

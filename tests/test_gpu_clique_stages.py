@@ -76,3 +76,18 @@ def test_pairs_of_a_child_given_away(n, p):
             for _ in range(2):
                 assert g.clique_count(k, cfg) == want
                 assert g.last_stats()["alg_bytes"] == by
+
+
+@pytest.mark.parametrize("n,p", [(70, 0.75), (115, 0.6), (150, 0.45)])
+def test_narrow_stages_beside_a_childs_bitmap(n, p):
+    # slices where a child's own bitmap fits LDS but its stages are narrowed,
+    # down to those too small for the prefix of k = 6's last step
+    s, d, nv = G.gnp(n, p, 500 + n)
+    ref = O.csr_from_edges(s, d, nv)
+    _, ro = O.relabel(ref, oriented=True)
+    want, by = O.clique_count(ref, 6), O.clique_bytes(ro, 6)
+    g = dm.Graph.from_edges(s, d, nv)
+    for lds in range(1536, 9216, 192):
+        print("case gnp n=%d clique k=6 lds=%d" % (n, lds), flush=True)
+        assert g.clique_count(6, dm.config(vwave=64, lds_bytes=lds, watchdog_s=60.0)) == want
+        assert g.last_stats()["alg_bytes"] == by
