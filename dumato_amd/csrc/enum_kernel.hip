@@ -1814,7 +1814,7 @@ struct Worker {
         // hash gets the LDS first; as wide as the LDS left allows
         int sw = W;
         char *st = nullptr, *cu = nullptr;
-        if (NW > 1 && K >= 6 && lds_top + kChildBytes <= lds_lo + p.lds_per_worker) cu = alloc(kChildBytes);
+        if ((K == 6 || (K > 6 && NW > 1)) && lds_top + kChildBytes <= lds_lo + p.lds_per_worker) cu = alloc(kChildBytes);
         if (K >= 6) {
             while (sw > 8 && lds_top + (K - 5) * stage_bytes(sw, NW) > lds_lo + p.lds_per_worker) sw >>= 1;
             st = alloc((int64_t)(K - 5) * stage_bytes(sw, NW));
@@ -2036,8 +2036,10 @@ struct Worker {
         // 8, 2.97 -> 2.45 ms.  Below `alone` pairs a child is better off in a
         // batch of several: 16 / 24 / 40 measured 2.54 / 2.45 / 2.79 ms, and
         // with child_quads 16 / 24 / 32 2.11 / 2.04 / 2.04.)  At k = 6 a full
-        // wave then takes child_quads, whose order keeps its lanes level.
-        const bool own = NW > 1 && cu && n <= 64;
+        // wave then takes child_quads, whose order keeps its lanes level; for
+        // that a one-word root's children get bitmaps too (6-cliques of R-MAT
+        // s14 0.41 -> 0.34 ms, s13 0.27 -> 0.22; from 32 pairs on 0.35 and 0.23).
+        const bool own = cu && n <= 64;
         uint64_t *const crow = (uint64_t *)cu;
         int32_t *const cdp = (int32_t *)(crow + 65);
         uint64_t *const ccol = (uint64_t *)(cdp + 64);
@@ -2109,7 +2111,7 @@ struct Worker {
             }
             front = g.bcast(front, 0);
             maybe_donate(1, front >= heavy ? 2 : 0);
-            if (front >= (NW > 1 && cu ? alone : 2 * heavy) && R.cur < R.end) {
+            if (front >= (cu ? alone : 2 * heavy) && R.cur < R.end) {
                 const int i = R.cur;
                 R.cur = i + 1;
                 if (g.gl == 0) by += (unsigned long long)dp[i];
