@@ -812,7 +812,7 @@ __device__ __attribute__((noinline)) void light_rows(const int64_t *off_, const 
     if (d > 0) span[sc - d] = (uint32_t)g.gl + 1;
     lsync();
     const uint64_t first = g.ballot(span[g.gl] != 0), upto = (2ull << g.gl) - 1;
-    const int s = 63 - __builtin_clzll(first & upto | 1);
+    const int s = 63 - __builtin_clzll((first & upto) | 1);
     const int e = first & ~upto ? __builtin_ctzll(first & ~upto) : T;
     const int r = (int)span[s] - 1;
     const int64_t ls = __shfl(d > 0 ? (long long)ostart[v] : 0ll, r < 0 ? 0 : r, W);
@@ -1318,7 +1318,7 @@ struct Worker {
     //
     // A job is published without fences: each of its 16 words is one 64-bit
     // agent-scope atomic store with the request's tag in the high half; the
-    // reader accepts the slot once all 16 tags match.
+    // reader accepts the slot, a refusal too, once all 16 tags match.
 
     // Boundary j (0 <= j <= parts) when the children [cur, end) of level l are
     // cut into `parts` pieces of equal estimated work.  A clique child i of a
@@ -1400,7 +1400,7 @@ struct Worker {
             left &= left - 1;
             uint64_t *const dst = p.q[(uint32_t)q - 1].w;
             for (int j = g.gl; j < kJobWords; j += W)
-                __hip_atomic_store(dst + j, (q & 0xffffffff00000000ull) | (uint32_t)f(r, j), __ATOMIC_RELAXED,
+                __hip_atomic_store(dst + j, slot_word((uint32_t)(q >> 32), f(r, j)), __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_AGENT);
         }
     }
@@ -2408,21 +2408,20 @@ DEV int poll_slot(Worker<W, MODE> &wk, int wid, uint32_t tag, JobHead &jh) {
     const Grp<W> &g = wk.g;
     const uint64_t *src = wk.p.q[wid].w;
     int v[(kJobWords + W - 1) / W];
-    bool mine_ok = true, none = false;
+    bool mine_ok = true;
 #pragma unroll
     for (int r = 0; r < (kJobWords + W - 1) / W; r++) {
         const int j = g.gl + r * W;
         v[r] = 0;
         if (j < kJobWords) {
             uint64_t x = __hip_atomic_load(src + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if ((uint32_t)(x >> 32) != tag) mine_ok = false;
+            if (!slot_word_of(x, tag)) mine_ok = false;
             v[r] = (int32_t)(uint32_t)x;
-            if (j == 0) none = mine_ok && v[r] == kNoJob;
         }
     }
-    if (g.ballot(none) != 0) return 3;
     if (g.ballot(!mine_ok) != 0) return 0;
     const int w0 = g.bcast(v[0], 0), w1 = g.bcast(v[0], 1), w2 = g.bcast(v[0], 2), w3 = g.bcast(v[0], 3);
+    if (w0 == kNoJob) return 3;
     if (w0 == kStaticJobs) {
         wk.own_base = (int64_t)(((uint64_t)(uint32_t)g.bcast(v[0], 5) << 32) | (uint32_t)g.bcast(v[0], 4));
         wk.own_cur = w1;
@@ -2460,9 +2459,12 @@ DEV bool go_idle(const EnumParams &p, const Grp<W> &g, BlockLDS *blk) {
     if (!g.bcast(last, 0)) return false;
     if (g.gl < kMailSlots) {
         const unsigned long long rq = atomicExch(p.mail + (size_t)blockIdx.x * kMailStride + g.gl, kMailIdle);
-        if (rq != 0 && rq != kMailIdle)
-            __hip_atomic_store(p.q[(uint32_t)rq - 1].w, (rq & 0xffffffff00000000ull) | (uint32_t)kNoJob,
-                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (rq != 0 && rq != kMailIdle) {
+            uint64_t *const dst = p.q[(uint32_t)rq - 1].w;
+            for (int j = 0; j < kRefusalWords; j++)
+                __hip_atomic_store(dst + j, slot_word((uint32_t)(rq >> 32), refusal_value(j)), __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+        }
     }
     int end = 0;
     if (g.gl == 0) {
@@ -2572,8 +2574,7 @@ __global__ __launch_bounds__(kThreads, WAVES) void enum_kernel(EnumParams p) {
                         break;
                     }
                 }
-                // request tags: the epoch and a count, never 0
-                const uint32_t tag = (wk.epoch << 8) | (seq % 255u + 1);
+                const uint32_t tag = request_tag(wk.epoch, seq);
                 if (asked >= 0) {
                     const int r = poll_slot(wk, wid, tag, jh);
                     if (r) {
@@ -2888,12 +2889,13 @@ __global__ void fill_u32_kernel(uint32_t *ptr, uint32_t value, size_t count) {
 }
 
 // Resets the scheduler state of a launch; graph-capturable (no memset or
-// host copies).  Bumps the epoch so queue slots of earlier launches never
-// match.
+// host copies).  Clears the job slots, so that nothing an earlier launch left
+// there matches a request, whatever the epoch (16 bytes a thread: 0.8 MB for
+// 6,144 workers).
 __global__ void enum_init_kernel(SchedCounters *sc, unsigned long long njobs, int32_t *epoch, int32_t *sq_cur,
                                  int nworkers, unsigned long long *results, size_t nresults,
                                  unsigned long long *done_ticks, int nq, unsigned long long *start_ticks,
-                                 unsigned long long *mail, int blocks) {
+                                 unsigned long long *mail, int blocks, Job *q, int slots) {
     size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     size_t stride = (size_t)gridDim.x * blockDim.x;
     if (i == 0) {
@@ -2912,6 +2914,7 @@ __global__ void enum_init_kernel(SchedCounters *sc, unsigned long long njobs, in
     for (size_t t = i; t < (size_t)blocks * kMailStride; t += stride)
         mail[t] = t % kMailStride < kMailSlots ? kMailIdle : 0;
     for (size_t t = i; t < (size_t)nworkers; t += stride) sq_cur[t] = 0;
+    for (size_t t = i; t < (size_t)slots * sizeof(Job) / 16; t += stride) ((ulong2 *)q)[t] = ulong2{0, 0};
     for (size_t t = i; t < nresults; t += stride) results[t] = 0;
     if (done_ticks)
         for (size_t t = i; t < (size_t)nq; t += stride) done_ticks[t] = 0;
@@ -2998,10 +3001,12 @@ int enum_launch(const EnumParams &p, int mode, int vwave, int blocks, int thread
 
 int enum_init_launch(const EnumParams &p, unsigned long long njobs, int32_t *epoch, unsigned long long *results,
                      size_t nresults, unsigned long long *done_ticks, int nq, int launch_blocks, void *stream) {
-    size_t work = std::max<size_t>({(size_t)p.nworkers, nresults, (size_t)nq, (size_t)1});
+    const int slots = (int)std::min<int64_t>(p.nworkers, p.q_cap);
+    size_t work = std::max<size_t>({(size_t)slots * sizeof(Job) / 16, (size_t)p.nworkers, nresults, (size_t)nq, (size_t)1});
     int blocks = (int)std::min<size_t>((work + 255) / 256, 1024);
     hipLaunchKernelGGL(enum_init_kernel, dim3(blocks), dim3(256), 0, (hipStream_t)stream, p.sc, njobs, epoch, p.sq_cur,
-                       p.nworkers, results, nresults, done_ticks, nq, p.start_ticks, p.mail, launch_blocks);
+                       p.nworkers, results, nresults, done_ticks, nq, p.start_ticks, p.mail, launch_blocks, p.q,
+                       slots);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return set_error(DM_ERR_HIP, "init launch: %s", hipGetErrorString(e));
     return DM_OK;

@@ -115,8 +115,19 @@ SchedStats sched_totals(const SchedCounters &c);
 // Word 0 of a job in a worker's slot is its level, or kStaticJobs: the records
 // [word 1, word 2) of the static queue that starts at record (or, strided, at
 // worker) word 4 | word 5 << 32; or kNoJob: the request was not taken.
+// Every answer, a refusal too, writes all kJobWords words with the request's
+// tag, and none is taken before all of them carry it.  So one writer at a time
+// has a worker's slot, all its words carry the tag of the request before (none
+// at first: the init kernel clears the slots), and a partly written answer
+// never matches, although tags repeat after 255 requests and 2^24 launches.
 constexpr int32_t kStaticJobs = 0x100;
 constexpr int32_t kNoJob = 0x200;
+// a worker's seq-th request of a launch; never 0, and never the one before's
+constexpr uint32_t request_tag(uint32_t epoch, uint32_t seq) { return (epoch << 8) | (seq % 255u + 1); }
+constexpr uint64_t slot_word(uint32_t tag, int32_t value) { return ((uint64_t)tag << 32) | (uint32_t)value; }
+constexpr bool slot_word_of(uint64_t word, uint32_t tag) { return (uint32_t)(word >> 32) == tag; }
+constexpr int32_t refusal_value(int word) { return word == 0 ? kNoJob : 0; }
+constexpr int kRefusalWords = kJobWords;
 // A block's mailbox, a line: kMailSlots words that hold 0 (open), a request
 // (asking worker + 1, its tag in the high half) or kMailIdle (no worker of the
 // block has work); word kMailOver is the epoch of a launch that is over.
