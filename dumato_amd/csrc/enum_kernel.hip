@@ -522,9 +522,7 @@ __device__ __attribute__((noinline)) LeafSum motif_leaf(const int64_t *off_, con
         tl.mul = 0x9E3779B1u;
         // up to 6/7 full; a failed insertion is rare from there on down
         if ((8 << b) > space || 7 * tot > 6 * (2 << b) || !tl.build(g, puid, pupm, pnu, c, nc, q, newc)) {
-            b = 9;
-            while ((1 << b) < tot + tot / 2) b++;
-            r.big = b;
+            r.big = leaf_table_bits(tot);
             return r;
         }
     } else {

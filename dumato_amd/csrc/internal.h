@@ -240,6 +240,14 @@ constexpr int motif_leaf_fixed(int W, int K) {
     return (W * 8 + kLeafCap / 8 + 32 + (1 << (K - 2)) * 12 +
             (K <= 6 ? leaf_copies(K) * (4 << (2 * (K - 2))) : (1 << (K - 2)) * ((1 << (K - 2)) + 1) * 2) + 15) & ~15;
 }
+// The leaf's table in the arena, where the LDS slice does not hold it: 2^bits
+// slots of 4 B for `tot` elements, between 1/3 and 2/3 full (512 slots at least).
+constexpr int leaf_table_bits(int64_t tot) {
+    int b = 9;
+    while (((int64_t)1 << b) < tot + tot / 2) b++;
+    return b;
+}
+constexpr int64_t leaf_table_bytes(int64_t tot) { return (int64_t)4 << leaf_table_bits(tot); }
 size_t enum_lds_bytes(int vwave, int threads, int kmax, int ncls_single, int hist_slots, int lds_per_worker);
 int enum_occupancy(int vwave, int mode, int threads, size_t lds, int *blocks_per_cu);
 int enum_launch(const EnumParams &p, int mode, int vwave, int blocks, int threads, size_t lds,

@@ -284,12 +284,14 @@ int64_t arena_bound_for(int32_t maxdeg, int32_t max_out_, int K, bool motif) {
     int64_t md = std::max<int64_t>(maxdeg, 1);
     int64_t b = 256;
     if (motif) {
-        // levels 1..K-4: ids and masks of U and E; level K-3: the leaf's table
-        // where LDS does not hold it (at most 9.5 B per element, 2 KB at least)
-        for (int l = 1; l <= K - 3; l++) b += 10 * (int64_t)(l + 1) * md + 64;
-        b += 4 * md + (int64_t)(K - 2) * md + 64;
-        b += 4372;
-        if (K == 3) b = std::max<int64_t>(b, 4096 + 10 * (int64_t)std::max(max_out_, 1));
+        // levels 1..K-4: ids and masks of U and E
+        for (int l = 1; l <= K - 4; l++) b += 10 * (int64_t)(l + 1) * md + 64;
+        // below them the last level's scratch while it is made, then the leaf's
+        // table where LDS does not hold it: of all a root's out-neighbours at
+        // k = 3, of K-2 neighbour lists otherwise
+        int64_t rest = 4 * md + (int64_t)(K - 2) * md + 64 + 4372;
+        if (K > 3) rest += 10 * (int64_t)(K - 2) * md + 64;
+        b += std::max(rest, leaf_table_bytes(K == 3 ? std::max(max_out_, 1) : (int64_t)(K - 2) * md) + 16);
     } else {
         int64_t mo = std::max<int64_t>(max_out_, 1);
         for (int l = 1; l <= K - 3; l++) b += 4 * mo + 16;
