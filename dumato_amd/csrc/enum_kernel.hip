@@ -1639,6 +1639,21 @@ struct Worker {
         bytes += r.bytes;
     }
 
+    // k = 3: the root's children [R.cur, R.end), kMotif3Chunk per donation check
+    // (each chunk builds the root's table again)
+    static constexpr int kMotif3Chunk = 512;
+    DEV void motif3_root() {
+        Lvl &R = ws.lv()[0];
+        while (!abort) {
+            maybe_donate(1);
+            const int cur = uni<W>(R.cur), end = uni<W>(R.end);
+            if (cur >= end) return;
+            const int to = end - cur <= kMotif3Chunk ? end : cur + kMotif3Chunk;
+            R.cur = to;
+            motif_leaf_node(-1, 0, cur, to);
+        }
+    }
+
     // ---- clique levels ----------------------------------------------------------
     DEV void clique_root_level(int32_t v) {
         Lvl &L = ws.lv()[0];
@@ -2256,8 +2271,8 @@ struct Worker {
             if (!motif && K == 3 && triangle_root(L.cur, L.end)) return;
             if (k == K - 3) {
                 // a motif job comes here only at k = 3, whose root is the leaf
-                if (motif) motif_leaf_node(-1, 0, L.cur, L.end);
-                else clique_leaf_phase(k, L.cur, L.end);
+                if (motif) return motif3_root();
+                clique_leaf_phase(k, L.cur, L.end);
                 if (abort) return;
                 lds_top = L.mark_lds;
                 g_top = L.mark_glb;
