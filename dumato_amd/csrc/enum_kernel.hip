@@ -1907,6 +1907,9 @@ struct Worker {
         wsync();
         bytes += 4ull * (unsigned long long)d;
         if (K == 3) {
+            // (larger sizes look in pair_phase)
+            if (check_abort()) return;
+            maybe_donate(0);
             if (g.gl < T) {
                 cnt += (unsigned long long)__popcll(rows[g.gl]);
                 bytes += 4ull * (unsigned long long)dp[g.gl];
