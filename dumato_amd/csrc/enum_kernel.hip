@@ -1613,6 +1613,7 @@ struct Worker {
     }
 
     // ---- motif leaf ------------------------------------------------------------
+    static constexpr int kMotif3Chunk = 512;  // (each builds the root's table again)
     // Leaf node of child i0 of level pl = K-4 (k >= 4), or the root itself at
     // k = 3 (pl = -1) with the elements [lo, hi) of its list as children.
     DEV void motif_leaf_node(int pl, int i0, int lo, int hi) {
@@ -1637,21 +1638,6 @@ struct Worker {
         }
         cnt += r.cnt;
         bytes += r.bytes;
-    }
-
-    // k = 3: the root's children [R.cur, R.end), kMotif3Chunk per donation check
-    // (each chunk builds the root's table again)
-    static constexpr int kMotif3Chunk = 512;
-    DEV void motif3_root() {
-        Lvl &R = ws.lv()[0];
-        while (!abort) {
-            maybe_donate(1);
-            const int cur = uni<W>(R.cur), end = uni<W>(R.end);
-            if (cur >= end) return;
-            const int to = end - cur <= kMotif3Chunk ? end : cur + kMotif3Chunk;
-            R.cur = to;
-            motif_leaf_node(-1, 0, cur, to);
-        }
     }
 
     // ---- clique levels ----------------------------------------------------------
@@ -2272,9 +2258,7 @@ struct Worker {
             if (check_abort()) return;
             Lvl &L = ws.lv()[k];
             if (!motif && K == 3 && triangle_root(L.cur, L.end)) return;
-            if (k == K - 3) {
-                // a motif job comes here only at k = 3, whose root is the leaf
-                if (motif) return motif3_root();
+            if (!motif && k == K - 3) {
                 clique_leaf_phase(k, L.cur, L.end);
                 if (abort) return;
                 lds_top = L.mark_lds;
@@ -2285,12 +2269,18 @@ struct Worker {
             maybe_donate(k + 1);
             const int i = uni<W>(L.cur);
             if (i < uni<W>(L.end)) {
-                L.cur = i + 1;
-                if (motif && k == K - 4) {
-                    motif_leaf_node(k, i, 0, 0x7fffffff);
+                if (motif && k >= K - 4) {
+                    // a child makes a leaf node; at k = 3 the root is one, its
+                    // children taken kMotif3Chunk per donation check
+                    const bool root = K == 3;
+                    const int left = uni<W>(L.end) - i;
+                    const int to = root ? i + (left < kMotif3Chunk ? left : kMotif3Chunk) : i + 1;
+                    L.cur = to;
+                    motif_leaf_node(root ? -1 : k, i, root ? i : 0, root ? to : 0x7fffffff);
                     if (abort) return;
                     continue;
                 }
+                L.cur = i + 1;
                 if (motif) {
                     const int32_t c = uni<W>(L.eid[i]);
                     const int pmc = uni<W>(epm_at(L, i));
