@@ -50,7 +50,7 @@ namespace dm {
 constexpr int kThreads = 256;
 // Waves per SIMD each instantiation is compiled for: 3 (168 VGPRs) for the
 // clique kernel, whose bitmap roots need the LDS of three blocks a CU, 4 (128
-// VGPRs) for the full-wave motif kernel.  Motif sizes k >= 5 get a second
+// VGPRs) for the full-wave motif kernel.  Motif sizes 5 and 6 get a second
 // full-wave motif kernel at 6 waves (80 VGPRs; what is spilled belongs to the
 // levels above the leaf, whose own registers fit).  k = 4 has larger tables,
 // which 4 waves leave room for: at 5 / 6 waves Chung-Lu 18K 1.225 -> 1.193 /
@@ -2936,7 +2936,7 @@ size_t enum_lds_bytes(int vwave, int threads, int kmax, int ncls_single, int his
     return b;
 }
 
-// launch modes: 0 cliques, 1 motifs, 2 motifs of size >= 5 (the
+// launch modes: 0 cliques, 1 motifs, 2 motifs of sizes 5 and 6 (the
 // full-wave motif kernel at kDeepMotifWaves; narrower widths keep mode 1's)
 template <int W>
 static const void *kernel_mode(int mode) {

@@ -227,9 +227,15 @@ constexpr int job_steal_min(int32_t q) { return (q >> kQueryBits) & 0xff; }
 constexpr int32_t make_job_query(int q, int steal_min) { return q | (steal_min << kQueryBits); }
 
 // kernels (enum_kernel.hip)
-// mode: 0 cliques, 1 motifs, 2 motifs of size >= 5 (a motif kernel budgeted
-// for more waves per SIMD)
-inline int launch_mode(bool motif, int K) { return motif ? (K >= 5 ? 2 : 1) : 0; }
+// mode: 0 cliques, 1 motifs, 2 motifs of sizes 5 and 6 (a motif kernel budgeted
+// for more waves per SIMD: 6, 4 in mode 1).  Size 7's class counters and fixed
+// leaf part leave a worker at 6 waves 800 B for the leaf's table, less than the
+// smallest one, so every table was built in memory; at 4 waves it has 4 KB
+// (Barabasi-Albert 600 of 3 edges a vertex, full grid, 48.9 -> 42.2 ms; Chung-Lu
+// 3,000 of 4,000 edges 13.6 -> 11.7, 8,000 of 10,000 28.9 -> 25.5).  Size 6 has a
+// 2 KB table at 6 waves and stays there: Barabasi-Albert 1,500 19.9 ms, 22.4 at 4;
+// Chung-Lu 12,000 8.6, 9.2; light ones the other way round, Chung-Lu 1,000 1.37, 1.12.
+inline int launch_mode(bool motif, int K) { return !motif ? 0 : K == 5 || K == 6 ? 2 : 1; }
 // The motif leaf's LDS without its table, per worker of W lanes: recs u64[W] |
 // bits u64[kLeafCap / 64 + 4] | qs u64[npm] | n u32[npm] | e u32[copies][npm * npm]
 // (k = 7: [npm (npm + 1) / 2]), npm = 2^(K-2) mask values.  A motif launch gives
