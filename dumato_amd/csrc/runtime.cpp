@@ -73,6 +73,7 @@ int graph_finish(dm_graph *g) {
     rc.adj.resize(c.adj.size());
     g->ostart.assign(n, 0);
     int32_t max_out = 0;
+    double squares = 0;
     for (int32_t r = 0; r < n; r++) {
         int32_t v = order[r];
         int64_t b = rc.off[r];
@@ -83,8 +84,10 @@ int graph_finish(dm_graph *g) {
         const int64_t up = std::upper_bound(rc.adj.begin() + b, rc.adj.begin() + b + d, r) - rc.adj.begin();
         g->ostart[r] = up;
         max_out = std::max<int32_t>(max_out, (int32_t)(b + d - up));
+        squares += (double)d * (double)d;
     }
     g->max_out = max_out;
+    g->degree_squares = squares;
     return DM_OK;
 }
 
@@ -243,6 +246,13 @@ static int max_lds_uncached(int vwave, int threads, int mode, int K, int ncls_si
     return lds;
 }
 
+// Estimate of the elements of a motif query's leaf nodes: a prefix vertex is
+// reached by an edge, where the mean degree is that of a neighbour.
+static double leaf_elements(const dm_graph *g, int K) {
+    const double sum = (double)g->rcsr.off[g->rcsr.n];
+    return sum > 0 ? sum * std::pow(g->degree_squares / sum, K - 3) : 0;
+}
+
 int pick_shape(dm_graph *g, int K, bool motif, const dm_config &cfg, Shape &sh) {
     DeviceCtx *c = g->dev->ctx;
     int vw = cfg.vwave;
@@ -267,14 +277,23 @@ int pick_shape(dm_graph *g, int K, bool motif, const dm_config &cfg, Shape &sh) 
     sh.threads = threads;
     sh.lds_per_worker = lds;
     sh.lds_total = lds_total;
-    // No more workers than vertices (2,048 at least: few roots may be heavy):
-    // a worker without a root only adds to the traffic on the scheduler's
-    // words.  (Default shape, 6,144 workers at k >= 5 against this cap: a
-    // 3,301-vertex sparse graph's k = 5 motifs 2.36 -> 1.76 ms; 2,000-vertex
-    // triangles, 3,072 workers, 0.30 -> 0.22 ms.)
+    // No more workers than vertices (2,048 at least, a block per CU at least)
+    // where that leaves a worker little to do: one without a root only adds to
+    // the launch and to the requests.  (Capped, against the full grid: 3,301-vertex
+    // sparse k = 5 motifs 0.44 ms, 0.46; 2,000-vertex random graph, triangles 42 us,
+    // 48, 3-motifs 54 us, 73; 500 vertices, k = 5, 0.39 ms, 0.43.)  A motif query
+    // with work for more takes the full grid: capped, Barabasi-Albert on 600
+    // vertices k = 7 104 ms, 42 uncapped at 4 waves; on 1,500 k = 6 42, 20, k = 5 1.24,
+    // 0.96; complete graph on 200 k = 4 1.18, 1.03.  By estimated elements of leaf
+    // nodes a worker, over 20 graphs and sizes: up to 364 the full grid is 3-11%
+    // slower, at 410 and 484 equal, from 636 on 5-71% faster.  Cliques keep the cap
+    // (2,048 workers of 3,072): between 14% faster and 15% slower than the full
+    // grid on graphs this small.
     const int wpb = threads / vw;
-    const int useful = (std::max(g->rcsr.n, 2048) + wpb - 1) / wpb;
-    sh.blocks = cfg.blocks > 0 ? cfg.blocks : std::min(bpc * c->num_cu, useful);
+    const int full = bpc * c->num_cu;
+    const int useful = std::max((std::max(g->rcsr.n, 2048) + wpb - 1) / wpb, c->num_cu);
+    const bool much = motif && leaf_elements(g, K) >= 500.0 * useful * wpb;
+    sh.blocks = cfg.blocks > 0 ? cfg.blocks : much ? full : std::min(full, useful);
     sh.workers = sh.blocks * wpb;
     return DM_OK;
 }

@@ -100,6 +100,7 @@ struct dm_graph {
     std::vector<int32_t> perm, inv;  // perm[orig] = rank, inv[rank] = orig
     std::vector<int64_t> ostart;     // per rank: index of the first neighbour above it
     int32_t max_out = 0;
+    double degree_squares = 0;       // sum over the vertices
     dm::DeviceGraph *dev = nullptr;
     dm_stats last{};
     std::vector<uint64_t> last_costs, last_counts;  // original ids
