@@ -172,6 +172,11 @@ template <class P, class T>
 DEV void ladd(P *a, T v) {
     (void)__hip_atomic_fetch_add(a, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
 }
+// to LDS words that other waves of the block add to as well
+template <class P, class T>
+DEV void badd(P *a, T v) {
+    (void)__hip_atomic_fetch_add(a, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
 template <class P>
 DEV void lor(P *a, uint64_t v) {
     (void)__hip_atomic_fetch_or(a, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
@@ -627,14 +632,14 @@ __device__ __attribute__((noinline)) LeafSum motif_leaf(const int64_t *off_, con
         const uint64_t pr = root ? rpairs : i == j ? ni * (ni - 1) / 2 : ni * nj;
         if (pr == 0) continue;
         const uint64_t ee = edges(i, j);
-        if (ee) ladd(shist + lut[child(i) + ((uint64_t)(j | npm) << o2)], ee);
-        if (pr != ee) ladd(shist + lut[child(i) + ((uint64_t)j << o2)], pr - ee);
+        if (ee) badd(shist + lut[child(i) + ((uint64_t)(j | npm) << o2)], ee);
+        if (pr != ee) badd(shist + lut[child(i) + ((uint64_t)j << o2)], pr - ee);
         leaves += pr;
     }
     for (int i = 1 + g.gl; i < npm; i += W) {
         uint64_t nw = qs[i];
         for (int j = 0; j < npm; j++) nw -= i == j ? 2 * edges(i, i) : i > j ? edges(i, j) : edges(j, i);
-        if (nw) ladd(shist + lut[child(i) + ((uint64_t)npm << o2)], nw);
+        if (nw) badd(shist + lut[child(i) + ((uint64_t)npm << o2)], nw);
         leaves += nw;
     }
     lsync();
