@@ -476,13 +476,55 @@ DEV void stream_lists(const Grp<W> &g, lds_u64 *recs, lds_u64 *bits, glb_i32 *li
     }
 }
 
+// The edges that a leaf node has counted so far in 32 bits (e at LDS address
+// e_at, all copies) go to the class counters, whose sums wrap at 64 bits like the
+// final ones: its part of the adjacent pairs, taken from the others and from the
+// pairs with a new neighbour.  ind: the prefix's bits of the class table's index.
+// Returns this lane's share of the leaves.
+template <int W>
+DEV unsigned long long leaf_flush(const Grp<W> &g, glb_u16 *lut, lds_u64 *shist, lds_u32 *e, uint64_t ind, int K) {
+    const int npm = 1 << (K - 2), lw = K - 2, o2 = quick_off(K - 1);
+    const bool sq = K <= 6;
+    const int ne = sq ? npm * npm : npm * (npm + 1) / 2, copies = leaf_copies(K);
+    unsigned long long leaves = 0;
+    auto child = [&](int i) -> uint64_t { return K == 3 ? 0 : ind + ((uint64_t)i << quick_off(K - 2)); };
+    for (int t = g.gl; t < ne; t += W) {
+        uint64_t ee = 0;
+        for (int k = 0; k < copies; k++) {
+            ee += e[k * ne + t];
+            e[k * ne + t] = 0;
+        }
+        if (!ee) continue;
+        int i = t >> lw, j = t & (npm - 1);
+        if (!sq) {
+            for (i = 0; (i + 1) * (i + 2) / 2 <= t;) i++;
+            j = t - i * (i + 1) / 2;
+        }
+        if (i < j) j = i, i = t & (npm - 1);
+        if (!i) continue;
+        if (j) {
+            badd(shist + lut[child(i) + ((uint64_t)(j | npm) << o2)], ee);
+            badd(shist + lut[child(i) + ((uint64_t)j << o2)], 0 - ee);
+            badd(shist + lut[child(j) + ((uint64_t)npm << o2)], 0 - ee);
+            leaves -= ee;
+        }
+        badd(shist + lut[child(i) + ((uint64_t)npm << o2)], 0 - ee);
+        leaves -= ee;
+    }
+    lsync();
+    return leaves;
+}
+
 // The counts of one leaf node, added to the class counters at LDS address shist_at.  (c, pmc):
 // the child of the parent's list (puid, pupm, pnu) that makes the node, its
 // mask; K = 3: the root alone, c = id[0], whose elements [lo, hi) are taken
 // as children.  lds_at: motif_leaf_fixed bytes of LDS, then `space` bytes for the table;
-// gtab: a table of 2^space slots in memory instead.  Not inlined: the node's
+// gtab: a table of 2^space slots in memory instead.  WIDE: such a node of many
+// elements, whose edge counts are flushed now and then; a function of its own, as
+// flushing in the one function cost the k = 5 kernel 3% (Barabasi-Albert 12K 33.1
+// -> 34.0 ms), a call from there 20%.  Not inlined: the node's
 // registers are then its own, not shared with the search around it.
-template <int W>
+template <int W, bool WIDE>
 __device__ __attribute__((noinline)) LeafSum motif_leaf(const int64_t *off_, const int32_t *adj_, const int64_t *ostart_,
                                                         const uint16_t *lut_, const int32_t *puid_,
                                                         const uint8_t *pupm_, uint32_t shist_at, uint32_t lds_at,
@@ -518,7 +560,7 @@ __device__ __attribute__((noinline)) LeafSum motif_leaf(const int64_t *off_, con
     const int ne = sq ? npm * npm : npm * (npm + 1) / 2, copies = leaf_copies(K);
     LeafTab<true> tl;
     LeafTab<false> tg;
-    if (!gtab) {
+    if (!WIDE && !gtab) {
         // at most 45% full while the space allows it
         int b = 7;
         while ((16 << b) <= space && 9 * (2 << b) < 20 * tot) b++;
@@ -552,8 +594,15 @@ __device__ __attribute__((noinline)) LeafSum motif_leaf(const int64_t *off_, con
     const int lw = K - 2;
     unsigned long long qnew = 0, by = 0, leaves = 0, rpairs = 0;
     lds_u32 *const ecopy = e + (g.gl & (copies - 1)) * ne;
+    const uint64_t ind = root ? 0 : pind + (K - 3 >= 2 ? (uint64_t)pmc << quick_off(K - 3) : 0);
     auto scan = [&](const auto &tab) {
         for (int j0 = 0; j0 < tot; j0 += W) {
+        if (WIDE && j0 && j0 % kLeafFlush == 0) {
+            if (enew) ladd(e + (sq ? (newc << lw) + newc : newc * (newc + 1) / 2 + newc), enew);
+            enew = 0;
+            lsync();
+            leaves += leaf_flush(g, lut, shist, e, ind, K);
+        }
         const int j = j0 + g.gl;
         int32_t x = 0;
         int code = 0;
@@ -601,7 +650,7 @@ __device__ __attribute__((noinline)) LeafSum motif_leaf(const int64_t *off_, con
         });
         }
     };
-    if (gtab) scan(tg);
+    if (WIDE || gtab) scan(tg);
     else scan(tl);
     if (nnew) ladd(nm + newc, nnew);
     if (qnew) ladd(qs + newc, (uint64_t)qnew);
@@ -621,7 +670,6 @@ __device__ __attribute__((noinline)) LeafSum motif_leaf(const int64_t *off_, con
         if (!sq) return e[i * (i + 1) / 2 + j];
         return i == j ? (uint64_t)e[(i << lw) + i] : (uint64_t)e[(i << lw) + j] + e[(j << lw) + i];
     };
-    const uint64_t ind = root ? 0 : pind + (K - 3 >= 2 ? (uint64_t)pmc << quick_off(K - 3) : 0);
     auto child = [&](int i) -> uint64_t { return root ? 0 : ind + ((uint64_t)i << quick_off(K - 2)); };
     const int o2 = quick_off(K - 1);
     if (root) rpairs = g.lsum(rpairs);
@@ -1626,18 +1674,18 @@ struct Worker {
         const Lvl &P = ws.lv()[pl < 0 ? 0 : pl];
         const int32_t c = pl < 0 ? v0 : P.eid[i0];
         const int pmc = pl < 0 ? 0 : epm_at(P, i0), pnu = pl < 0 ? 0 : P.nu, sd = pl < 0 ? 0 : P.sdeg;
-        auto run = [&](uint32_t *gtab, int space) {
-            return motif_leaf<W>(p.off, p.adj, p.ostart, lut, P.uid, P.upm, lds_at(shist), lds_at(lds_lo), gtab,
-                                 P.ind, v0, K, c, pmc, pnu, sd, lo, hi, space);
+        auto run = [&](auto wide, uint32_t *gtab, int space) {
+            return motif_leaf<W, decltype(wide)::value>(p.off, p.adj, p.ostart, lut, P.uid, P.upm, lds_at(shist),
+                                                        lds_at(lds_lo), gtab, P.ind, v0, K, c, pmc, pnu, sd, lo, hi, space);
         };
-        LeafSum r = run(nullptr, p.lds_per_worker - motif_leaf_fixed(W, K));
+        LeafSum r = run(std::false_type{}, nullptr, p.lds_per_worker - motif_leaf_fixed(W, K));
         if (r.big) {
             // U does not fit the LDS table: one in the arena
             char *const mg = g_top;
             const int b = r.big;
             uint32_t *const gtab = (uint32_t *)alloc_glb((int64_t)4 << b);
             if (abort) return;
-            r = run(gtab, b);
+            r = b >= kLeafWideBits ? run(std::true_type{}, gtab, b) : run(std::false_type{}, gtab, b);
             g_top = mg;
             if (r.big) fail(2);
         }

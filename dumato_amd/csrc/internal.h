@@ -241,6 +241,13 @@ inline int launch_mode(bool motif, int K) { return !motif ? 0 : K == 5 || K == 6
 // (k = 7: [npm (npm + 1) / 2]), npm = 2^(K-2) mask values.  A motif launch gives
 // each worker at least this.
 constexpr int kLeafCap = 2048;  // stream positions per chunk
+// A leaf node's edges are counted in 32 bits: where its table has fewer than
+// 2^kLeafWideBits slots its elements have fewer than 2^32 pairs; of a wider node
+// the sums go to the 64-bit class counters after every kLeafFlush elements, whose
+// out-lists have fewer than 2^32 entries together (with ids in degree order an
+// out-degree is at most sqrt(2E): 2^22 from 2^43 edges on).
+constexpr int kLeafWideBits = 13;
+constexpr int kLeafFlush = 1024;
 constexpr int leaf_copies(int K) { return K <= 4 ? 8 : K == 5 ? 2 : 1; }
 constexpr int motif_leaf_fixed(int W, int K) {
     return (W * 8 + kLeafCap / 8 + 32 + (1 << (K - 2)) * 12 +
