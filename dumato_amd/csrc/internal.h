@@ -139,6 +139,13 @@ constexpr int kMailOver = 8;
 constexpr int kMailPub = 9;
 constexpr int kMailPubs = kMailStride - kMailPub;
 constexpr unsigned long long kMailIdle = 0xffffffffull;
+// The static scratch holds a launch's mailboxes and, after them, job slots in
+// this many lines: a slot for every worker of a default launch, whose arenas
+// (4,864 B at least) limit them to 13,400 in at most 2,048 blocks.  Of larger
+// grids that a caller asks for the last workers never ask for work.
+constexpr int kScratchLines = 16384;
+static_assert(sizeof(Job) == kMailStride * 8, "a slot and a mailbox are a line each");
+constexpr int scratch_slots(int workers, int blocks) { return std::min(workers, kScratchLines - blocks); }
 
 // One counting query of a launch.  A single-graph call has one; a batch
 // has one per (graph, pattern, k).

@@ -44,16 +44,14 @@ constexpr size_t kSoLut = 32 << 10;                   // class table (uint16)
 constexpr size_t kLutBytes = (size_t)2 << 20;         // 2^20 entries: k <= 7
 constexpr size_t kSoCur = kSoLut + kLutBytes;         // static-queue cursors
 constexpr size_t kMaxWorkers = 65536;
-constexpr size_t kSoQueue = kSoCur + kMaxWorkers * 4;  // the workers' job slots
-constexpr uint32_t kQueueSlots = 8192;
-constexpr size_t kSoMail = kSoQueue + (size_t)kQueueSlots * sizeof(Job);  // the blocks' mailboxes
-constexpr size_t kMaxBlocks = 8192;
-constexpr size_t kSoArena = kSoMail + kMaxBlocks * kMailStride * 8;
+constexpr size_t kSoMail = kSoCur + kMaxWorkers * 4;   // the blocks' mailboxes, then the workers' job slots
+constexpr size_t kMaxBlocks = kScratchLines - 1;
+constexpr size_t kSoArena = kSoMail + (size_t)kScratchLines * sizeof(Job);
 constexpr size_t kArenaBytes = kScratchBytes - kSoArena;
 static_assert(sizeof(SchedCounters) <= kSoEpoch - kSoSc, "counters overlap the epoch");
 static_assert(sizeof(QueryDesc) <= kSoRes - kSoQd, "query descriptor overlaps the results");
 static_assert(kSoRes + kResSlots * 8 <= kSoLut, "results overlap the class table");
-static_assert(kSoQueue % 256 == 0 && kSoArena % 256 == 0, "misaligned scratch regions");
+static_assert(kSoMail % 256 == 0 && kSoArena % 256 == 0, "misaligned scratch regions");
 
 // Device address of `scratch` per device, taken once per device with the
 // device current.  (In host code the array's name only stands for it.)
@@ -70,10 +68,9 @@ static int scratch_on(DeviceCtx *c, char **out) {
         hipError_t e = hipGetSymbolAddress((void **)&p, HIP_SYMBOL(scratch));
         if (e != hipSuccess || !p)
             return set_error(DM_ERR_HIP, "hipGetSymbolAddress(scratch): %s", hipGetErrorString(e));
-        // queue slots and the epoch start at zero (epoch 0 never matches a
-        // launch); cleared with a kernel, not a memset
+        // the epoch starts at zero (the job slots are cleared for each launch);
+        // with a kernel, not a memset
         int r = fill_u32_launch(p + kSoEpoch, 0, 1, c->stream);
-        if (!r) r = fill_u32_launch(p + kSoQueue, 0, (size_t)kQueueSlots * sizeof(Job) / 4, c->stream);
         if (r) return r;
         e = hipStreamSynchronize(c->stream);
         if (e != hipSuccess) return set_error(DM_ERR_HIP, "scratch clear: %s", hipGetErrorString(e));
@@ -173,9 +170,9 @@ static int noalloc_count(dm_graph *g, bool motif, int K, const dm_config &cfg, u
     p.sq_jobs = nullptr;  // strided static partition
     p.sq_cur = (int32_t *)(sp + kSoCur);
     p.res_copies = 1;
-    p.q = (Job *)(sp + kSoQueue);
-    p.q_cap = kQueueSlots;
     p.mail = (unsigned long long *)(sp + kSoMail);
+    p.q = (Job *)(sp + kSoMail) + sh.blocks;
+    p.q_cap = (uint32_t)scratch_slots(sh.workers, sh.blocks);
     p.epoch = (const int32_t *)(sp + kSoEpoch);
     p.sc = (SchedCounters *)(sp + kSoSc);
     p.arena = sp + kSoArena;
