@@ -430,6 +430,17 @@ class Worker {
             const int32_t last = getId(l);
             const int32_t *prev = list(l - 1);
             const int np = fixed()[l - 1];
+            if (d_.motif) {  // extend(begin, end)'s lists do not ascend
+                for (int base = 0; base < np; base += U * W) {
+                    int32_t x[U];
+                    bool ok[U];
+                    load(prev, np, base, x, ok);
+#pragma unroll
+                    for (int u = 0; u < U; u++) w += write(out, w, x[u], ok[u] && x[u] > last);
+                }
+                set_count(l, w, set_next);
+                return;
+            }
             // (ascending: they follow the vertex's place, which is where the
             // step down took it unless a donated job brought it)
             int lo = next()[l - 1], hi = np;
