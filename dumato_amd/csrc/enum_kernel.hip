@@ -1183,6 +1183,82 @@ __device__ __attribute__((noinline)) PairSum child_quads(uint32_t rows_at, uint3
     return r;
 }
 
+// Lists past the bitmaps (roots of more than 256 out-neighbours, or bitmaps off),
+// in functions of their own: inlined, their loops ran on the registers that the
+// bitmap paths left and on spilled ones.  Latency-bound: a chain of loads a child,
+// then one a search step.  (R-MAT s15 of edge factor 8, bitmaps off, k = 5: 32.4 ms
+// inlined, 29.4 so, 20.9 with fewer looks at the mailbox; R-MAT s18 of edge factor
+// 16, k = 5: 670, 637, 588.)
+
+// Whether x is in the ascending list a[0, n), n > 0.
+template <class P>
+DEV bool list_has(P a, int n, int32_t x) {
+    int lo = 0;
+    for (int len = n; len > 1;) {
+        const int half = len >> 1;
+        lo += a[lo + half - 1] < x ? half : 0;
+        len -= half;
+    }
+    return a[lo] == x;
+}
+// Intersection of two ascending lists into out (sorted): the shorter one is
+// strided, the longer searched.
+template <int W>
+__device__ __attribute__((noinline)) int list_intersect(const int32_t *A, int na, const int32_t *B, int nb,
+                                                        int32_t *out) {
+    A = unil<W>(A), B = unil<W>(B), out = unil<W>(out), na = uni<W>(na), nb = uni<W>(nb);
+    const Grp<W> g;
+    const int32_t *S = na > nb ? B : A, *L = na > nb ? A : B;
+    const int ns = na > nb ? nb : na, nl = na > nb ? na : nb;
+    if (ns == 0 || S[ns - 1] < L[0] || L[nl - 1] < S[0]) return 0;
+    int w = 0;
+    for (int base = 0; base < ns; base += W) {
+        const int t = base + g.gl;
+        const int32_t x = t < ns ? S[t] : -1;
+        const bool found = t < ns && list_has(L, nl, x);
+        const uint64_t m = g.ballot(found);
+        if (found) out[w + g.below(m)] = x;
+        w += __popcll(m);
+    }
+    return w;
+}
+// Common elements of the last level's candidates uid[i + 1, nu) and N+(uid[i]), for
+// children i from lo up to hi, as many as start before `until` (one at least,
+// kListRun at most): this lane's count, the children's out-degrees (all lanes the
+// same) and the next child.
+constexpr int kListRun = 64;
+struct ListSum {
+    unsigned long long cnt, by;
+    int next;
+};
+template <int W>
+__device__ __attribute__((noinline)) ListSum list_leaf(const int64_t *off_, const int32_t *adj_, const int64_t *ostart_,
+                                                       const int32_t *uid, int nu, int lo, int hi, uint64_t until) {
+    glb_i64 *const off = (glb_i64 *)unil<W>(off_), *const ostart = (glb_i64 *)unil<W>(ostart_);
+    glb_i32 *const adj = (glb_i32 *)unil<W>(adj_);
+    uid = unil<W>(uid), nu = uni<W>(nu), lo = uni<W>(lo), hi = uni<W>(hi), until = unil<W>(until);
+    const Grp<W> g;
+    ListSum r{0, 0, lo};
+    if (hi - lo > kListRun) hi = lo + kListRun;
+    do {
+        const int i = r.next;
+        const int32_t c = uni<W>(uid[i]);
+        const int64_t os = unil<W>(ostart[c]);
+        const int na = (int)(unil<W>(off[c + 1]) - os), nb = nu - i - 1;
+        glb_i32 *const A = adj + os;
+        const int32_t *const B = uid + i + 1;
+        r.by += (unsigned long long)na;
+        r.next = i + 1;
+        if (na == 0 || nb == 0 || A[na - 1] < B[0] || B[nb - 1] < A[0]) continue;
+        if (na <= nb) {
+            for (int t = g.gl; t < na; t += W) r.cnt += list_has(B, nb, A[t]) ? 1 : 0;
+        } else {
+            for (int t = g.gl; t < nb; t += W) r.cnt += list_has(A, na, B[t]) ? 1 : 0;
+        }
+    } while (r.next < hi && now_ticks() < until);
+    return r;
+}
+
 // A job's head, in registers; its prefix ids go to the worker's LDS record (jid).
 struct JobHead {
     int lvl, lo, hi, q;
@@ -1399,7 +1475,7 @@ struct Worker {
     DEV unsigned long long *mailbox(int b) const { return p.mail + (size_t)b * kMailStride; }
 
     // Requests waiting in this block's mailbox, looked for at most once per
-    // period, which doubles (16-fold at most) while none comes: their number;
+    // period, which doubles after a look that found none: their number;
     // rq: lane i's own (i < kMailSlots; 0: none).
     DEV int requests(unsigned long long &rq) {
         const uint64_t now = now_ticks();
@@ -1413,7 +1489,7 @@ struct Worker {
             if (rq == kMailIdle) rq = 0, (void)atomicCAS(m, kMailIdle, 0ull);
         }
         const int n = __popcll(g.ballot(rq != 0));
-        poll_shift = n ? 0 : 1;
+        if (n == 0) poll_shift = 1;
         return n;
     }
 
@@ -1487,10 +1563,17 @@ struct Worker {
     // min_first > 0: the job's own level may be cut down to pieces of that
     // many children (heavy children, where steal_min would leave too much);
     // min_pairs > 0: the same for the pairs of a bitmap root's child (level 1).
-    DEV void maybe_donate(int top, int min_first = 0, int min_pairs = 0) {
+    // lists: the worker is on the list path, whose children are short beside a
+    // look at the mailbox; while its looks find askers and nothing to give, the
+    // period doubles, 16-fold at most.  (R-MAT s15 of edge factor 8, bitmaps off,
+    // k = 6 181 -> 127 ms; with the same on the bitmap paths k = 7 of R-MAT s13 of
+    // edge factor 16 3.6 -> 4.2.)
+    DEV void maybe_donate(int top, int min_first = 0, int min_pairs = 0, bool lists = false) {
         unsigned long long rq = 0;
         int n = requests(rq);
         if (n == 0) return;
+        const int shift = poll_shift;
+        poll_shift = 0;
         if (own_cur >= own_end && own_queue >= 0) claim_shared(n);
         if (own_cur < own_end) {
             const int cur = own_cur, len = own_end - cur;
@@ -1509,8 +1592,7 @@ struct Worker {
             own_end = cut(1);
             return;
         }
-        if (!p.steal) return;
-        if (range_hi - v0 - 1 >= 2) {
+        if (p.steal && range_hi - v0 - 1 >= 2) {
             const int lo = v0 + 1, len = range_hi - lo;
             n = accept(rq, len - 1, true);
             if (n == 0) return;
@@ -1524,7 +1606,7 @@ struct Worker {
         }
         // a clique's last level has cheap children: split it only in bigger pieces
         const int leaf_min = 4 * job_sm;
-        for (int l = job_lvl; l < top; l++) {
+        for (int l = p.steal ? job_lvl : top; l < top; l++) {
             const int cur = ws.lv()[l].cur, end = ws.lv()[l].end;
             const int minc = min_pairs > 0 && l == 1                ? min_pairs
                              : min_first > 0 && l == job_lvl ? min_first
@@ -1533,7 +1615,7 @@ struct Worker {
             if (end - cur < minc) continue;
             int most = (end - cur) / minc - 1;
             most = most < 1 ? 1 : most > end - cur - 1 ? end - cur - 1 : most;
-            if (most < 1) return;
+            if (most < 1) break;
             n = accept(rq, most, true);
             if (n == 0) return;
             publish();
@@ -1551,6 +1633,8 @@ struct Worker {
             if (g.gl == 0) ws.st()[kStDonated] += (unsigned long long)n;
             return;
         }
+        // nothing to give: the askers go elsewhere
+        if (lists) poll_shift = shift < 4 ? shift + 1 : 4;
     }
 
     // ---- motif levels ----------------------------------------------------------
@@ -1706,40 +1790,6 @@ struct Worker {
     DEV const int32_t *onbr(int32_t v) const { return p.adj + p.ostart[v]; }
     DEV int odeg(int32_t v) const { return (int)(p.off[v + 1] - p.ostart[v]); }
 
-    // Intersection of two sorted lists: stride the shorter one, binary-search
-    // the longer.  WRITE: compact survivors (sorted) into out and return the
-    // count; otherwise return this lane's partial count.
-    template <bool WRITE>
-    DEV int intersect(const int32_t *A, int na, const int32_t *B, int nb, int32_t *out) {
-        const int32_t *S = A, *L = B;
-        int ns = na, nl = nb;
-        if (na > nb) {
-            S = B; L = A; ns = nb; nl = na;
-        }
-        if (ns == 0 || nl == 0) return 0;
-        if (S[ns - 1] < L[0] || L[nl - 1] < S[0]) return 0;
-        int w = 0;
-        for (int base = 0; base < ns; base += W) {
-            int t = base + g.gl;
-            bool in = t < ns;
-            bool found = false;
-            int32_t x = 0;
-            if (in) {
-                x = S[t];
-                int pos = lower_bound(L, nl, x);
-                found = pos < nl && L[pos] == x;
-            }
-            if constexpr (WRITE) {
-                uint64_t m = g.ballot(found);
-                if (found) out[w + g.below(m)] = x;
-                w += __popcll(m);
-            } else {
-                w += found ? 1 : 0;
-            }
-        }
-        return w;
-    }
-
     DEV void clique_forward(int l, int i) {
         Lvl &P = ws.lv()[l];
         Lvl &N = ws.lv()[l + 1];
@@ -1752,7 +1802,7 @@ struct Worker {
         const int cap = na < nb ? na : nb;
         int32_t *out = (int32_t *)alloc((int64_t)(cap > 0 ? cap : 1) * 4);
         if (abort) return;
-        int w = intersect<true>(onbr(c), na, B, nb, out);
+        const int w = list_intersect<W>(onbr(c), na, B, nb, out);
         wsync();
         N.uid = out;
         N.nu = w;
@@ -1761,18 +1811,18 @@ struct Worker {
 
     DEV void clique_leaf_phase(int l, int lo, int hi) {
         Lvl &P = ws.lv()[l];
-        for (int i = lo; i < hi; i++) {
+        while (lo < hi) {
             if (check_abort()) return;
             // donation of this level's tail happens through lv[l].cur/end
-            P.cur = i + 1;
-            maybe_donate(l + 1);
-            hi = P.end;
-            if (i >= hi) break;
-            const int32_t c = P.uid[i];
-            const int na = odeg(c);
-            int part = intersect<false>(onbr(c), na, P.uid + i + 1, P.nu - i - 1, nullptr);
-            cnt += (unsigned long long)part;
-            if (g.gl == 0) bytes += 4ull * (unsigned long long)na;
+            P.cur = lo;
+            maybe_donate(l + 1, 0, 0, true);
+            hi = uni<W>(P.end);
+            if (lo >= hi) break;
+            const ListSum r = list_leaf<W>(p.off, p.adj, p.ostart, P.uid, P.nu, lo, hi,
+                                           last_poll + (p.poll_ticks << poll_shift));
+            cnt += r.cnt;
+            if (g.gl == 0) bytes += 4ull * r.by;
+            lo = uni<W>(r.next);
         }
     }
 
@@ -2319,7 +2369,7 @@ struct Worker {
                 k--;
                 continue;
             }
-            maybe_donate(k + 1);
+            maybe_donate(k + 1, 0, 0, !motif);
             const int i = uni<W>(L.cur);
             if (i < uni<W>(L.end)) {
                 if (motif && k >= K - 4) {
@@ -2613,8 +2663,9 @@ __global__ __launch_bounds__(kThreads, WAVES) void enum_kernel(EnumParams p) {
         bool idle = false, all_started = false;
         uint32_t seq = 0;  // requests of this launch
         int asked = -1;    // mailbox word that holds this worker's request
-        int waited = 0;    // polls since it was written
-        int backoff = 1;
+        int waited = 0;    // time since it was written, in sleeps
+        // sleeps of the next round, the most of a round now, rounds at that many
+        int backoff = 1, most = 4, dry = 0;
         uint32_t spins = 0;
         const bool can_ask = (uint32_t)wid < p.q_cap;
         open_own_queue(wk, wid);
@@ -2643,7 +2694,8 @@ __global__ __launch_bounds__(kThreads, WAVES) void enum_kernel(EnumParams p) {
                     got = r == 1;
                     if (r == 2) got = take_own(wk, jh);
                     // no answer for long: ask elsewhere (unless it is coming)
-                    if (r == 0 && ++waited >= 24) {
+                    waited += backoff;
+                    if (r == 0 && waited >= 96) {
                         int back = 0;
                         const unsigned long long rq = ((unsigned long long)tag << 32) | (uint32_t)(wid + 1);
                         if (g.gl == 0) back = atomicCAS(p.mail + asked, rq, 0ull) == rq;
@@ -2692,10 +2744,22 @@ __global__ __launch_bounds__(kThreads, WAVES) void enum_kernel(EnumParams p) {
                     break;
                 }
                 // sleep only when no lane of this wave has work: s_sleep
-                // stalls the whole wave, including busy narrower workers
+                // stalls the whole wave, including busy narrower workers.  The
+                // longer nothing comes the longer: the polls and requests of
+                // thousands of idle waves slow the few busy ones' loads (with
+                // sleeps of 4 x 512 cycles at most R-MAT s15 k = 5 with bitmaps
+                // and stealing off 129 ms, 73 so; Chung-Lu 1,000 k = 6 without
+                // stealing 14.6 -> 11.6).  A step every 64 rounds, so sleeps stay
+                // a few percent of the time idle (every 16: R-MAT s17 k = 6 2.53
+                // -> 2.72 ms; every 64 2.56).
                 if (__ballot(1) == ~0ull) {
                     for (int b = 0; b < backoff; b++) __builtin_amdgcn_s_sleep(8);
-                    backoff = backoff < 4 ? backoff * 2 : 4;
+                    if (backoff < most) {
+                        backoff *= 2;
+                    } else if (++dry >= 64 && most < 256) {
+                        dry = 0;
+                        most *= 2;
+                    }
                 }
                 continue;
             }
@@ -2703,7 +2767,7 @@ __global__ __launch_bounds__(kThreads, WAVES) void enum_kernel(EnumParams p) {
                 idle = false;
                 go_busy<W>(p, g, blk);
             }
-            backoff = 1;
+            backoff = 1, most = 4, dry = 0;
             const int jq = job_query(jh.q);
             bool ok = jh.q >= 0 && jq < p.nq;
             int merged = 0;  // further jobs done with this one
