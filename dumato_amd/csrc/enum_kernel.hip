@@ -705,6 +705,9 @@ __device__ __attribute__((noinline)) LeafSum motif_leaf(const int64_t *off_, con
 // 83 M triangles; one child at a time, each entry searched in the longer list:
 // 5.19 -> 1.81 ms).  lds_at: recs u64[W] | bits u64[kLeafCap / 64 + 8] | table.
 constexpr int kTriFixed = 64 * 8 + kLeafCap / 8 + 64;
+// (the triangles' own: at 8 lanes the table fits the default slice of 1,456 B only
+// so; R-MAT s15 of edge factor 8, k = 3, 1.34 -> 0.20 ms)
+constexpr int tri_fixed(int W) { return kTriFixed - (64 - W) * 8; }
 struct TriSum {
     unsigned long long cnt, by;  // this lane's share; by: out-degrees of the children
 };
@@ -719,7 +722,7 @@ __device__ __attribute__((noinline)) TriSum triangles(const int64_t *off_, const
     lds_u64 *const recs = (lds_u64 *)(uintptr_t)(uint32_t)uni<W>((int)at);
     lds_u64 *const bits = recs + W;
     LeafTab<true> tab;
-    tab.t = (lds_u32 *)(recs + kTriFixed / 8);
+    tab.t = (lds_u32 *)(recs + tri_fixed(W) / 8);
     tab.b = b, tab.sh = 32 - b, tab.mul = 0x9E3779B1u;
     const int64_t ls = unil<W>(ostart[v0]);
     glb_i32 *const L = adj + ls;
@@ -1250,11 +1253,11 @@ __device__ __attribute__((noinline)) ListSum list_leaf(const int64_t *off_, cons
         r.by += (unsigned long long)na;
         r.next = i + 1;
         if (na == 0 || nb == 0 || A[na - 1] < B[0] || B[nb - 1] < A[0]) continue;
-        if (na <= nb) {
-            for (int t = g.gl; t < na; t += W) r.cnt += list_has(B, nb, A[t]) ? 1 : 0;
-        } else {
-            for (int t = g.gl; t < nb; t += W) r.cnt += list_has(A, na, B[t]) ? 1 : 0;
-        }
+        // (one loop: narrow workers of a wave then share it, R-MAT s15 k = 3 with
+        // lists, 8 lanes, 1.74 -> 1.30 ms)
+        const int32_t *const G = (const int32_t *)A, *const S = na <= nb ? G : B, *const L = na <= nb ? B : G;
+        const int ns = na <= nb ? na : nb, nl = na <= nb ? nb : na;
+        for (int t = g.gl; t < ns; t += W) r.cnt += list_has(L, nl, S[t]) ? 1 : 0;
     } while (r.next < hi && now_ticks() < until);
     return r;
 }
@@ -1477,9 +1480,10 @@ struct Worker {
     // Requests waiting in this block's mailbox, looked for at most once per
     // period, which doubles after a look that found none: their number;
     // rq: lane i's own (i < kMailSlots; 0: none).
+    DEV uint64_t period() const { return p.poll_ticks << poll_shift; }
     DEV int requests(unsigned long long &rq) {
         const uint64_t now = now_ticks();
-        if (now - last_poll < (p.poll_ticks << poll_shift)) return 0;
+        if (now - last_poll < period()) return 0;
         last_poll = now;
         rq = 0;
         if (g.gl < kMailSlots) {
@@ -1819,7 +1823,7 @@ struct Worker {
             hi = uni<W>(P.end);
             if (lo >= hi) break;
             const ListSum r = list_leaf<W>(p.off, p.adj, p.ostart, P.uid, P.nu, lo, hi,
-                                           last_poll + (p.poll_ticks << poll_shift));
+                                           last_poll + period());
             cnt += r.cnt;
             if (g.gl == 0) bytes += 4ull * r.by;
             lo = uni<W>(r.next);
@@ -1833,8 +1837,8 @@ struct Worker {
         const int d = R.nu;
         int b = 7;
         while (9 * (2 << b) < 20 * d) b++;  // at most 45% full
-        while (b > 7 && kTriFixed + (8 << b) > p.lds_per_worker && 7 * d <= 6 * (1 << b)) b--;
-        if (kTriFixed + (8 << b) > p.lds_per_worker) return false;
+        while (b > 7 && tri_fixed(W) + (8 << b) > p.lds_per_worker && 7 * d <= 6 * (1 << b)) b--;
+        if (tri_fixed(W) + (8 << b) > p.lds_per_worker) return false;
         R.cur = lo;
         R.end = hi < d ? hi : d;
         for (bool first = true;; first = false) {
@@ -2706,7 +2710,7 @@ __global__ __launch_bounds__(kThreads, WAVES) void enum_kernel(EnumParams p) {
                     // a random word of a random block's mailbox; a block without
                     // work, or another request there, says so at once
                     const unsigned long long rq = ((unsigned long long)tag << 32) | (uint32_t)(wid + 1);
-                    for (int a = 0; a < 4 && asked < 0; a++) {
+                    for (int a = 0; a < (W > 16 ? W / 16 : 1) && asked < 0; a++) {
                         seed = seed * 1664525u + 1013904223u;
                         const int b = (int)((seed >> 8) % gridDim.x) * kMailStride + (int)(seed >> 29);
                         int in = 0;
@@ -2751,9 +2755,12 @@ __global__ __launch_bounds__(kThreads, WAVES) void enum_kernel(EnumParams p) {
                 // and stealing off 129 ms, 73 so; Chung-Lu 1,000 k = 6 without
                 // stealing 14.6 -> 11.6).  A step every 64 rounds, so sleeps stay
                 // a few percent of the time idle (every 16: R-MAT s17 k = 6 2.53
-                // -> 2.72 ms; every 64 2.56).
+                // -> 2.72 ms; every 64 2.56).  Narrow workers sleep longer and ask
+                // fewer at a time, as there are more of them to a wave (R-MAT s15
+                // k = 3 with lists, 8 lanes, 2.4 -> 1.7 ms; k = 5, 16 lanes, 2.01 ->
+                // 1.84).
                 if (__ballot(1) == ~0ull) {
-                    for (int b = 0; b < backoff; b++) __builtin_amdgcn_s_sleep(8);
+                    for (int b = 0; b < backoff * (64 / W); b++) __builtin_amdgcn_s_sleep(8);
                     if (backoff < most) {
                         backoff *= 2;
                     } else if (++dry >= 64 && most < 256) {
