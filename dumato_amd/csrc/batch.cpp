@@ -260,7 +260,7 @@ static int batch_build(dm_batch *b, const std::vector<dm_query> &qs, const dm_co
         const int ncls_single = qs.size() == 1 ? P.wslots : 0;
         const int hs = qs.size() == 1 ? 0 : P.wslots;
         P.lds = lds > 0 ? lds : max_lds_per_worker(vw, threads, P.mode, P.kmax, ncls_single, hs);
-        if (P.qs[0].motif) P.lds = std::max(P.lds, motif_leaf_fixed(vw, P.kmax));
+        if (P.qs[0].motif) P.lds = motif_lds(vw, threads, P.mode, P.kmax, ncls_single, hs, P.lds, lds > 0);
         P.lds_total = enum_lds_bytes(vw, threads, P.kmax, ncls_single, hs, P.lds);
         int bpc = 0;
         if ((r = enum_occupancy(vw, P.mode, threads, P.lds_total, &bpc))) return r;

@@ -584,7 +584,7 @@ __device__ __attribute__((noinline)) LeafSum motif_leaf(const int64_t *off_, con
             tg.mul = tg.mul * 0x2545F491u + 2;  // another odd multiplier
         }
     }
-    for (int j = g.gl; j < ne * copies; j += W) e[j] = 0;
+    for (int j = g.gl; j < ne * copies / 2; j += W) ((lds_u64 *)e)[j] = 0;
     for (int j = g.gl; j < npm; j += W) nm[j] = 0, qs[j] = 0;
     lsync();
 
@@ -673,19 +673,33 @@ __device__ __attribute__((noinline)) LeafSum motif_leaf(const int64_t *off_, con
     auto child = [&](int i) -> uint64_t { return root ? 0 : ind + ((uint64_t)i << quick_off(K - 2)); };
     const int o2 = quick_off(K - 1);
     if (root) rpairs = g.lsum(rpairs);
-    for (int t = g.gl; t < npm * npm; t += W) {
-        const int i = t >> (K - 2), j = t & (npm - 1);
-        if (j == 0 || i < j) continue;
+    auto pair = [&](int i, int j) {
         const uint64_t ni = nm[i], nj = nm[j];
         const uint64_t pr = root ? rpairs : i == j ? ni * (ni - 1) / 2 : ni * nj;
-        if (pr == 0) continue;
+        if (pr == 0) return;
         const uint64_t ee = edges(i, j);
         if (ee) badd(shist + lut[child(i) + ((uint64_t)(j | npm) << o2)], ee);
         if (pr != ee) badd(shist + lut[child(i) + ((uint64_t)j << o2)], pr - ee);
         leaves += pr;
+    };
+    if (W < 64 && npm > W) {
+        // few lanes for many masks, most of them without elements (Chung-Lu 1,000
+        // of 1,500 edges, k = 7: 8 lanes 27.2 -> 19.5 ms, 16 lanes 12.4 -> 9.2)
+        uint32_t some = 0;
+        for (int k = 0; k < npm; k += W) some |= (uint32_t)g.ballot(nm[k + g.gl] != 0) << k;
+        for (; some; some &= some - 1) {
+            const int i = __builtin_ctz(some);
+            for (int j = 1 + g.gl; j <= i; j += W) pair(i, j);
+        }
+    } else {
+        for (int t = g.gl; t < npm * npm; t += W) {
+            const int i = t >> (K - 2), j = t & (npm - 1);
+            if (j != 0 && i >= j) pair(i, j);
+        }
     }
     for (int i = 1 + g.gl; i < npm; i += W) {
         uint64_t nw = qs[i];
+        if (!nm[i]) continue;
         for (int j = 0; j < npm; j++) nw -= i == j ? 2 * edges(i, i) : i > j ? edges(i, j) : edges(j, i);
         if (nw) badd(shist + lut[child(i) + ((uint64_t)npm << o2)], nw);
         leaves += nw;

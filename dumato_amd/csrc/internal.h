@@ -268,6 +268,7 @@ constexpr int leaf_table_bits(int64_t tot) {
     return b;
 }
 constexpr int64_t leaf_table_bytes(int64_t tot) { return (int64_t)4 << leaf_table_bits(tot); }
+constexpr int kLeafTableMin = 1024;  // the smallest table in LDS
 size_t enum_lds_bytes(int vwave, int threads, int kmax, int ncls_single, int hist_slots, int lds_per_worker);
 int enum_occupancy(int vwave, int mode, int threads, size_t lds, int *blocks_per_cu);
 int enum_launch(const EnumParams &p, int mode, int vwave, int blocks, int threads, size_t lds,

@@ -253,6 +253,23 @@ static double leaf_elements(const dm_graph *g, int K) {
     return sum > 0 ? sum * std::pow(g->degree_squares / sum, K - 3) : 0;
 }
 
+// A motif worker's slice: the leaf's fixed part at least; unless the caller chose
+// the size, room for the smallest table beside it, where that takes no more than
+// a third of the blocks a CU (narrow workers' default slices have none, and each
+// leaf built its table in memory.  8 lanes: Barabasi-Albert 1,500 k = 5 2.62 ->
+// 2.00 ms with 2 blocks of 3, random 5,000 k = 4 0.94 -> 0.62, but 2,000 k = 6 41 -> 48
+// with one of 2; 16 lanes: Barabasi-Albert 600 k = 7 152 -> 119 with 2 as before).
+int motif_lds(int vwave, int threads, int mode, int K, int ncls_single, int hist_slots, int lds, bool chosen) {
+    const int least = motif_leaf_fixed(vwave, K), room = least + kLeafTableMin;
+    lds = std::max(lds, least);
+    if (chosen || lds >= room) return lds;
+    int now = 0, then = 0;
+    if (enum_occupancy(vwave, mode, threads, enum_lds_bytes(vwave, threads, K, ncls_single, hist_slots, lds), &now) ||
+        enum_occupancy(vwave, mode, threads, enum_lds_bytes(vwave, threads, K, ncls_single, hist_slots, room), &then))
+        return lds;
+    return 3 * then >= 2 * now ? room : lds;
+}
+
 int pick_shape(dm_graph *g, int K, bool motif, const dm_config &cfg, Shape &sh) {
     DeviceCtx *c = g->dev->ctx;
     int vw = cfg.vwave;
@@ -268,7 +285,7 @@ int pick_shape(dm_graph *g, int K, bool motif, const dm_config &cfg, Shape &sh) 
     const int dl = max_lds_per_worker(vw, threads, launch_mode(motif, K), K, ncls, 0);
     int lds = cfg.lds_bytes > 0 ? cfg.lds_bytes : threads == 256 ? tuned_lds(g, K, motif, vw, dl) : dl;
     lds = (lds + 15) & ~15;
-    if (motif) lds = std::max(lds, motif_leaf_fixed(vw, K));
+    if (motif) lds = motif_lds(vw, threads, launch_mode(motif, K), K, ncls, 0, lds, cfg.lds_bytes > 0);
     size_t lds_total = enum_lds_bytes(vw, threads, K, ncls, 0, lds);
     int bpc = 0;
     if ((r = enum_occupancy(vw, launch_mode(motif, K), threads, lds_total, &bpc))) return r;

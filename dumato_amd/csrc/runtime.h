@@ -173,6 +173,7 @@ void free_device_graph(DeviceGraph *d);
 int device_lut(DeviceCtx *c, int K, const uint16_t **out);
 // Threads per block for cfg.waves_per_block (1, 2 or 4 waves; 0 = 4).
 int block_threads(const dm_config &cfg, int *threads);
+int motif_lds(int vwave, int threads, int mode, int K, int ncls_single, int hist_slots, int lds, bool chosen);
 int pick_shape(dm_graph *g, int K, bool motif, const dm_config &cfg, Shape &sh);
 bool root_has_work(const dm_graph *g, int32_t v, int K, bool motif);
 void plain_partition(const dm_graph *g, const std::vector<int32_t> &roots, int K, bool motif, int workers,

@@ -23,3 +23,17 @@ def test_default_slices_hold_a_table(tmp_path):
         tot, hist = g.motif_count(k, dm.config(vwave=64, watchdog_s=60.0))
         assert tot == want[0] and np.array_equal(hist, want[1])
         assert g.last_stats()["lds_bytes"] >= fixed[k - 3] + SMALLEST_TABLE
+
+
+@pytest.mark.parametrize("w,k", [(8, 4), (8, 5), (8, 7), (16, 7), (32, 7)])
+def test_narrow_slices_hold_a_table(tmp_path, w, k):
+    fixed = int(hostcc.run(tmp_path, 'printf("%%d", motif_leaf_fixed(%d, %d));' % (w, k)))
+    s, d, n = G.gnp(24, 0.3, 2 + k)
+    g, ref = dm.Graph.from_edges(s, d, n), O.csr_from_edges(s, d, n)
+    print("case narrow slice w=%d k=%d" % (w, k), flush=True)
+    table = dict(table=(dm.pattern_table(7)[0], dm.num_classes(7))) if k == 7 else {}
+    wt, wh = O.motif_count(ref, k, **table)
+    for kw in (dict(), dict(lds_bytes=256)):
+        tot, hist = g.motif_count(k, dm.config(vwave=w, watchdog_s=60.0, **kw))
+        assert tot == wt and np.array_equal(hist, wh)
+        assert (g.last_stats()["lds_bytes"] >= fixed + SMALLEST_TABLE) == (not kw)
