@@ -319,17 +319,14 @@ def roofline(st, kern_ms, total):
     if os.path.exists(PROFILE_COUNTERS):
         rec = json.load(open(PROFILE_COUNTERS)).get("motif4_chunglu18k", {})
     valu = rec.get("valu_insts")
-    steal = rec.get("valu_insts_steal_loop", 0.0)
     traffic = rec.get("hbm_bytes")
     t = kern_ms / 1e3
     achieved = valu / t / 1e9 if valu else None
     alg = st["alg_bytes"]
-    # frac counts every VALU instruction issued; frac_enumeration leaves out
-    # the idle workers' loop where the profile has its share
+    # frac counts every VALU instruction issued, the idle workers' too
     return {"bound": "valu", "achieved": achieved, "peak": VALU_PEAK_GINST, "unit": "Ginst/s",
             "frac": achieved / VALU_PEAK_GINST if achieved else None, "traffic": traffic,
-            "frac_enumeration": (valu - steal) / t / 1e9 / VALU_PEAK_GINST if valu else None,
-            "valu_insts_per_launch": valu, "valu_insts_steal_loop": steal,
+            "valu_insts_per_launch": valu,
             "counters": "profiles/enum_kernel_motif4_chunglu18k.md",
             "hbm_GBs": traffic / t / 1e9 if traffic else None,
             "hbm_frac": traffic / t / 1e9 / HBM_PEAK_GBS if traffic else None,
