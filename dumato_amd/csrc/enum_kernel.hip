@@ -603,6 +603,7 @@ __device__ __attribute__((noinline)) LeafSum motif_leaf(const int64_t *off_, con
             lsync();
             leaves += leaf_flush(g, lut, shist, e, ind, K);
         }
+        if (WIDE && root && (j0 + W <= lo || j0 >= hi)) continue;
         const int j = j0 + g.gl;
         int32_t x = 0;
         int code = 0;
@@ -1768,7 +1769,9 @@ struct Worker {
     }
 
     // ---- motif leaf ------------------------------------------------------------
-    static constexpr int kMotif3Chunk = 512;  // (each builds the root's table again)
+    // k = 3: children of the root to a chunk (each builds the root's table again)
+    static constexpr int kMotif3Chunk = 512;
+    DEV static int motif3_chunk(int children) { return children <= 8 * kMotif3Chunk ? kMotif3Chunk : (children + 7) / 8; }
     // Leaf node of child i0 of level pl = K-4 (k >= 4), or the root itself at
     // k = 3 (pl = -1) with the elements [lo, hi) of its list as children.
     DEV void motif_leaf_node(int pl, int i0, int lo, int hi) {
@@ -2392,10 +2395,10 @@ struct Worker {
             if (i < uni<W>(L.end)) {
                 if (motif && k >= K - 4) {
                     // a child makes a leaf node; at k = 3 the root is one, its
-                    // children taken kMotif3Chunk per donation check
+                    // children taken a chunk per donation check
                     const bool root = K == 3;
-                    const int left = uni<W>(L.end) - i;
-                    const int to = root ? i + (left < kMotif3Chunk ? left : kMotif3Chunk) : i + 1;
+                    const int left = uni<W>(L.end) - i, chunk = motif3_chunk(uni<W>(L.ne));
+                    const int to = root ? i + (left < chunk ? left : chunk) : i + 1;
                     L.cur = to;
                     motif_leaf_node(root ? -1 : k, i, root ? i : 0, root ? to : 0x7fffffff);
                     if (abort) return;

@@ -11,7 +11,7 @@ from tests import graphs as G
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n", [1367, 2732, 2733, 2800, 2843])
+@pytest.mark.parametrize("n", [1367, 2732, 2733, 2800, 2843, 4200])
 @pytest.mark.parametrize("w", [64, 16])
 def test_complete_graphs(n, w):
     print("case K%d motif k=3 w=%d" % (n, w), flush=True)
